@@ -14,6 +14,7 @@
 // 256-point chunk, chunk sums in FP64.  A condition check of every point's
 // FP32 sum sends ill-conditioned points to an FP64 recomputation.
 #include "srw_sr_dev.h"
+#include <algorithm>
 
 // ------------------------------------------------------------------------
 // Field and RK4 (FP64)
@@ -640,13 +641,16 @@ __global__ void __launch_bounds__(256) k_sr_tables(const srwd_trj_info* __restri
                                                    const double* X, const double* Y, const double* IBx,
                                                    const double* IBz, long long ldT,
                                                    srwd_rec* rec, srwd_chunk* chunk, double* Qout,
-                                                   long long ldI, long long ldC, long long maxInt, double* T64)
+                                                   long long ldI, long long ldC, double* T64, srwd_mrec* M,
+                                                   long long ldM)
 {
     long long gi = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     int tr = blockIdx.y;
-    if (gi >= maxInt) return;
     const srwd_trj_info I = info[tr];
-    if (gi >= I.nInt) return;
+    if (gi >= I.nInt) {
+        if (gi < ldM) M[tr * ldM + gi] = srwd_mrec{0., 0., 0., 0., 0.f, 0.f, 0.f, 0.f};
+        return;
+    }
     bool byDiv = I.nInt < 10000;   // srradint.h:1046-1050: manual "faster" below 10000 points
     const double* cx = X + tr * ldT; const double* cz = Y + tr * ldT;
     const double* ix = IBx + tr * ldT; const double* iz = IBz + tr * ldT;
@@ -688,6 +692,7 @@ __global__ void __launch_bounds__(256) k_sr_tables(const srwd_trj_info* __restri
     R.bPx = (float)(bd * Pxd);
     R.bPz = (float)(bd * Pzd);
     rec[tr * ldI + gi] = R;
+    M[tr * ldM + gi] = srwd_mrec{Xv, Zv, inv, s * I.gammaEm2 + IB, R.b, R.bPx, R.bPz, 0.f};
     Qout[tr * ldI + gi] = Q;
     // FP64 trajectory values at the point, for the FP64 recomputation of
     // ill-conditioned points (k_sr_fp64)
@@ -1049,7 +1054,7 @@ __global__ void __launch_bounds__(256) k_sr_integral_tile(const srwd_item* __res
                 const srwd_req Rq = F.reqs[Ie.traj];
                 double sumSqX = 0., sumSqZ = 0.;
                 if (F.cond) {
-                    const double* c = F.cond + 5 * Ie.traj;
+                    const double* c = F.cond + SRWD_COND * Ie.traj;
                     const double xr = F.coord[Rq.xOff + ix], zr = F.coord[Rq.zOff + iz];
                     sumSqX = c[0] * xr * xr - 2. * xr * c[1] + c[3];
                     sumSqZ = c[0] * zr * zr - 2. * zr * c[2] + c[4];
@@ -1087,6 +1092,9 @@ __global__ void __launch_bounds__(256) k_sr_integral_tile(const srwd_item* __res
 // Energy-tile items: the phasor of energy k carries k times the rounding of
 // the step's phase and the recurrence's roundings on top.
 #define SRWD_EPS_TERM_TILE 4e-6
+// Mesh items (sr_mesh.hip): phases reduced in FP64 before their sine and
+// cosine, phasors as FP16 pairs of about 22 bits.
+#define SRWD_EPS_TERM_MESH 1e-6
 
 // Terminating terms, the derivative correction, the float store and the
 // mirrored parts of one point; S = sum over the integration points of
@@ -1128,7 +1136,8 @@ __device__ void sr_finish_point(const srwd_item& IT, const srwd_trj_info& I, con
     if (fpList) {
         // condition check of the FP32 sums against the point's field
         // magnitude: hand the point to the FP64 pass
-        const double eps = IT.tiled ? SRWD_EPS_TERM_TILE : SRWD_EPS_TERM;
+        const double eps = IT.tiled == SRWD_ITEM_MESH ? SRWD_EPS_TERM_MESH
+                                                      : (IT.tiled ? SRWD_EPS_TERM_TILE : SRWD_EPS_TERM);
         const double e2 = eps * eps * w * w, t2 = condTol * condTol;
         const double mag2 = ex.re * ex.re + ex.im * ex.im + ez.re * ez.re + ez.im * ez.im;
         if (e2 * (fmax(sumSqX, 0.) + fmax(sumSqZ, 0.)) > t2 * mag2) {
@@ -1161,27 +1170,32 @@ __device__ void sr_finish_point(const srwd_item& IT, const srwd_trj_info& I, con
 // Sums of squared terms per trajectory, from the integration records:
 // cond[0..4] = sum b^2, sum b bPx, sum b bPz, sum bPx^2, sum bPz^2, so that
 // the squared x terms of point (xo, zo) add up to
-// cond[0] xo^2 - 2 xo cond[1] + cond[3] (and the z terms likewise).
+// cond[0] xo^2 - 2 xo cond[1] + cond[3] (and the z terms likewise); and the
+// largest |b|, |bPx| and |bPz| in cond[5..7].
 __global__ void __launch_bounds__(256) k_cond_sums(const srwd_trj_info* __restrict__ info,
                                                    const srwd_rec* __restrict__ rec, long long ldI, double* cond)
 {
     int tr = blockIdx.x;
     long long n = info[tr].nInt;
     const srwd_rec* R = rec + (long long)tr * ldI;
-    double v[5] = {0, 0, 0, 0, 0};
+    double v[SRWD_COND] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (long long i = threadIdx.x; i < n; i += blockDim.x) {
         double bb = R[i].b, px = R[i].bPx, pz = R[i].bPz;
         v[0] += bb * bb; v[1] += bb * px; v[2] += bb * pz; v[3] += px * px; v[4] += pz * pz;
+        v[5] = fmax(v[5], fabs(bb)); v[6] = fmax(v[6], fabs(px)); v[7] = fmax(v[7], fabs(pz));
     }
-    __shared__ double sh[5][256];
-    for (int k = 0; k < 5; k++) sh[k][threadIdx.x] = v[k];
+    __shared__ double sh[SRWD_COND][256];
+    for (int k = 0; k < SRWD_COND; k++) sh[k][threadIdx.x] = v[k];
     __syncthreads();
     for (int off = 128; off > 0; off >>= 1) {
         if ((int)threadIdx.x < off)
-            for (int k = 0; k < 5; k++) sh[k][threadIdx.x] += sh[k][threadIdx.x + off];
+            for (int k = 0; k < SRWD_COND; k++) {
+                const double a = sh[k][threadIdx.x], c = sh[k][threadIdx.x + off];
+                sh[k][threadIdx.x] = k < 5 ? a + c : fmax(a, c);
+            }
         __syncthreads();
     }
-    if (threadIdx.x < 5) cond[5 * tr + threadIdx.x] = sh[threadIdx.x][0];
+    if (threadIdx.x < SRWD_COND) cond[SRWD_COND * tr + threadIdx.x] = sh[threadIdx.x][0];
 }
 
 // One workgroup per (entry, part): an entry is (first item, 256-point block)
@@ -1217,7 +1231,7 @@ __global__ void __launch_bounds__(256) k_sr_finalize(const srwd_item* __restrict
     const srwd_req Rq = reqs[IT.traj];
     double sumSqX = 0., sumSqZ = 0.;
     if (cond) {
-        const double* c = cond + 5 * IT.traj;
+        const double* c = cond + SRWD_COND * IT.traj;
         double xo = coord[Rq.xOff + ix], zo = coord[Rq.zOff + iz];
         sumSqX = c[0] * xo * xo - 2. * xo * c[1] + c[3];
         sumSqZ = c[0] * zo * zo - 2. * zo * c[2] + c[4];
@@ -1537,12 +1551,13 @@ int srwd_launch_traj(const srwd_traj_job* dJobs, const srwd_field* dFields, int 
 int srwd_launch_tables(const srwd_trj_info* dInfo, int nTraj, long long maxInt, const double* dX,
                        const double* dXp, const double* dY, const double* dYp, long long ldT,
                        double* dIBx, double* dIBz, srwd_rec* dRec, srwd_chunk* dChunk, double* dQ,
-                       long long ldI, long long ldC, srwd_edge* dEdge, double* dT64, hipStream_t st)
+                       long long ldI, long long ldC, srwd_edge* dEdge, double* dT64, srwd_mrec* dMrec, long long ldM,
+                       hipStream_t st)
 {
     hipLaunchKernelGGL(k_quad_terms, dim3(2 * nTraj), dim3(SRWD_QT_THREADS), 0, st, dInfo, dXp, dYp, ldT, dIBx,
                        dIBz);
-    hipLaunchKernelGGL(k_sr_tables, dim3((unsigned)((maxInt + 255) / 256), nTraj), dim3(256), 0, st, dInfo,
-                       dX, dY, dIBx, dIBz, ldT, dRec, dChunk, dQ, ldI, ldC, maxInt, dT64);
+    hipLaunchKernelGGL(k_sr_tables, dim3((unsigned)((std::max(maxInt, ldM) + 255) / 256), nTraj), dim3(256), 0, st,
+                       dInfo, dX, dY, dIBx, dIBz, ldT, dRec, dChunk, dQ, ldI, ldC, dT64, dMrec, ldM);
     hipLaunchKernelGGL(k_sr_edges, dim3((2 * nTraj + 63) / 64), dim3(64), 0, st, dInfo, nTraj, dX, dY,
                        dIBx, dIBz, ldT, dEdge);
     return hipGetLastError() == hipSuccess ? 0 : -1;

@@ -45,6 +45,7 @@ struct Buffers {
     DBuf X, Xp, Y, Yp, IBx, IBz, Samp, Jobs, Fields, Info;
     DBuf Rec, Chunk, Q, Edge, Mesh, Rx, Items, BlockItem, RowTraj, RowE, RowN, A, Part, Warn;
     DBuf Cond, FpList, FpCount;   // condition check of the FP32 sums and its FP64 recomputation list
+    DBuf Mrec;                    // integration-point records of the mesh kernel
     DBuf T64;                     // FP64 trajectory values per integration point (FP64 recomputation)
     DBuf Req, Coord, BlkReq, Last;   // requests, observation coordinates, edge-derivative state
     DBuf SrBlocks;                // SR launch lists {item, block}

@@ -94,15 +94,38 @@ struct srwd_item {
     int npts;                 // nxc * nzc
     double actNorm;           // normalisation constant * eph * 0.80654658e-3
     int drow;                 // phase-table row of the energy step (energy tiles), -1 if none
-    int tiled;                // 1: computed by the energy-tile kernel (its FP32 error model differs)
+    int tiled;                // kernel of the item's sums (their error models differ): SRWD_ITEM_*
     double de;                // energy step of the request's mesh
 };
+
+// srwd_item::tiled: one energy per workgroup, energy tiles, matrix product
+#define SRWD_ITEM_POINT 0
+#define SRWD_ITEM_TILE 1
+#define SRWD_ITEM_MESH 2
 
 #define SRWD_CHUNK 256
 // Photon energies per workgroup of the energy-tile SR kernel (4 or 8): the
 // phasor of energy k is advanced from that of energy k - 1 by one complex
 // multiply.
 #define SRWD_TILE_E 8
+
+// Integration-point record of the mesh kernel (sr_mesh.hip): trajectory
+// position, 1/(yObs - s), s/gamma^2 + the integrals of the squared angles
+// (FP64) and the weighted 1/R^2 b with b times the projected positions, as in
+// srwd_rec.  Records past a trajectory's last integration point, up to the
+// leading dimension, are zero.
+struct srwd_mrec {
+    double X, Z, inv, sQ;
+    float b, bPx, bPz, pad;
+};
+// Mesh kernel: points of a tile along x and along z; integration points
+// between two flushes of its FP32 sums into FP64 (the unit in which an
+// s-range is split).  srwd_mesh_ld is the record count of a trajectory.
+#define SRWD_MESH_TILE 64
+#define SRWD_MESH_UNIT 64
+inline long long srwd_mesh_ld(long long nInt) { return (nInt + SRWD_MESH_UNIT - 1) / SRWD_MESH_UNIT * SRWD_MESH_UNIT; }
+// Doubles per trajectory of the condition sums (srwd_launch_cond_sums).
+#define SRWD_COND 8
 
 // One request of a field computation, for the parts that follow the
 // reference's point loop (rows, then columns, then photon energies of the
@@ -138,7 +161,8 @@ int srwd_launch_nz(srwd_trj_info* dInfo, int nTraj, const double* dX, const doub
 int srwd_launch_tables(const srwd_trj_info* dInfo, int nTraj, long long maxInt, const double* dX,
                        const double* dXp, const double* dY, const double* dYp, long long ldT,
                        double* dIBx, double* dIBz, srwd_rec* dRec, srwd_chunk* dChunk, double* dQ,
-                       long long ldI, long long ldC, srwd_edge* dEdge, double* dT64, hipStream_t st);
+                       long long ldI, long long ldC, srwd_edge* dEdge, double* dT64, srwd_mrec* dMrec, long long ldM,
+                       hipStream_t st);
 int srwd_launch_rx(const srwd_trj_info* dInfo, int nTraj, long long maxNp, const double* dX, const double* dY,
                    const double* dIBx, const double* dIBz, long long ldT, double* dSamp, const double* dMesh,
                    double* dRx, hipStream_t st);
@@ -184,6 +208,14 @@ int srwd_launch_sr_fused(const srwd_item* dItems, const int2* dBlocks, int nBloc
                          const srwd_trj_info* dInfo, const srwd_rec* dRec, const srwd_chunk* dChunk, const float* dA,
                          long long ldI, long long ldC, long long nPointsPad, double* dPart, const srwd_fuse& F,
                          hipStream_t st);
+// The sums of mesh items (sr_mesh.hip) over a list of tiles of
+// SRWD_MESH_TILE x SRWD_MESH_TILE points: dTiles[i] = {item, tile} with the
+// tiles of an item numbered along x, then z.  dRec: ldM records per
+// trajectory (srwd_mesh_ld of the longest, zero past a trajectory's end),
+// dCond: the condition sums.
+int srwd_launch_sr_mesh(const srwd_item* dItems, const int2* dTiles, int nTiles, const srwd_trj_info* dInfo,
+                        const srwd_mrec* dRec, long long ldM, const double* dCond, int nSplit, long long nPointsPad,
+                        double* dPart, hipStream_t st);
 // Edge-derivative state of the reference's point loop: per block of
 // SRWD_EDGE_BLOCK points of each request (dBlkReq: its request) and edge, the
 // last point at or before the block's end whose far-field expansion at that
@@ -194,7 +226,7 @@ int srwd_launch_edge_state(const srwd_req* dReq, int nReq, const int* dBlkReq, l
                            long long* dLast, hipStream_t st);
 // Entries (first item, 256-point block in the item) of groups of g items
 // (g consecutive photon energies of one request, g divides 256; 1 for single
-// items).  dCond (5 doubles per trajectory, from srwd_launch_cond_sums)
+// items).  dCond (SRWD_COND doubles per trajectory, from srwd_launch_cond_sums)
 // enables the condition check of the FP32 sums (estimated error <= condTol
 // of the point's field magnitude): points that fail it are appended to
 // dFpList (item's band-relative block * 256 + point in the block;

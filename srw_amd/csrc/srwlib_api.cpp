@@ -205,6 +205,35 @@ static int h2d(void* dst, const void* src, size_t bytes, hipStream_t st)
     return hipMemcpyAsync(dst, g_ctx.up + at, bytes, hipMemcpyHostToDevice, st) == hipSuccess ? 0 : SRWL_AMD_ERR_GPU;
 }
 
+// Tiles of the mesh kernel over nx x nz computed points.
+static int mesh_tiles(int nx, int nz)
+{
+    const int T = SRWD_MESH_TILE;
+    return ((nx + T - 1) / T) * ((nz + T - 1) / T);
+}
+
+// Whether the sums of a request over nxc x nzc computed points go to the mesh
+// kernel.
+static bool mesh_kernel_pays(int nxc, int nzc, int ne)
+{
+    (void)ne;
+    const long long T2 = SRWD_MESH_TILE * SRWD_MESH_TILE;
+    return mesh_tiles(nxc, nzc) * T2 <= 4LL * nxc * nzc;
+}
+
+// Parts of the s-range of a mesh pass of nTiles tiles and nPts points.
+static int mesh_split(long long nTiles, long long nUnits, long long nPts)
+{
+    int best = 1;
+    double bestT = 1e300;
+    for (long long n = 1; n <= std::min<long long>(nUnits, 128); n++) {
+        const double rounds = (double)((std::max(1LL, nTiles) * n + 511) / 512);
+        const double t = rounds * (double)((nUnits + n - 1) / n) * 4e-6 + (double)n * nPts * 64. / 4e12;
+        if (t < bestT * 0.98) { bestT = t; best = (int)n; }
+    }
+    return best;
+}
+
 // Runs the single-electron SR computation for a set of requests.  Outputs
 // stay on the device: request j writes ne*nx*ny complex values of Ex and Ez
 // starting at float2 offset outOff[j] of dEx / dEz.
@@ -334,10 +363,12 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     double* dMesh = (double*)B.Mesh.get(sizeof(double) * 4 * nT);
     double* dRx = (double*)B.Rx.get(sizeof(double) * 4 * nT);
     double* dT64 = g_ctx.condTol > 0 ? (double*)B.T64.get(sizeof(double) * SRWD_T64 * (size_t)ldI * nT) : nullptr;
-    if (!dRec || !dChunk || !dQ || !dEdge || !dMesh || !dRx || (g_ctx.condTol > 0 && !dT64))
+    const long long ldM = srwd_mesh_ld(maxInt);
+    srwd_mrec* dMrec = (srwd_mrec*)B.Mrec.get(sizeof(srwd_mrec) * (size_t)ldM * nT);
+    if (!dRec || !dChunk || !dQ || !dEdge || !dMesh || !dRx || !dMrec || (g_ctx.condTol > 0 && !dT64))
         return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
     if (srwd_launch_tables(dInfo, nT, maxInt, dX, dXp, dY, dYp, ldT, dIBx, dIBz, dRec, dChunk, dQ, ldI, ldC,
-                           dEdge, dT64, st))
+                           dEdge, dT64, dMrec, ldM, st))
         return SRWL_AMD_ERR_GPU;
     std::vector<double> meshLim(4 * nT);
     for (int j = 0; j < nT; j++) {
@@ -434,8 +465,16 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     std::vector<long long> rowN;
     const double normBase = 1. / 137.0360411;
     std::vector<int> rowBase(nT);
+    // requests whose mesh goes to the matrix-product kernel (no phase table)
+    std::vector<char> isMesh(nT);
+    bool allMesh = true;
+    for (int j = 0; j < nT; j++) {
+        isMesh[j] = mesh_kernel_pays(reqs[j].nxc, reqs[j].nzc, (int)jobs[j].mesh.ne);
+        allMesh = allMesh && isMesh[j];
+    }
     for (int j = 0; j < nT; j++) {
         rowBase[j] = (int)rowTraj.size();
+        if (isMesh[j]) continue;
         const SRWLRadMesh& m = jobs[j].mesh;
         for (int ie = 0; ie < (int)m.ne; ie++) {
             rowTraj.push_back(j); rowE.push_back(coord[reqs[j].eOff + ie]); rowN.push_back(info[j].nInt);
@@ -448,7 +487,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     std::vector<double> eStepOf(nT, 0.);
     for (int j = 0; j < nT; j++) {
         const SRWLRadMesh& m = jobs[j].mesh;
-        if (g_ctx.tileE < 2 || m.ne < g_ctx.tileE) continue;
+        if (isMesh[j] || g_ctx.tileE < 2 || m.ne < g_ctx.tileE) continue;
         eStepOf[j] = (m.eFin - m.eStart) / (m.ne - 1);
         dRowOf[j] = (int)rowTraj.size();
         rowTraj.push_back(j); rowE.push_back(eStepOf[j]); rowN.push_back(info[j].nInt);
@@ -469,10 +508,10 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     // download would be, the request has energy tiles, and one pass without
     // an s-range split fills the GPU.
     int nDl = 0;
-    if (nBands > 1 && g_ctx.streamRows && dRowOf[0] >= 0 && g_ctx.forceSplit <= 1) {
+    if (nBands > 1 && g_ctx.streamRows && (isMesh[0] || dRowOf[0] >= 0) && g_ctx.forceSplit <= 1) {
         SrRegion G = sr_region(jobs[0].mesh, info[0]);
         const long long ne = jobs[0].mesh.ne, blocks = ((long long)G.nxc * G.nzc + 255) / 256;
-        if ((ne / g_ctx.tileE + ne % g_ctx.tileE) * blocks >= 1024) {
+        if (isMesh[0] || (ne / g_ctx.tileE + ne % g_ctx.tileE) * blocks >= 1024) {
             // bands only set the copies' granularity here: more of them keep
             // the copy after the last flag short
             nDl = g_ctx.forceBands > 0 ? nBands : std::min(16, G.nzc);
@@ -482,11 +521,16 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     std::vector<srwd_item> items;
     std::vector<int> blockItem;
     std::vector<int> bandBlock0(nBands + 1, 0), bandRow0(nBands + 1, 0);
-    // SR launch lists: {item, block of the item}; tile blocks name the first
-    // item of a group of SRWD_TILE_E energies
-    std::vector<int2> tileBlocks, restBlocks;
+    // finalize lists: {item, block of the item}; tile blocks name the first
+    // item of a group of SRWD_TILE_E energies.  The sums have lists of their
+    // own: the same without the mesh items, and the mesh items' tiles.
+    std::vector<int2> tileBlocks, restBlocks, srTileBlocks, srRestBlocks, meshTiles;
     std::vector<int> bandTile0(nBands + 1, 0), bandRest0(nBands + 1, 0);
+    std::vector<int> bandSrTile0(nBands + 1, 0), bandSrRest0(nBands + 1, 0), bandMesh0(nBands + 1, 0);
     for (int b = 0; b < nBands; b++) {
+        bandMesh0[b] = (int)meshTiles.size();
+        bandSrTile0[b] = (int)srTileBlocks.size();
+        bandSrRest0[b] = (int)srRestBlocks.size();
         bandBlock0[b] = (int)blockItem.size();
         bandTile0[b] = (int)tileBlocks.size();
         bandRest0[b] = (int)restBlocks.size();
@@ -507,7 +551,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             if (r1 <= r0) continue;
             double normConst = std::sqrt(normBase * J.Iavg * 1.E+09 / 1.602189246E-19);
             const int tE = g_ctx.tileE;
-            const int nTiled = dRowOf[j] >= 0 ? (ne / tE) * tE : 0;
+            const int nTiled = dRowOf[j] >= 0 || (isMesh[j] && tE > 1) ? (ne / tE) * tE : 0;
             for (int ie = 0; ie < ne; ie++) {
                 srwd_item it;
                 std::memset(&it, 0, sizeof(it));
@@ -526,12 +570,20 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
                 it.actNorm = normConst * it.eph * 0.80654658E-03;
                 it.drow = dRowOf[j];
                 it.de = eStepOf[j];
-                it.tiled = ie < nTiled ? 1 : 0;
+                it.tiled = isMesh[j] ? SRWD_ITEM_MESH : (ie < nTiled ? SRWD_ITEM_TILE : SRWD_ITEM_POINT);
                 int nb = (it.npts + 255) / 256;
                 const int me = (int)items.size();
                 for (int q = 0; q < nb; q++) blockItem.push_back(me);
-                if (!it.tiled) for (int q = 0; q < nb; q++) restBlocks.push_back(make_int2(me, q));
+                if (ie >= nTiled) for (int q = 0; q < nb; q++) restBlocks.push_back(make_int2(me, q));
                 else if (ie % tE == 0) for (int q = 0; q < nb; q++) tileBlocks.push_back(make_int2(me, q));
+                if (isMesh[j]) {
+                    const int nt = mesh_tiles(G.nxc, r1 - r0);
+                    for (int q = 0; q < nt; q++) meshTiles.push_back(make_int2(me, q));
+                } else if (ie >= nTiled) {
+                    for (int q = 0; q < nb; q++) srRestBlocks.push_back(make_int2(me, q));
+                } else if (ie % tE == 0) {
+                    for (int q = 0; q < nb; q++) srTileBlocks.push_back(make_int2(me, q));
+                }
                 items.push_back(it);
             }
         }
@@ -539,11 +591,17 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     bandBlock0[nBands] = (int)blockItem.size();
     bandTile0[nBands] = (int)tileBlocks.size();
     bandRest0[nBands] = (int)restBlocks.size();
-    std::vector<int> dlRow0, dlLast;
+    bandMesh0[nBands] = (int)meshTiles.size();
+    bandSrTile0[nBands] = (int)srTileBlocks.size();
+    bandSrRest0[nBands] = (int)srRestBlocks.size();
+    std::vector<int> dlRow0, dlLast, dlTile0, dlRest0;
     if (nDl) {
-        // the tile blocks in row order (every energy group of a 256-point
-        // block before the next block), so that rows are finished in order
-        std::stable_sort(tileBlocks.begin(), tileBlocks.end(), [](int2 a, int2 b) { return a.y < b.y; });
+        // the blocks in row order (every energy group of a 256-point block
+        // before the next block), so that rows are finished in order
+        auto byRow = [](int2 a, int2 b) { return a.y < b.y; };
+        std::stable_sort(tileBlocks.begin(), tileBlocks.end(), byRow);
+        std::stable_sort(restBlocks.begin(), restBlocks.end(), byRow);
+        std::stable_sort(srTileBlocks.begin(), srTileBlocks.end(), byRow);
         SrRegion G = sr_region(jobs[0].mesh, info[0]);
         dlRow0.resize(nDl + 1);
         for (int q = 0; q <= nDl; q++)
@@ -561,6 +619,17 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             for (int q = bandOf(it.iz0 + p0 / it.nxc); q <= bandOf(it.iz0 + p1 / it.nxc); q++) dlLast[q] = i;
         }
         for (int q = 1; q < nDl; q++) dlLast[q] = std::max(dlLast[q], dlLast[q - 1]);
+        // first entry of each band in the finalize lists (entry i belongs to
+        // the first band whose rows start after its points do)
+        auto firstAt = [&](const std::vector<int2>& l, int row) {
+            const long long p = (long long)row * items[0].nxc;
+            return (int)(std::lower_bound(l.begin(), l.end(), p,
+                                          [](int2 a, long long v) { return (long long)a.y * 256 < v; }) - l.begin());
+        };
+        for (int q = 0; q <= nDl; q++) {
+            dlTile0.push_back(q ? firstAt(tileBlocks, dlRow0[q]) : 0);
+            dlRest0.push_back(q ? firstAt(restBlocks, dlRow0[q]) : 0);
+        }
         bandRow0 = dlRow0;
     }
     int nItems = (int)items.size();
@@ -570,18 +639,33 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     long long nPointsPad = (long long)nBlocks * 256;
     // split the integration range when a band's mesh alone does not fill the GPU
     long long minChunks = ldC;
-    for (auto& I : info) minChunks = std::min(minChunks, (I.nInt + SRWD_CHUNK - 1) / SRWD_CHUNK);
+    long long minUnits = ldM / SRWD_MESH_UNIT;
+    for (auto& I : info) {
+        minChunks = std::min(minChunks, (I.nInt + SRWD_CHUNK - 1) / SRWD_CHUNK);
+        minUnits = std::min(minUnits, srwd_mesh_ld(I.nInt) / SRWD_MESH_UNIT);
+    }
     // workgroups of a band: every block of the single-energy items, one per
     // group of SRWD_TILE_E energies for the tiles (the tile kernel's
     // workgroups each do SRWD_TILE_E times the work, so fewer fill the GPU)
-    const int nWG = (int)(tileBlocks.size() + restBlocks.size());
-    const int bandWG = (nWG + nBands - 1) / nBands;
-    const int wgTarget = tileBlocks.empty() ? 4096 : 1024;
-    int nSplit = (int)std::min<long long>(std::max<long long>(1, (wgTarget + bandWG - 1) / bandWG), minChunks);
+    const int nWG = (int)(srTileBlocks.size() + srRestBlocks.size());
+    int nSplit = 1;
+    if (allMesh) {
+        nSplit = mesh_split((long long)meshTiles.size() / nBands, minUnits, nPointsPad / nBands);
+        // a no-allocation call keeps its partial sums within what one block
+        // per 256 points would take
+        if (g_arena) nSplit = std::min(nSplit, std::max(1, 4096 / nBlocks));
+    } else {
+        const int bandWG = (nWG + nBands - 1) / nBands;
+        const int wgTarget = srTileBlocks.empty() ? 4096 : 1024;
+        nSplit = (int)std::min<long long>(std::max<long long>(1, (wgTarget + bandWG - 1) / bandWG), minChunks);
+    }
     if (g_ctx.forceSplit > 0) nSplit = (int)std::min<long long>(g_ctx.forceSplit, minChunks);
     srwd_item* dItems = (srwd_item*)B.Items.get(sizeof(srwd_item) * nItems);
     int* dBlockItem = (int*)B.BlockItem.get(sizeof(int) * nBlocks);
-    int2* dSrBlocks = (int2*)B.SrBlocks.get(sizeof(int2) * (size_t)std::max(1, nWG));
+    std::vector<int2> srLists;   // finalize lists, then the lists of the sums
+    for (auto* l : {&tileBlocks, &restBlocks, &srTileBlocks, &srRestBlocks, &meshTiles})
+        srLists.insert(srLists.end(), l->begin(), l->end());
+    int2* dSrBlocks = (int2*)B.SrBlocks.get(sizeof(int2) * srLists.size());
     int* dRowTraj = (int*)B.RowTraj.get(sizeof(int) * nRows);
     double* dRowE = (double*)B.RowE.get(sizeof(double) * nRows);
     long long* dRowN = (long long*)B.RowN.get(sizeof(long long) * nRows);
@@ -591,7 +675,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     // condition check of the FP32 sums and the FP64 recomputation list (one band at a time)
     int maxBandBlocks = 0;
     for (int b = 0; b < nBands; b++) maxBandBlocks = std::max(maxBandBlocks, bandBlock0[b + 1] - bandBlock0[b]);
-    double* dCond = (double*)B.Cond.get(sizeof(double) * 5 * nT);
+    double* dCond = (double*)B.Cond.get(sizeof(double) * SRWD_COND * nT);
     // one list per compute stream: consecutive bands run on alternate streams
     const int nLists = nBands > 1 ? 2 : 1;
     int* dFpList = (int*)B.FpList.get(sizeof(int) * 256 * (size_t)maxBandBlocks * nLists);
@@ -602,16 +686,16 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     if (int e_ = h2d(dItems, items.data(), sizeof(srwd_item) * nItems, st)) return e_;
     if (int e_ = h2d(dBlockItem, blockItem.data(), sizeof(int) * nBlocks, st)) return e_;
     int2* dTileBlocks = dSrBlocks;
-    int2* dRestBlocks = dSrBlocks + tileBlocks.size();
-    if (!tileBlocks.empty())
-        if (int e_ = h2d(dTileBlocks, tileBlocks.data(), sizeof(int2) * tileBlocks.size(), st)) return e_;
-    if (!restBlocks.empty())
-        if (int e_ = h2d(dRestBlocks, restBlocks.data(), sizeof(int2) * restBlocks.size(), st)) return e_;
+    int2* dRestBlocks = dTileBlocks + tileBlocks.size();
+    int2* dSrTile = dRestBlocks + restBlocks.size();
+    int2* dSrRest = dSrTile + srTileBlocks.size();
+    int2* dMeshTiles = dSrRest + srRestBlocks.size();
+    if (int e_ = h2d(dSrBlocks, srLists.data(), sizeof(int2) * srLists.size(), st)) return e_;
     if (int e_ = h2d(dRowTraj, rowTraj.data(), sizeof(int) * nRows, st)) return e_;
     if (int e_ = h2d(dRowE, rowE.data(), sizeof(double) * nRows, st)) return e_;
     if (int e_ = h2d(dRowN, rowN.data(), sizeof(long long) * nRows, st)) return e_;
     HIPCHK(hipMemsetAsync(dWarn, 0, sizeof(int), st));
-    if (srwd_launch_phase_table(dQ, ldI, dRowTraj, dRowE, dRowN, nRows, maxInt, dA, st)) return SRWL_AMD_ERR_GPU;
+    if (nRows > 0 && srwd_launch_phase_table(dQ, ldI, dRowTraj, dRowE, dRowN, nRows, maxInt, dA, st)) return SRWL_AMD_ERR_GPU;
     if (srwd_launch_cond_sums(dInfo, nT, dRec, ldI, dCond, st)) return SRWL_AMD_ERR_GPU;
     HIPCHK(hipMemsetAsync(dFpCount, 0, sizeof(int) * (size_t)nBands, st));
     g_ctx.lastSrBlocks = nBlocks;
@@ -662,7 +746,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         // --- streamed rows (see above) ---------------------------------------
         pin = pinned_staging(2 * compBytes);
         if (!pin) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
-        const int nTile = (int)tileBlocks.size(), nRest = (int)restBlocks.size();
+        const int nTile = (int)srTileBlocks.size(), nRest = (int)srRestBlocks.size();
         if ((size_t)nTile > g_ctx.blockDoneCap) {
             if (g_ctx.blockDone) (void)hipHostFree(g_ctx.blockDone);
             g_ctx.blockDone = nullptr;
@@ -694,11 +778,47 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             g_ctx.bandEv.push_back(e);
         }
         const double* cnd = g_ctx.condTol > 0 ? dCond : nullptr;
+        auto copy_band = [&](int b) -> int {   // band b into the pinned staging, its event after it
+            int r[4];
+            rows_of_band(b, r);
+            for (int k = 0; k < 4; k += 2) {
+                if (r[k + 1] <= r[k]) continue;
+                size_t o = rowBytes * r[k], n = rowBytes * (r[k + 1] - r[k]);
+                HIPCHK(hipMemcpyAsync(pin + o, (char*)dEx + o, n, hipMemcpyDeviceToHost, g_ctx.copyStream));
+                HIPCHK(hipMemcpyAsync(pin + compBytes + o, (char*)dEz + o, n, hipMemcpyDeviceToHost,
+                                      g_ctx.copyStream));
+            }
+            HIPCHK(hipEventRecord(g_ctx.bandEv[4 * b + 1], g_ctx.copyStream));
+            return 0;
+        };
+        if (!meshTiles.empty()) {
+            // mesh items: the sums of the whole field are short against its
+            // download, so one launch forms them and the finalize pass runs
+            // band by band, each band's copy queued behind it
+            if (g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev0, st));
+            if (srwd_launch_sr_mesh(dItems, dMeshTiles, (int)meshTiles.size(), dInfo, dMrec, ldM, dCond, nSplit,
+                                    nPointsPad, dPart, st))
+                return SRWL_AMD_ERR_GPU;
+            if (g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev1, st));
+            for (int b = 0; b < nDl; b++) {
+                if (srwd_launch_finalize(dItems, dTileBlocks + dlTile0[b], dlTile0[b + 1] - dlTile0[b],
+                                         std::max(1, g_ctx.tileE), dInfo, dEdge, termin, dPart, nSplit, nPointsPad, dEx,
+                                         dEz, dWarn, cnd, g_ctx.condTol, dFpList, dFpCount, dReq, dCoord, dLast, st) ||
+                    srwd_launch_finalize(dItems, dRestBlocks + dlRest0[b], dlRest0[b + 1] - dlRest0[b], 1, dInfo, dEdge,
+                                         termin, dPart, nSplit, nPointsPad, dEx, dEz, dWarn, cnd, g_ctx.condTol, dFpList,
+                                         dFpCount, dReq, dCoord, dLast, st))
+                    return SRWL_AMD_ERR_GPU;
+                HIPCHK(hipEventRecord(g_ctx.bandEv[4 * b], st));
+                HIPCHK(hipStreamWaitEvent(g_ctx.copyStream, g_ctx.bandEv[4 * b], 0));
+                rc = copy_band(b);
+                if (rc) return rc;
+            }
+        } else {
         // the single-energy items (energies left over from the groups) on the
         // second stream, finished there by the two-pass form
         HIPCHK(hipEventRecord(g_ctx.evFork, st));
         HIPCHK(hipStreamWaitEvent(g_ctx.stream2, g_ctx.evFork, 0));
-        if (srwd_launch_sr(dItems, dRestBlocks, nRest, 0, dInfo, dRec, dChunk, dA, ldI, ldC, 1, nPointsPad, dPart,
+        if (srwd_launch_sr(dItems, dSrRest, nRest, 0, dInfo, dRec, dChunk, dA, ldI, ldC, 1, nPointsPad, dPart,
                            g_ctx.stream2) ||
             srwd_launch_finalize(dItems, dRestBlocks, nRest, 1, dInfo, dEdge, termin, dPart, 1, nPointsPad, dEx, dEz,
                                  dWarn, cnd, g_ctx.condTol, dFpList, dFpCount, dReq, dCoord, dLast, g_ctx.stream2))
@@ -709,12 +829,13 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         F.cond = cnd; F.condTol = g_ctx.condTol; F.fpList = dFpList; F.fpCount = dFpCount;
         F.reqs = dReq; F.coord = dCoord; F.last = dLast; F.blockDone = g_ctx.blockDone; F.epoch = epoch;
         if (g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev0, st));
-        if (srwd_launch_sr_fused(dItems, dTileBlocks, nTile, g_ctx.tileE, dInfo, dRec, dChunk, dA, ldI, ldC,
+        if (srwd_launch_sr_fused(dItems, dSrTile, nTile, g_ctx.tileE, dInfo, dRec, dChunk, dA, ldI, ldC,
                                  nPointsPad, dPart, F, st))
             return SRWL_AMD_ERR_GPU;
         if (g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev1, st));
         HIPCHK(hipEventRecord(g_ctx.evTiles, st));
         HIPCHK(hipStreamWaitEvent(st, g_ctx.evJoin, 0));
+        }
         // FP64 recomputation, every store also recorded for the host
         if (g_ctx.condTol > 0 &&
             srwd_launch_sr_fp64(dItems, dBlockItem, dInfo, dEdge, termin, dT64, ldI, dEx, dEz, dWarn, dFpList,
@@ -742,22 +863,19 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         const auto t0 = std::chrono::steady_clock::now();
         bool late = false;
         int cursor = 0, nextDl = 0, nextCopy = 0;
+        if (!meshTiles.empty())
+            for (; nextCopy < nDl; nextCopy++) {
+                HIPCHK(hipEventSynchronize(g_ctx.bandEv[4 * nextCopy + 1]));
+                host_copy_band(nextCopy);
+            }
         for (unsigned spin = 0; nextCopy < nDl && !late;) {
             while (cursor < nTile && done[cursor] == epoch) cursor++;
             bool progress = false;
             while (nextDl < nDl && cursor > dlLast[nextDl]) {
                 const int b = nextDl++;
                 if (b == 0) HIPCHK(hipStreamWaitEvent(g_ctx.copyStream, g_ctx.evJoin, 0));
-                int r[4];
-                rows_of_band(b, r);
-                for (int k = 0; k < 4; k += 2) {
-                    if (r[k + 1] <= r[k]) continue;
-                    size_t o = rowBytes * r[k], n = rowBytes * (r[k + 1] - r[k]);
-                    HIPCHK(hipMemcpyAsync(pin + o, (char*)dEx + o, n, hipMemcpyDeviceToHost, g_ctx.copyStream));
-                    HIPCHK(hipMemcpyAsync(pin + compBytes + o, (char*)dEz + o, n, hipMemcpyDeviceToHost,
-                                          g_ctx.copyStream));
-                }
-                HIPCHK(hipEventRecord(g_ctx.bandEv[4 * b + 1], g_ctx.copyStream));
+                rc = copy_band(b);
+                if (rc) return rc;
                 progress = true;
             }
             if (nextCopy < nextDl && hipEventQuery(g_ctx.bandEv[4 * nextCopy + 1]) == hipSuccess) {
@@ -815,15 +933,18 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             const int nTile = bandTile0[b + 1] - bandTile0[b], nRest = bandRest0[b + 1] - bandRest0[b];
             // an unbanded pass runs the few single-energy blocks on the second
             // stream, beside the energy tiles, instead of after them
-            const bool side = nBands == 1 && nTile > 0 && nRest > 0;
+            const int nSrTile = bandSrTile0[b + 1] - bandSrTile0[b], nSrRest = bandSrRest0[b + 1] - bandSrRest0[b];
+            const bool side = nBands == 1 && nSrTile > 0 && nSrRest > 0;
             if (side) {
                 HIPCHK(hipEventRecord(g_ctx.evFork, sb));
                 HIPCHK(hipStreamWaitEvent(g_ctx.stream2, g_ctx.evFork, 0));
             }
-            if (srwd_launch_sr(dItems, dRestBlocks + bandRest0[b], nRest, 0, dInfo, dRec, dChunk, dA, ldI, ldC, nSplit,
+            if (srwd_launch_sr(dItems, dSrRest + bandSrRest0[b], nSrRest, 0, dInfo, dRec, dChunk, dA, ldI, ldC, nSplit,
                                nPointsPad, dPart, side ? g_ctx.stream2 : sb) ||
-                srwd_launch_sr(dItems, dTileBlocks + bandTile0[b], nTile, g_ctx.tileE, dInfo, dRec, dChunk, dA, ldI,
-                               ldC, nSplit, nPointsPad, dPart, sb))
+                srwd_launch_sr(dItems, dSrTile + bandSrTile0[b], nSrTile, g_ctx.tileE, dInfo, dRec, dChunk, dA, ldI,
+                               ldC, nSplit, nPointsPad, dPart, sb) ||
+                srwd_launch_sr_mesh(dItems, dMeshTiles + bandMesh0[b], bandMesh0[b + 1] - bandMesh0[b], dInfo, dMrec,
+                                    ldM, dCond, nSplit, nPointsPad, dPart, sb))
                 return SRWL_AMD_ERR_GPU;
             if (side) {
                 HIPCHK(hipEventRecord(g_ctx.evJoin, g_ctx.stream2));
