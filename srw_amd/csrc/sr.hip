@@ -14,7 +14,6 @@
 // 256-point chunk, chunk sums in FP64.  A condition check of every point's
 // FP32 sum sends ill-conditioned points to an FP64 recomputation.
 #include "srw_sr_dev.h"
-#include <algorithm>
 
 // ------------------------------------------------------------------------
 // Field and RK4 (FP64)
@@ -647,8 +646,16 @@ __global__ void __launch_bounds__(256) k_sr_tables(const srwd_trj_info* __restri
     long long gi = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     int tr = blockIdx.y;
     const srwd_trj_info I = info[tr];
+    // record groups of the mesh kernel, x side and z side
+    srwd_mrec* const Mx = M + 2 * tr * ldM + (gi >> 3);
+    srwd_mrec* const Mz = Mx + ldM;
+    const int gl = (int)(gi & 7);
     if (gi >= I.nInt) {
-        if (gi < ldM) M[tr * ldM + gi] = srwd_mrec{0., 0., 0., 0., 0.f, 0.f, 0.f, 0.f};
+        if (gi >= 8 * ldM) return;
+        for (srwd_mrec* m : {Mx, Mz}) {
+            if (gl == 0 && (gi & ~7LL) >= I.nInt) m->crd = m->inv = m->q = 0.;
+            m->dq[gl] = m->du[gl] = m->di[gl] = m->b[gl] = m->p[gl] = 0.f;
+        }
         return;
     }
     bool byDiv = I.nInt < 10000;   // srradint.h:1046-1050: manual "faster" below 10000 points
@@ -692,7 +699,21 @@ __global__ void __launch_bounds__(256) k_sr_tables(const srwd_trj_info* __restri
     R.bPx = (float)(bd * Pxd);
     R.bPz = (float)(bd * Pzd);
     rec[tr * ldI + gi] = R;
-    M[tr * ldM + gi] = srwd_mrec{Xv, Zv, inv, s * I.gammaEm2 + IB, R.b, R.bPx, R.bPz, 0.f};
+    {
+        // increments from the group's reference point, which one of each 8
+        // neighbouring lanes holds
+        const int ref = (gi | 7) - 3 < I.nInt ? 4 : 0;
+        const int l0 = ((threadIdx.x & 63) & ~7) + ref;
+        const double sQ = s * I.gammaEm2 + IB, qx = sQ + Xv * U, qz = Zv * V;
+        const double dqx = qx - __shfl(qx, l0, 64), dqz = qz - __shfl(qz, l0, 64);
+        const double dU = U - __shfl(U, l0, 64), dV = V - __shfl(V, l0, 64), di = inv - __shfl(inv, l0, 64);
+        if (gl == ref) {
+            Mx->crd = Xv; Mx->inv = inv; Mx->q = sQ;
+            Mz->crd = Zv; Mz->inv = inv; Mz->q = 0.;
+        }
+        Mx->dq[gl] = (float)dqx; Mx->du[gl] = (float)dU; Mx->di[gl] = (float)di; Mx->p[gl] = (float)Pxd;
+        Mz->dq[gl] = (float)dqz; Mz->du[gl] = (float)dV; Mz->di[gl] = (float)di; Mz->p[gl] = (float)Pzd;
+    }
     Qout[tr * ldI + gi] = Q;
     // FP64 trajectory values at the point, for the FP64 recomputation of
     // ill-conditioned points (k_sr_fp64)
@@ -1054,7 +1075,7 @@ __global__ void __launch_bounds__(256) k_sr_integral_tile(const srwd_item* __res
                 const srwd_req Rq = F.reqs[Ie.traj];
                 double sumSqX = 0., sumSqZ = 0.;
                 if (F.cond) {
-                    const double* c = F.cond + SRWD_COND * Ie.traj;
+                    const double* c = F.cond + 5 * Ie.traj;
                     const double xr = F.coord[Rq.xOff + ix], zr = F.coord[Rq.zOff + iz];
                     sumSqX = c[0] * xr * xr - 2. * xr * c[1] + c[3];
                     sumSqZ = c[0] * zr * zr - 2. * zr * c[2] + c[4];
@@ -1094,7 +1115,7 @@ __global__ void __launch_bounds__(256) k_sr_integral_tile(const srwd_item* __res
 #define SRWD_EPS_TERM_TILE 4e-6
 // Mesh items (sr_mesh.hip): phases reduced in FP64 before their sine and
 // cosine, phasors as FP16 pairs of about 22 bits.
-#define SRWD_EPS_TERM_MESH 1e-6
+#define SRWD_EPS_TERM_MESH 2e-6
 
 // Terminating terms, the derivative correction, the float store and the
 // mirrored parts of one point; S = sum over the integration points of
@@ -1170,32 +1191,49 @@ __device__ void sr_finish_point(const srwd_item& IT, const srwd_trj_info& I, con
 // Sums of squared terms per trajectory, from the integration records:
 // cond[0..4] = sum b^2, sum b bPx, sum b bPz, sum bPx^2, sum bPz^2, so that
 // the squared x terms of point (xo, zo) add up to
-// cond[0] xo^2 - 2 xo cond[1] + cond[3] (and the z terms likewise); and the
-// largest |b|, |bPx| and |bPz| in cond[5..7].
-__global__ void __launch_bounds__(256) k_cond_sums(const srwd_trj_info* __restrict__ info,
-                                                   const srwd_rec* __restrict__ rec, long long ldI, double* cond)
+// cond[0] xo^2 - 2 xo cond[1] + cond[3] (and the z terms likewise).  The
+// largest |b|, |bPx| and |bPz| give the amplitude scales of the mesh records.
+#define SRWD_CS_THREADS 512
+__global__ void __launch_bounds__(SRWD_CS_THREADS) k_cond_sums(const srwd_trj_info* __restrict__ info,
+                                                               const srwd_rec* __restrict__ rec, long long ldI,
+                                                               double* cond, srwd_mrec* M, long long ldM,
+                                                               const double* __restrict__ mesh, double* scale)
 {
     int tr = blockIdx.x;
     long long n = info[tr].nInt;
     const srwd_rec* R = rec + (long long)tr * ldI;
-    double v[SRWD_COND] = {0, 0, 0, 0, 0, 0, 0, 0};
+    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (long long i = threadIdx.x; i < n; i += blockDim.x) {
         double bb = R[i].b, px = R[i].bPx, pz = R[i].bPz;
         v[0] += bb * bb; v[1] += bb * px; v[2] += bb * pz; v[3] += px * px; v[4] += pz * pz;
         v[5] = fmax(v[5], fabs(bb)); v[6] = fmax(v[6], fabs(px)); v[7] = fmax(v[7], fabs(pz));
     }
-    __shared__ double sh[SRWD_COND][256];
-    for (int k = 0; k < SRWD_COND; k++) sh[k][threadIdx.x] = v[k];
-    __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off)
-            for (int k = 0; k < SRWD_COND; k++) {
-                const double a = sh[k][threadIdx.x], c = sh[k][threadIdx.x + off];
-                sh[k][threadIdx.x] = k < 5 ? a + c : fmax(a, c);
-            }
-        __syncthreads();
+    __shared__ double sh[SRWD_CS_THREADS / 64][8];
+    const int lane = threadIdx.x & 63;
+    for (int k = 0; k < 8; k++) {
+        double x = v[k];
+        for (int off = 32; off > 0; off >>= 1) {
+            const double y = __shfl_xor(x, off, 64);
+            x = k < 5 ? x + y : fmax(x, y);
+        }
+        if (lane == 0) sh[threadIdx.x >> 6][k] = x;
     }
-    if (threadIdx.x < SRWD_COND) cond[SRWD_COND * tr + threadIdx.x] = sh[threadIdx.x][0];
+    __syncthreads();
+    for (int k = 0; k < 8; k++) {
+        double x = sh[0][k];
+        for (int q = 1; q < SRWD_CS_THREADS / 64; q++) x = k < 5 ? x + sh[q][k] : fmax(x, sh[q][k]);
+        v[k] = x;
+    }
+    if (threadIdx.x < 5) cond[5 * tr + threadIdx.x] = v[threadIdx.x];
+    const double* ml = mesh + 4 * tr;
+    for (int side = 0; side < 2; side++) {
+        const double a = v[5] * fmax(fabs(ml[2 * side]), fabs(ml[2 * side + 1])) + v[6 + side];
+        const int e = a > 0. ? 11 - ilogb(a) : 0;
+        const double f = ldexp(1., e);
+        srwd_mrec* m = M + (2 * tr + side) * ldM;
+        for (long long i = threadIdx.x; i < n; i += blockDim.x) m[i >> 3].b[i & 7] = (float)(R[i].b * f);
+        if (threadIdx.x == 0) scale[2 * tr + side] = ldexp(1., -e);
+    }
 }
 
 // One workgroup per (entry, part): an entry is (first item, 256-point block)
@@ -1231,7 +1269,7 @@ __global__ void __launch_bounds__(256) k_sr_finalize(const srwd_item* __restrict
     const srwd_req Rq = reqs[IT.traj];
     double sumSqX = 0., sumSqZ = 0.;
     if (cond) {
-        const double* c = cond + SRWD_COND * IT.traj;
+        const double* c = cond + 5 * IT.traj;
         double xo = coord[Rq.xOff + ix], zo = coord[Rq.zOff + iz];
         sumSqX = c[0] * xo * xo - 2. * xo * c[1] + c[3];
         sumSqZ = c[0] * zo * zo - 2. * zo * c[2] + c[4];
@@ -1244,49 +1282,53 @@ __global__ void __launch_bounds__(256) k_sr_finalize(const srwd_item* __restrict
 // FP64 sums of one point over the integration points of its trajectory
 // table T (n entries of SRWD_T64 doubles): the trajectory interpolated at
 // each point as the reference's manual methods do (srradint.cpp:1214-1258,
-// 1379-1604), the phase reduced and its sine and cosine taken with the
-// reference's Taylor series, the weights 7, 16, 14, ..., 16, 7 in units of
-// h/15.  With T and n uniform over the wave the table is read by scalar
+// 1379-1604), with the reference's Taylor sine and cosine and the weights
+// 7, 16, 14, ..., 16, 7 in units of h/15.  With T and n uniform over the wave the table is read by scalar
 // loads, once per wave.
 // List length from which k_sr_fp64 gives each point one lane (below it, one
 // wave): about where a serial walk of 10^4 integration points per lane costs
 // as much as the per-point table reads of the wave-per-point form.
 #define SRWD_FP64_LANE_MIN 32768
 
-// Branch-free form of cos_sin_taylor (the same operations on the taken path,
-// so the same results).
-__device__ __forceinline__ void cos_sin_taylor_sel(double x, double& c, double& s)
+// cos_sin_taylor in fewer operations: the same polynomials on the same reduced
+// argument within +/-PI/2 (the reference's PI, which its end terms reduce
+// with too), a rounding to the nearest multiple of PI in place of the
+// comparisons, odd multiples changing both signs.
+__device__ __forceinline__ void cos_sin_taylor_sel(double a, double& c, double& s)
 {
-    const double PI = 3.141592653590, TwoPI = 2. * PI, ThreePIdTwo = 1.5 * PI, HalfPI = 0.5 * PI;
-    const double One_dTwoPI = 1. / TwoPI;
-    const double a2c = -0.5, a4c = 1. / 24., a6c = -1. / 720., a8c = 1. / 40320., a10c = -1. / 3628800.;
-    const double a3s = -1. / 6., a5s = 1. / 120., a7s = -1. / 5040., a9s = 1. / 362880., a11s = -1. / 39916800.;
-    x -= TwoPI * (double)(int)(x * One_dTwoPI);
-    x = x < 0. ? x + TwoPI : x;
-    const bool hi = x > ThreePIdTwo, chs = !hi && x > HalfPI;
-    x = hi ? x - TwoPI : (chs ? x - PI : x);
-    double x2 = x * x;
-    c = 1. + x2 * (a2c + x2 * (a4c + x2 * (a6c + x2 * (a8c + x2 * a10c))));
-    s = x * (1. + x2 * (a3s + x2 * (a5s + x2 * (a7s + x2 * (a9s + x2 * a11s)))));
-    c = chs ? -c : c;
-    s = chs ? -s : s;
+    const double PI = 3.141592653590;
+    const double n = rint(a * (1. / PI)), x = fma(-n, PI, a), y = x * x;
+    double q = fma(y, -1. / 3628800., 1. / 40320.), p = fma(y, -1. / 39916800., 1. / 362880.);
+    q = fma(y, q, -1. / 720.);
+    p = fma(y, p, -1. / 5040.);
+    q = fma(y, q, 1. / 24.);
+    p = fma(y, p, 1. / 120.);
+    q = fma(y, q, -0.5);
+    p = fma(y, p, -1. / 6.);
+    const double cs = fma(y, q, 1.), sn = x * fma(y, p, 1.);
+    const int sg = (int)((unsigned)(int)n << 31);
+    c = __hiloint2double(__double2hiint(cs) ^ sg, __double2loint(cs));
+    s = __hiloint2double(__double2hiint(sn) ^ sg, __double2loint(sn));
+}
+
+// One term of the FP64 sums: kph is the phase constant, T the trajectory values of integration point i of n.
+template <typename TP>
+__device__ __forceinline__ void fp64_term(TP T, int i, int n, double xo, double zo, double kph, double* acc)
+{
+    const double dx = xo - T[0], dz = zo - T[1], inv = T[5];
+    double c, sn;
+    cos_sin_taylor_sel(kph * fma(fma(dx, dx, dz * dz), inv, T[4]), c, sn);
+    const double wi = ((i == 0 || i == n - 1) ? 7. : ((i & 1) ? 16. : 14.)) * inv;
+    const double ax = wi * fma(-dx, inv, T[2]), az = wi * fma(-dz, inv, T[3]);
+    acc[0] = fma(ax, c, acc[0]); acc[1] = fma(ax, sn, acc[1]);
+    acc[2] = fma(az, c, acc[2]); acc[3] = fma(az, sn, acc[3]);
 }
 
 template <typename TP>
 __device__ __forceinline__ void fp64_point_sums(TP T, int n, double xo, double zo, double kph, double* acc)
 {
 #pragma unroll 2
-    for (int i = 0; i < n; i++) {
-        const int o = i * SRWD_T64;
-        double Xv = T[o], Zv = T[o + 1], Btx = T[o + 2], Btz = T[o + 3], sQ = T[o + 4], inv = T[o + 5];
-        double dx = xo - Xv, dz = zo - Zv;
-        double ph = kph * (sQ + (dx * dx + dz * dz) * inv);
-        double c, sn;
-        cos_sin_taylor_sel(ph, c, sn);
-        double wt = (i == 0 || i == n - 1) ? 7. : ((i & 1) ? 16. : 14.);
-        double ax = wt * ((Btx - dx * inv) * inv), az = wt * ((Btz - dz * inv) * inv);
-        acc[0] += ax * c; acc[1] += ax * sn; acc[2] += az * c; acc[3] += az * sn;
-    }
+    for (int i = 0; i < n; i++) fp64_term(T + i * SRWD_T64, i, n, xo, zo, kph, acc);
 }
 
 __device__ __forceinline__ const double* wave_first_ptr(const double* p)
@@ -1333,20 +1375,11 @@ __global__ void __launch_bounds__(256) k_sr_fp64(const srwd_item* __restrict__ i
             int ix = local % IT.nxc, iz = IT.iz0 + local / IT.nxc;
             const srwd_req& Rq = reqs[IT.traj];
             double xo = coord[Rq.xOff + ix], zo = coord[Rq.zOff + iz];
-            double kph = SRWD_KPH(IT.eph);
+            const double kph = SRWD_KPH(IT.eph);
             const double* T = T64 + (long long)IT.traj * ldI * SRWD_T64;
             double acc[4] = {0, 0, 0, 0};
-            for (long long i = lane; i < I.nInt; i += 64) {
-                const double* t = T + i * SRWD_T64;
-                double Xv = t[0], Zv = t[1], Btx = t[2], Btz = t[3], sQ = t[4], inv = t[5];
-                double dx = xo - Xv, dz = zo - Zv;
-                double ph = kph * (sQ + (dx * dx + dz * dz) * inv);
-                double c, sn;
-                cos_sin_taylor(ph, c, sn);
-                double wt = (i == 0 || i == I.nInt - 1) ? 7. : ((i & 1) ? 16. : 14.);
-                double ax = wt * ((Btx - dx * inv) * inv), az = wt * ((Btz - dz * inv) * inv);
-                acc[0] += ax * c; acc[1] += ax * sn; acc[2] += az * c; acc[3] += az * sn;
-            }
+            for (int i = lane; i < (int)I.nInt; i += 64)
+                fp64_term(T + (long long)i * SRWD_T64, i, (int)I.nInt, xo, zo, kph, acc);
             for (int m = 0; m < 4; m++)
                 for (int off = 32; off > 0; off >>= 1) acc[m] += __shfl_down(acc[m], off);
             if (lane == 0)
@@ -1368,7 +1401,7 @@ __global__ void __launch_bounds__(256) k_sr_fp64(const srwd_item* __restrict__ i
                 int ix = local % IT.nxc, iz = IT.iz0 + local / IT.nxc;
                 const srwd_req& Rq = reqs[IT.traj];
                 double xo = coord[Rq.xOff + ix], zo = coord[Rq.zOff + iz];
-                double kph = SRWD_KPH(IT.eph);
+                const double kph = SRWD_KPH(IT.eph);
                 const double* T = T64 + (long long)IT.traj * ldI * SRWD_T64;
                 const int n = (int)I.nInt;
                 double acc[4] = {0, 0, 0, 0};
@@ -1430,7 +1463,7 @@ __global__ void __launch_bounds__(256) k_sr_fp64_sums(const srwd_item* __restric
             int ix = local % IT.nxc, iz = IT.iz0 + local / IT.nxc;
             const srwd_req& Rq = reqs[traj];
             double xo = coord[Rq.xOff + ix], zo = coord[Rq.zOff + iz];
-            double kph = SRWD_KPH(IT.eph);
+            const double kph = SRWD_KPH(IT.eph);
             const double* T = T64 + (long long)traj * ldI * SRWD_T64;
             const int n = (int)info[traj].nInt;
             double acc[4] = {0, 0, 0, 0};
@@ -1556,7 +1589,7 @@ int srwd_launch_tables(const srwd_trj_info* dInfo, int nTraj, long long maxInt, 
 {
     hipLaunchKernelGGL(k_quad_terms, dim3(2 * nTraj), dim3(SRWD_QT_THREADS), 0, st, dInfo, dXp, dYp, ldT, dIBx,
                        dIBz);
-    hipLaunchKernelGGL(k_sr_tables, dim3((unsigned)((std::max(maxInt, ldM) + 255) / 256), nTraj), dim3(256), 0, st,
+    hipLaunchKernelGGL(k_sr_tables, dim3((unsigned)((8 * ldM + 255) / 256), nTraj), dim3(256), 0, st,
                        dInfo, dX, dY, dIBx, dIBz, ldT, dRec, dChunk, dQ, ldI, ldC, dT64, dMrec, ldM);
     hipLaunchKernelGGL(k_sr_edges, dim3((2 * nTraj + 63) / 64), dim3(64), 0, st, dInfo, nTraj, dX, dY,
                        dIBx, dIBz, ldT, dEdge);
@@ -1623,9 +1656,10 @@ int srwd_launch_finalize(const srwd_item* dItems, const int2* dEntries, int nEnt
 }
 
 int srwd_launch_cond_sums(const srwd_trj_info* dInfo, int nTraj, const srwd_rec* dRec, long long ldI, double* dCond,
-                          hipStream_t st)
+                          srwd_mrec* dMrec, long long ldM, const double* dMesh, double* dScale, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_cond_sums, dim3(nTraj), dim3(256), 0, st, dInfo, dRec, ldI, dCond);
+    hipLaunchKernelGGL(k_cond_sums, dim3(nTraj), dim3(SRWD_CS_THREADS), 0, st, dInfo, dRec, ldI, dCond, dMrec, ldM,
+                       dMesh, dScale);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

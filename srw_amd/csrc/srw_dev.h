@@ -109,23 +109,29 @@ struct srwd_item {
 // multiply.
 #define SRWD_TILE_E 8
 
-// Integration-point record of the mesh kernel (sr_mesh.hip): trajectory
-// position, 1/(yObs - s), s/gamma^2 + the integrals of the squared angles
-// (FP64) and the weighted 1/R^2 b with b times the projected positions, as in
-// srwd_rec.  Records past a trajectory's last integration point, up to the
-// leading dimension, are zero.
+// Integration-point records of the mesh kernel (sr_mesh.hip) for one side (x
+// or z) of a trajectory, in groups of 8 consecutive points: at the group's
+// reference point (the fifth, or the first where the trajectory ends before
+// it) the position, 1/(yObs - s) and the phase terms that do not
+// depend on the observation point (q = s/gamma^2 + the integrals of the
+// squared angles on the x side, 0 on the z side); per point the increments of
+// q + crd^2/(yObs - s), crd/(yObs - s) and 1/(yObs - s) from the reference point,
+// the weighted 1/R^2 b of srwd_rec times the side's amplitude scale, and the
+// projected position.  Points past the last integration point are zero.
 struct srwd_mrec {
-    double X, Z, inv, sQ;
-    float b, bPx, bPz, pad;
+    double crd, inv, q, pad;
+    float dq[8], du[8], di[8], b[8], p[8];
 };
 // Mesh kernel: points of a tile along x and along z; integration points
 // between two flushes of its FP32 sums into FP64 (the unit in which an
-// s-range is split).  srwd_mesh_ld is the record count of a trajectory.
+// s-range is split).  srwd_mesh_ld is the group count of a side
 #define SRWD_MESH_TILE 64
-#define SRWD_MESH_UNIT 64
-inline long long srwd_mesh_ld(long long nInt) { return (nInt + SRWD_MESH_UNIT - 1) / SRWD_MESH_UNIT * SRWD_MESH_UNIT; }
-// Doubles per trajectory of the condition sums (srwd_launch_cond_sums).
-#define SRWD_COND 8
+#define SRWD_MESH_UNIT 32
+// (whole units and one more stage of 16, which the kernel reads ahead).
+inline long long srwd_mesh_ld(long long nInt)
+{
+    return (nInt + SRWD_MESH_UNIT - 1) / SRWD_MESH_UNIT * (SRWD_MESH_UNIT / 8) + 2;
+}
 
 // One request of a field computation, for the parts that follow the
 // reference's point loop (rows, then columns, then photon energies of the
@@ -210,11 +216,11 @@ int srwd_launch_sr_fused(const srwd_item* dItems, const int2* dBlocks, int nBloc
                          hipStream_t st);
 // The sums of mesh items (sr_mesh.hip) over a list of tiles of
 // SRWD_MESH_TILE x SRWD_MESH_TILE points: dTiles[i] = {item, tile} with the
-// tiles of an item numbered along x, then z.  dRec: ldM records per
-// trajectory (srwd_mesh_ld of the longest, zero past a trajectory's end),
-// dCond: the condition sums.
+// tiles of an item numbered along x, then z.  dRec: the two
+// sides of every trajectory, ldM groups each (srwd_mesh_ld of the longest);
+// dScale: the inverse amplitude scales of the two sides, 2 per trajectory.
 int srwd_launch_sr_mesh(const srwd_item* dItems, const int2* dTiles, int nTiles, const srwd_trj_info* dInfo,
-                        const srwd_mrec* dRec, long long ldM, const double* dCond, int nSplit, long long nPointsPad,
+                        const srwd_mrec* dRec, long long ldM, const double* dScale, int nSplit, long long nPointsPad,
                         double* dPart, hipStream_t st);
 // Edge-derivative state of the reference's point loop: per block of
 // SRWD_EDGE_BLOCK points of each request (dBlkReq: its request) and edge, the
@@ -226,7 +232,7 @@ int srwd_launch_edge_state(const srwd_req* dReq, int nReq, const int* dBlkReq, l
                            long long* dLast, hipStream_t st);
 // Entries (first item, 256-point block in the item) of groups of g items
 // (g consecutive photon energies of one request, g divides 256; 1 for single
-// items).  dCond (SRWD_COND doubles per trajectory, from srwd_launch_cond_sums)
+// items).  dCond (5 doubles per trajectory, from srwd_launch_cond_sums)
 // enables the condition check of the FP32 sums (estimated error <= condTol
 // of the point's field magnitude): points that fail it are appended to
 // dFpList (item's band-relative block * 256 + point in the block;
@@ -237,8 +243,12 @@ int srwd_launch_finalize(const srwd_item* dItems, const int2* dEntries, int nEnt
                          int nSplit, long long nPointsPad, float* dEx, float* dEz, int* dWarn, const double* dCond,
                          double condTol, int* dFpList, int* dFpCount, const srwd_req* dReq, const double* dCoord,
                          const long long* dLast, hipStream_t st);
+// It also scales the mesh records' b (see srwd_mrec) so that the largest
+// amplitude of a side over the integration points and the request's mesh
+// (dMesh: xStart, xEnd, zStart, zEnd per trajectory) lies in [2^11, 2^12),
+// and writes the inverse scales (powers of two) to dScale.
 int srwd_launch_cond_sums(const srwd_trj_info* dInfo, int nTraj, const srwd_rec* dRec, long long ldI, double* dCond,
-                          hipStream_t st);
+                          srwd_mrec* dMrec, long long ldM, const double* dMesh, double* dScale, hipStream_t st);
 // FP64 recomputation and store of the listed points (block indices relative
 // to dBlockItem, as passed to srwd_launch_finalize).
 // dT64: FP64 trajectory values (X, Z, X', Z', integral of the squared angles)

@@ -364,7 +364,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     double* dRx = (double*)B.Rx.get(sizeof(double) * 4 * nT);
     double* dT64 = g_ctx.condTol > 0 ? (double*)B.T64.get(sizeof(double) * SRWD_T64 * (size_t)ldI * nT) : nullptr;
     const long long ldM = srwd_mesh_ld(maxInt);
-    srwd_mrec* dMrec = (srwd_mrec*)B.Mrec.get(sizeof(srwd_mrec) * (size_t)ldM * nT);
+    srwd_mrec* dMrec = (srwd_mrec*)B.Mrec.get(sizeof(srwd_mrec) * 2 * (size_t)ldM * nT);
     if (!dRec || !dChunk || !dQ || !dEdge || !dMesh || !dRx || !dMrec || (g_ctx.condTol > 0 && !dT64))
         return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
     if (srwd_launch_tables(dInfo, nT, maxInt, dX, dXp, dY, dYp, ldT, dIBx, dIBz, dRec, dChunk, dQ, ldI, ldC,
@@ -642,7 +642,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     long long minUnits = ldM / SRWD_MESH_UNIT;
     for (auto& I : info) {
         minChunks = std::min(minChunks, (I.nInt + SRWD_CHUNK - 1) / SRWD_CHUNK);
-        minUnits = std::min(minUnits, srwd_mesh_ld(I.nInt) / SRWD_MESH_UNIT);
+        minUnits = std::min(minUnits, (I.nInt + SRWD_MESH_UNIT - 1) / SRWD_MESH_UNIT);
     }
     // workgroups of a band: every block of the single-energy items, one per
     // group of SRWD_TILE_E energies for the tiles (the tile kernel's
@@ -675,7 +675,8 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     // condition check of the FP32 sums and the FP64 recomputation list (one band at a time)
     int maxBandBlocks = 0;
     for (int b = 0; b < nBands; b++) maxBandBlocks = std::max(maxBandBlocks, bandBlock0[b + 1] - bandBlock0[b]);
-    double* dCond = (double*)B.Cond.get(sizeof(double) * SRWD_COND * nT);
+    double* dCond = (double*)B.Cond.get(sizeof(double) * 7 * nT);
+    double* dScale = dCond + 5 * nT;   // inverse amplitude scales of the mesh records, 2 per trajectory
     // one list per compute stream: consecutive bands run on alternate streams
     const int nLists = nBands > 1 ? 2 : 1;
     int* dFpList = (int*)B.FpList.get(sizeof(int) * 256 * (size_t)maxBandBlocks * nLists);
@@ -696,7 +697,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     if (int e_ = h2d(dRowN, rowN.data(), sizeof(long long) * nRows, st)) return e_;
     HIPCHK(hipMemsetAsync(dWarn, 0, sizeof(int), st));
     if (nRows > 0 && srwd_launch_phase_table(dQ, ldI, dRowTraj, dRowE, dRowN, nRows, maxInt, dA, st)) return SRWL_AMD_ERR_GPU;
-    if (srwd_launch_cond_sums(dInfo, nT, dRec, ldI, dCond, st)) return SRWL_AMD_ERR_GPU;
+    if (srwd_launch_cond_sums(dInfo, nT, dRec, ldI, dCond, dMrec, ldM, dMesh, dScale, st)) return SRWL_AMD_ERR_GPU;
     HIPCHK(hipMemsetAsync(dFpCount, 0, sizeof(int) * (size_t)nBands, st));
     g_ctx.lastSrBlocks = nBlocks;
     g_ctx.lastSrSplit = nSplit;
@@ -796,7 +797,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             // download, so one launch forms them and the finalize pass runs
             // band by band, each band's copy queued behind it
             if (g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev0, st));
-            if (srwd_launch_sr_mesh(dItems, dMeshTiles, (int)meshTiles.size(), dInfo, dMrec, ldM, dCond, nSplit,
+            if (srwd_launch_sr_mesh(dItems, dMeshTiles, (int)meshTiles.size(), dInfo, dMrec, ldM, dScale, nSplit,
                                     nPointsPad, dPart, st))
                 return SRWL_AMD_ERR_GPU;
             if (g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev1, st));
@@ -944,7 +945,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
                 srwd_launch_sr(dItems, dSrTile + bandSrTile0[b], nSrTile, g_ctx.tileE, dInfo, dRec, dChunk, dA, ldI,
                                ldC, nSplit, nPointsPad, dPart, sb) ||
                 srwd_launch_sr_mesh(dItems, dMeshTiles + bandMesh0[b], bandMesh0[b + 1] - bandMesh0[b], dInfo, dMrec,
-                                    ldM, dCond, nSplit, nPointsPad, dPart, sb))
+                                    ldM, dScale, nSplit, nPointsPad, dPart, sb))
                 return SRWL_AMD_ERR_GPU;
             if (side) {
                 HIPCHK(hipEventRecord(g_ctx.evJoin, g_ctx.stream2));
