@@ -156,7 +156,13 @@ extern "C" {
 // trajectories of up to ld points (512 threads per trajectory).
 inline long long srwd_pic_cap(long long ld) { return ((ld - 1 + 511) / 512) * 512 + 1; }
 
-// dScratch (20*srwd_pic_cap(ld) doubles per trajectory) selects the
+// Sweeps of the parallel-in-s RK4 that are launched (planar-undulator chains
+// converge in 7-8).
+#define SRWD_SW_MAX 11
+// Scratch of the parallel-in-s RK4, in doubles per trajectory.
+inline long long srwd_traj_scratch(long long ld) { return 20 * srwd_pic_cap(ld) + 2 * (SRWD_SW_MAX + 1) * 12; }
+
+// dScratch (srwd_traj_scratch(ld) doubles per trajectory) selects the
 // parallel-in-s solver; nullptr runs the serial kernel.
 // singleHarmonic: every field of dFields is one undulator with one harmonic.
 int srwd_launch_traj(const srwd_traj_job* dJobs, const srwd_field* dFields, int nTraj, double* dX,

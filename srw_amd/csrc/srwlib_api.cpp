@@ -334,7 +334,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         // user-supplied trajectories are re-uploaded after the RK pass overwrote them
         double* dPic = nullptr;
         if (!g_ctx.trajSerial) {
-            dPic = (double*)B.Pic.get(sizeof(double) * 20 * (size_t)srwd_pic_cap(ldT) * nT);
+            dPic = (double*)B.Pic.get(sizeof(double) * (size_t)srwd_traj_scratch(ldT) * nT);
             if (!dPic) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
         }
         int one = 1;
@@ -1406,7 +1406,7 @@ SRWL_EXPORT int srwlCalcPartTraj(SRWLPrtTrj* pTrj, SRWLMagFldC* pMagFld, double*
     HIPCHK(hipMemcpyAsync(dF, &f, sizeof(f), hipMemcpyHostToDevice, st));
     double* dPic = nullptr;
     if (!g_ctx.trajSerial) {
-        dPic = (double*)B.Pic.get(sizeof(double) * 20 * (size_t)srwd_pic_cap(pTrj->np));
+        dPic = (double*)B.Pic.get(sizeof(double) * (size_t)srwd_traj_scratch(pTrj->np));
         if (!dPic) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
     }
     int one = (f.n == 1 && f.u[0].nh == 1);

@@ -1,0 +1,85 @@
+"""The matrix-product SR kernel (64 x 64 point tiles of four 32 x 32 parts,
+integration points in groups of 8 and units of 32) against the FP64 oracle, at
+mesh sizes around the tile, at integration ranges around the group and the
+unit, and on both sides of the rule that chooses it.
+
+Tolerance: a term carries about 2e-7 of its magnitude (phase, sine, FP16 pair)
+and the terms add like a random walk, so a field that is not far below the sum
+of its terms agrees to about 1e-6; 1e-5 rel-L2 of both components together
+leaves a factor of 10 and is a tenth of the path's contract (1e-4)."""
+import numpy as np
+import pytest
+
+from srw_amd import workloads as W
+from tests import oracle_lib as oracle
+from tests.util import cfield, clone_wfr
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+
+
+def _error(w, mag, prec):
+    from srw_amd import srwlpy
+    wg, wo = clone_wfr(w), clone_wfr(w)
+    srwlpy.CalcElecFieldSR(wg, 0, mag, prec)
+    assert oracle.calc_field(wo, mag, prec) == 0
+    d = n = 0.
+    for c in ("arEx", "arEy"):
+        g, o = cfield(getattr(wg, c), wg), cfield(getattr(wo, c), wo)
+        d += np.linalg.norm(g - o) ** 2
+        n += np.linalg.norm(o) ** 2
+    return float(np.sqrt(d / n))
+
+
+def _case(nx, ny, ne=1, nper=12, np_traj=1201, tilt=False):
+    kw = dict(x=2e-5, xp=3e-6, y=-1e-5, yp=1e-6) if tilt else {}
+    beam = W.electron_beam(**kw)
+    e = W.first_harmonic_eV(beam.partStatMom1.gamma, 1.5, 0.02)
+    w = W.wavefront(beam, ne, 0.99 * e, 1.01 * e if ne > 1 else 0.99 * e, nx, ny, 1e-3, 0.7e-3, 20.)
+    return w, W.planar_undulator(1.5, 0.02, nper), W.traj_prec(np_traj, nper=nper)
+
+
+@pytest.mark.parametrize("nx,ny", [(32, 32), (33, 65), (64, 64), (65, 63), (128, 31), (40, 97), (16, 16), (200, 5)])
+def test_mesh_sizes_around_a_tile(nx, ny):
+    """The last two are too small or too narrow for the kernel: the per-point one."""
+    print("case:", nx, ny, flush=True)
+    e = _error(*_case(nx, ny, tilt=True))
+    print("rel-L2 %.2e" % e, flush=True)
+    assert e < TOL
+
+
+@pytest.mark.parametrize("n", [9, 31, 33, 35, 65, 67, 129])
+def test_integration_points_around_a_unit(n):
+    """n integration points: the step lies between the values at which the
+    count changes, where its rounding would decide the count."""
+    print("case:", n, flush=True)
+    w, mag, prec = _case(48, 40, nper=1, np_traj=301, tilt=True)
+    prec[1] = 2. * (0.5 * 0.02 + 4 * 0.02) / (n - 0.5)
+    e = _error(w, mag, prec)
+    print("rel-L2 %.2e" % e, flush=True)
+    assert e < TOL
+
+
+@pytest.mark.parametrize("ne", [3, 8, 11])
+def test_several_energies_and_mirror_symmetry(ne):
+    print("case:", ne, flush=True)
+    e = _error(*_case(70, 45, ne=ne))
+    print("rel-L2 %.2e" % e, flush=True)
+    assert e < TOL
+
+
+def test_batch_mixes_both_kernels():
+    """Requests on both sides of the rule in one batch, against single calls."""
+    from srw_amd import srwlpy
+    ws, ms, prec = [], [], None
+    for nx, ny in ((64, 40), (12, 9), (33, 100), (150, 2)):
+        w, m, prec = _case(nx, ny, tilt=True)
+        ws.append(w)
+        ms.append(m)
+    wb = [clone_wfr(w) for w in ws]
+    srwlpy.CalcElecFieldSRBatch(wb, ms, prec)
+    for w, m, b in zip(ws, ms, wb):
+        srwlpy.CalcElecFieldSR(w, 0, m, prec)
+        g, o = cfield(b.arEx, b), cfield(w.arEx, w)
+        assert np.linalg.norm(g - o) < 1e-6 * np.linalg.norm(o)
