@@ -817,68 +817,111 @@ __device__ __forceinline__ double interp_cub_half(const double* f, int i)
 }
 
 // Cumulative Simpson of the squared angle, zeroed at s0 (srtrjdat.cpp:1724-1805).
-// One 256-thread block per (trajectory, plane): the interval terms are formed
-// in parallel and summed with a block prefix scan.  Interval i (1-based) uses
-// the half-step cubic interpolant centred on nodes (i-1, i); as in the
-// reference, the first interval's left end term is 0.
+// Interval i (1-based) uses the half-step cubic interpolant centred on nodes
+// (i-1, i); as in the reference, the first interval's left end term is 0.
+// Two launches over blocks of SRWD_QT_THREADS points: the block totals of both
+// planes (and the zero-field flags), then each block's scan behind the totals
+// of the blocks before it.  One block per plane, walking its 10001 points in
+// segments, took 55 us, the flags 25 us; the two launches take 9 us.
 #define SRWD_QT_THREADS 256
-__global__ void __launch_bounds__(SRWD_QT_THREADS) k_quad_terms(const srwd_trj_info* __restrict__ info,
-                                                                const double* Xp, const double* Yp, long long ld,
+
+__device__ __forceinline__ double angle_term(const double* ang, long long i, long long n1, double stepMult)
+{
+    if (i < 1 || i > n1) return 0.;
+    const double* p;
+    int mid;
+    if (i == 1) { p = ang; mid = -1; }
+    else if (i < n1) { p = ang + (i - 2); mid = 0; }
+    else { p = ang + (n1 - 3); mid = 1; }
+    const double a = interp_cub_half(p, mid), f0 = (i == 1) ? 0. : ang[i - 1] * ang[i - 1];
+    return stepMult * (f0 + 4. * a * a + ang[i] * ang[i]);
+}
+
+// Sum over the block, known to every thread (sh: one value per wave).
+__device__ __forceinline__ double block_sum(double x, double* sh)
+{
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = x;
+    __syncthreads();
+    x = sh[0];
+    for (int q = 1; q < SRWD_QT_THREADS / 64; q++) x += sh[q];
+    return x;
+}
+
+// Totals of both planes per block (tot[2 * (tr * nb + b) + plane]) and
+// srtrjdat.cpp:2048-2062: a plane is treated as moving when any position or
+// angle sample is non-zero (the flags start at zero).
+__global__ void __launch_bounds__(SRWD_QT_THREADS) k_angle_totals(srwd_trj_info* info, const double* X, const double* Xp,
+                                                                  const double* Y, const double* Yp, long long ld,
+                                                                  double* tot)
+{
+    __shared__ double sh[SRWD_QT_THREADS / 64];
+    const int tr = blockIdx.y;
+    const long long np = info[tr].np, i = (long long)blockIdx.x * SRWD_QT_THREADS + threadIdx.x, o = tr * ld + i;
+    const double stepMult = 0.333333333333 * (0.5 * info[tr].sStep);
+    bool v = false, h = false;
+    if (i < np) {
+        v = X[o] != 0. || Xp[o] != 0.;
+        h = Y[o] != 0. || Yp[o] != 0.;
+    }
+    if (__any(v) && (threadIdx.x & 63) == 0) atomicOr(&info[tr].verNZ, 1);
+    if (__any(h) && (threadIdx.x & 63) == 0) atomicOr(&info[tr].horNZ, 1);
+    for (int pl = 0; pl < 2; pl++) {
+        const double t = block_sum(angle_term((pl ? Yp : Xp) + tr * ld, i, np - 1, stepMult), sh);
+        if (threadIdx.x == 0) tot[2 * ((long long)tr * gridDim.x + blockIdx.x) + pl] = t;
+    }
+}
+
+__global__ void __launch_bounds__(SRWD_QT_THREADS) k_angle_scan(const srwd_trj_info* __restrict__ info, const double* Xp,
+                                                                const double* Yp, long long ld, const double* tot,
                                                                 double* IBx, double* IBz)
 {
-    const int tr = blockIdx.x >> 1, pl = blockIdx.x & 1;
+    __shared__ double sh[SRWD_QT_THREADS / 64], inc[SRWD_QT_THREADS / 64];
+    const int tr = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const srwd_trj_info I = info[tr];
-    const double* ang = (pl == 0 ? Xp : Yp) + tr * ld;
-    double* out = (pl == 0 ? IBx : IBz) + tr * ld;
-    const long long np = I.np, n1 = np - 1;
-    const double stepMult = 0.333333333333 * (0.5 * I.sStep);
-    const int T = SRWD_QT_THREADS;
-    long long seg = (n1 + T - 1) / T;
-    long long i0 = 1 + threadIdx.x * seg, i1 = i0 + seg;
-    if (i1 > n1 + 1) i1 = n1 + 1;
-    auto term = [&](long long i) {
-        const double* p;
-        int mid;
-        if (i == 1) { p = ang; mid = -1; }
-        else if (i < n1) { p = ang + (i - 2); mid = 0; }
-        else { p = ang + (n1 - 3); mid = 1; }
-        double a = interp_cub_half(p, mid);
-        double f0 = (i == 1) ? 0. : ang[i - 1] * ang[i - 1];
-        return stepMult * (f0 + 4. * a * a + ang[i] * ang[i]);
-    };
-    double loc = 0.;
-    for (long long i = i0; i < i1; i++) loc += term(i);
-    __shared__ double sc[SRWD_QT_THREADS];
-    __shared__ double sv;
-    sc[threadIdx.x] = loc;
-    __syncthreads();
-    for (int off = 1; off < T; off <<= 1) {
-        double v = threadIdx.x >= off ? sc[threadIdx.x - off] : 0.;
+    const long long np = I.np, n1 = np - 1, i = (long long)blockIdx.x * SRWD_QT_THREADS + threadIdx.x;
+    if ((long long)blockIdx.x * SRWD_QT_THREADS >= np) return;
+    const double sStep = I.sStep, stepMult = 0.333333333333 * (0.5 * sStep);
+    // the integral's value at s0 is interpolated from six nodes, off .. off + 5
+    long long idx = (long long)((I.s0 - I.sStart) / sStep);
+    if (idx >= np - 1) idx = np - 2; else if (idx < 0) idx = 0;
+    double rel = I.s0 - (I.sStart + sStep * idx);
+    long long off;
+    if (idx < 2) { off = 0; rel -= (2 - idx) * sStep; }
+    else if (idx < np - 3) off = idx - 2;
+    else if (idx < np - 2) { off = idx - 3; rel += sStep; }
+    else { off = idx - 4; rel += 2 * sStep; }
+    const long long bo = off / SRWD_QT_THREADS;
+    for (int pl = 0; pl < 2; pl++) {
+        const double* ang = (pl ? Yp : Xp) + tr * ld;
+        const double* tt = tot + 2 * (long long)tr * gridDim.x + pl;
+        double before = 0., node = 0.;
+        for (long long b = threadIdx.x; b < gridDim.x; b += SRWD_QT_THREADS) {
+            const double t = tt[2 * b];
+            if (b < blockIdx.x) before += t;
+            if (b < bo) node += t;
+        }
+        const long long in = bo * SRWD_QT_THREADS + threadIdx.x;
+        if (in <= off) node += angle_term(ang, in, n1, stepMult);
+        double x = angle_term(ang, i, n1, stepMult);
+        for (int o = 1; o < 64; o <<= 1) {
+            const double u = __shfl_up(x, o, 64);
+            if (lane >= o) x += u;
+        }
+        before = block_sum(before, sh);
+        node = block_sum(node, sh);
         __syncthreads();
-        sc[threadIdx.x] += v;
+        if (lane == 63) inc[w] = x;
         __syncthreads();
+        for (int q = 0; q < w; q++) x += inc[q];
+        double f[6], c[6];
+        f[0] = node;
+        for (int k = 1; k < 6; k++) f[k] = f[k - 1] + angle_term(ang, off + k, n1, stepMult);
+        coefs5(sStep, f, c);
+        const double sv = c[0] + rel * (c[1] + rel * (c[2] + rel * (c[3] + rel * (c[4] + rel * c[5]))));
+        if (i < np) (pl ? IBz : IBx)[tr * ld + i] = (before + x) - sv;
     }
-    double run = threadIdx.x > 0 ? sc[threadIdx.x - 1] : 0.;
-    if (threadIdx.x == 0) out[0] = 0.;
-    for (long long i = i0; i < i1; i++) { run += term(i); out[i] = run; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double sStep = I.sStep;
-        long long idx = (long long)((I.s0 - I.sStart) / sStep);
-        if (idx >= np - 1) idx = np - 2; else if (idx < 0) idx = 0;
-        double rel = I.s0 - (I.sStart + sStep * idx);
-        long long off;
-        if (idx < 2) { off = 0; rel -= (2 - idx) * sStep; }
-        else if (idx < np - 3) off = idx - 2;
-        else if (idx < np - 2) { off = idx - 3; rel += sStep; }
-        else { off = idx - 4; rel += 2 * sStep; }
-        double c[6];
-        coefs5(sStep, out + off, c);
-        sv = c[0] + rel * (c[1] + rel * (c[2] + rel * (c[3] + rel * (c[4] + rel * c[5]))));
-    }
-    __syncthreads();
-    double v = sv;
-    for (long long j = threadIdx.x; j <= n1; j += T) out[j] -= v;
 }
 
 __device__ __forceinline__ double int_point_s(const srwd_trj_info& I, long long i)
@@ -886,7 +929,21 @@ __device__ __forceinline__ double int_point_s(const srwd_trj_info& I, long long 
     return (i == I.nInt - 1) ? I.sIntegFin : I.sIntegStart + (double)i * I.h;
 }
 
-// Integration-point tables.  One thread per (trajectory, integration point).
+// Edge data at the integration limits (srtrjdat.h:1006-1034), end 0 or 1.
+__device__ __forceinline__ void sr_edge(const srwd_trj_info& I, const double* cx, const double* cz, const double* ix,
+                                        const double* iz, int end, srwd_edge& E)
+{
+    const double s = end ? I.sIntegFin : I.sIntegStart;
+    const trj_pt px = eval_plane(I, cx, ix, -1. / I.betaNorm, s, true), pz = eval_plane(I, cz, iz, 1. / I.betaNorm, s, true);
+    double* v = E.v[end];
+    v[0] = px.dbds; v[1] = px.b; v[2] = px.bt; v[3] = px.crd; v[4] = px.ib;
+    v[5] = pz.dbds; v[6] = pz.b; v[7] = pz.bt; v[8] = pz.crd; v[9] = pz.ib;
+}
+
+// Integration-point tables.  One thread per (trajectory, integration point);
+// the blocks past nTab form the samples of the radius search (srtrjdat.cpp:
+// 1416-1460: the polynomials are used regardless of the zero-field flags) and,
+// the last one, the edge data, so that one launch serves all three.
 // Writes the FP32 record, the FP64 phase base Q_i and, for the first point of
 // each chunk, the FP64 chunk reference.
 __global__ void __launch_bounds__(256) k_sr_tables(const srwd_trj_info* __restrict__ info,
@@ -894,11 +951,26 @@ __global__ void __launch_bounds__(256) k_sr_tables(const srwd_trj_info* __restri
                                                    const double* IBz, long long ldT,
                                                    srwd_rec* rec, srwd_chunk* chunk, double* Qout,
                                                    long long ldI, long long ldC, double* T64, srwd_mrec* M,
-                                                   long long ldM)
+                                                   long long ldM, int nTab, double* samp, srwd_edge* edges)
 {
     long long gi = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     int tr = blockIdx.y;
     const srwd_trj_info I = info[tr];
+    if ((int)blockIdx.x >= nTab) {
+        const double* sx = X + tr * ldT; const double* sz = Y + tr * ldT;
+        const double* jx = IBx + tr * ldT; const double* jz = IBz + tr * ldT;
+        if (blockIdx.x == gridDim.x - 1) {
+            if (threadIdx.x < 2) sr_edge(I, sx, sz, jx, jz, threadIdx.x, edges[tr]);
+            return;
+        }
+        const long long i = (long long)(blockIdx.x - nTab) * blockDim.x + threadIdx.x;
+        if (i >= I.np) return;
+        const double s = I.sStart + (double)i * I.sStep;
+        const trj_pt px = eval_plane(I, sx, jx, -1. / I.betaNorm, s, true), pz = eval_plane(I, sz, jz, 1. / I.betaNorm, s, true);
+        double* o = samp + tr * ldT * 4;
+        o[i] = px.bt; o[ldT + i] = pz.bt; o[2 * ldT + i] = px.crd; o[3 * ldT + i] = pz.crd;
+        return;
+    }
     // record groups of the mesh kernel, x side and z side
     srwd_mrec* const Mx = M + 2 * tr * ldM + (gi >> 3);
     srwd_mrec* const Mz = Mx + ldM;
@@ -978,22 +1050,6 @@ __global__ void __launch_bounds__(256) k_sr_tables(const srwd_trj_info* __restri
         srwd_chunk C; C.inv = inv; C.U = U; C.V = V; C.pad = 0;
         chunk[tr * ldC + gi / SRWD_CHUNK] = C;
     }
-}
-
-// Edge data at the integration limits (srtrjdat.h:1006-1034).  One thread per (trajectory, end).
-__global__ void k_sr_edges(const srwd_trj_info* __restrict__ info, int nTraj, const double* X, const double* Y,
-                           const double* IBx, const double* IBz, long long ldT, srwd_edge* edges)
-{
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    int tr = t >> 1, end = t & 1;
-    if (tr >= nTraj) return;
-    const srwd_trj_info I = info[tr];
-    double s = end ? I.sIntegFin : I.sIntegStart;
-    trj_pt px = eval_plane(I, X + tr * ldT, IBx + tr * ldT, -1. / I.betaNorm, s, true);
-    trj_pt pz = eval_plane(I, Y + tr * ldT, IBz + tr * ldT, 1. / I.betaNorm, s, true);
-    double* v = edges[tr].v[end];
-    v[0] = px.dbds; v[1] = px.b; v[2] = px.bt; v[3] = px.crd; v[4] = px.ib;
-    v[5] = pz.dbds; v[6] = pz.b; v[7] = pz.bt; v[8] = pz.crd; v[9] = pz.ib;
 }
 
 // Phase table A[row][i] = frac(K'*Q_i) with K' the phase constant in
@@ -1446,7 +1502,7 @@ __device__ void sr_finish_point(const srwd_item& IT, const srwd_trj_info& I, con
 // the squared x terms of point (xo, zo) add up to
 // cond[0] xo^2 - 2 xo cond[1] + cond[3] (and the z terms likewise).  The
 // largest |b|, |bPx| and |bPz| give the amplitude scales of the mesh records.
-#define SRWD_CS_THREADS 512
+#define SRWD_CS_THREADS 1024
 __global__ void __launch_bounds__(SRWD_CS_THREADS) k_cond_sums(const srwd_trj_info* __restrict__ info,
                                                                const srwd_rec* __restrict__ rec, long long ldI,
                                                                double* cond, srwd_mrec* M, long long ldM,
@@ -1846,18 +1902,20 @@ int srwd_launch_traj(const srwd_traj_job* dJobs, const srwd_field* dFields, int 
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int srwd_launch_tables(const srwd_trj_info* dInfo, int nTraj, long long maxInt, const double* dX,
+int srwd_launch_tables(srwd_trj_info* dInfo, int nTraj, const double* dX,
                        const double* dXp, const double* dY, const double* dYp, long long ldT,
                        double* dIBx, double* dIBz, srwd_rec* dRec, srwd_chunk* dChunk, double* dQ,
                        long long ldI, long long ldC, srwd_edge* dEdge, double* dT64, srwd_mrec* dMrec, long long ldM,
-                       hipStream_t st)
+                       double* dSamp, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_quad_terms, dim3(2 * nTraj), dim3(SRWD_QT_THREADS), 0, st, dInfo, dXp, dYp, ldT, dIBx,
+    const unsigned nb = (unsigned)((ldT + SRWD_QT_THREADS - 1) / SRWD_QT_THREADS);
+    // the samples are written after the totals have been used
+    hipLaunchKernelGGL(k_angle_totals, dim3(nb, nTraj), dim3(SRWD_QT_THREADS), 0, st, dInfo, dX, dXp, dY, dYp, ldT, dSamp);
+    hipLaunchKernelGGL(k_angle_scan, dim3(nb, nTraj), dim3(SRWD_QT_THREADS), 0, st, dInfo, dXp, dYp, ldT, dSamp, dIBx,
                        dIBz);
-    hipLaunchKernelGGL(k_sr_tables, dim3((unsigned)((8 * ldM + 255) / 256), nTraj), dim3(256), 0, st,
-                       dInfo, dX, dY, dIBx, dIBz, ldT, dRec, dChunk, dQ, ldI, ldC, dT64, dMrec, ldM);
-    hipLaunchKernelGGL(k_sr_edges, dim3((2 * nTraj + 63) / 64), dim3(64), 0, st, dInfo, nTraj, dX, dY,
-                       dIBx, dIBz, ldT, dEdge);
+    const unsigned nTab = (unsigned)((8 * ldM + 255) / 256);
+    hipLaunchKernelGGL(k_sr_tables, dim3(nTab + (unsigned)((ldT + 255) / 256) + 1, nTraj), dim3(256), 0, st, dInfo, dX, dY,
+                       dIBx, dIBz, ldT, dRec, dChunk, dQ, ldI, ldC, dT64, dMrec, ldM, (int)nTab, dSamp, dEdge);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -1957,47 +2015,8 @@ int srwd_launch_edge_state(const srwd_req* dReq, int nReq, const int* dBlkReq, l
 }  // extern "C"
 
 // ------------------------------------------------------------------------
-// Zero-field flags and wavefront radius
+// Wavefront radius
 // ------------------------------------------------------------------------
-// srtrjdat.cpp:2048-2062: a plane is treated as moving when any position or
-// angle sample is non-zero.  One block per trajectory.
-__global__ void __launch_bounds__(256) k_nz_flags(srwd_trj_info* info, const double* X, const double* Xp,
-                                                  const double* Y, const double* Yp, long long ld)
-{
-    int tr = blockIdx.x;
-    long long np = info[tr].np;
-    __shared__ int fv, fh;
-    if (threadIdx.x == 0) { fv = 0; fh = 0; }
-    __syncthreads();
-    int v = 0, h = 0;
-    for (long long i = threadIdx.x; i < np; i += blockDim.x) {
-        long long o = tr * ld + i;
-        v |= (X[o] != 0. || Xp[o] != 0.);
-        h |= (Y[o] != 0. || Yp[o] != 0.);
-    }
-    if (v) atomicOr(&fv, 1);
-    if (h) atomicOr(&fh, 1);
-    __syncthreads();
-    if (threadIdx.x == 0) { info[tr].verNZ = fv; info[tr].horNZ = fh; }
-}
-
-// Trajectory samples for the radius search (srtrjdat.cpp:1416-1460: the
-// polynomials are used regardless of the zero-field flags).
-__global__ void __launch_bounds__(256) k_rx_samples(const srwd_trj_info* __restrict__ info, const double* X,
-                                                    const double* Y, const double* IBx, const double* IBz,
-                                                    long long ldT, double* samp, long long ldS)
-{
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    int tr = blockIdx.y;
-    const srwd_trj_info I = info[tr];
-    if (i >= I.np) return;
-    double s = I.sStart + (double)i * I.sStep;
-    trj_pt px = eval_plane(I, X + tr * ldT, IBx + tr * ldT, -1. / I.betaNorm, s, true);
-    trj_pt pz = eval_plane(I, Y + tr * ldT, IBz + tr * ldT, 1. / I.betaNorm, s, true);
-    double* o = samp + tr * ldS * 4;
-    o[i] = px.bt; o[ldS + i] = pz.bt; o[2 * ldS + i] = px.crd; o[3 * ldS + i] = pz.crd;
-}
-
 // srradstr.cpp:2310-2501 (FindAverageDistanceToSource) with the full
 // trajectory range.  mesh[4*tr] = xStart, xEnd, zStart, zEnd; out[4*tr] =
 // Robs, RobsAbsErr, xc, zc.  One block per trajectory: each of the four
@@ -2006,7 +2025,8 @@ __global__ void __launch_bounds__(256) k_rx_samples(const srwd_trj_info* __restr
 // sample.  Each thread visits its samples in increasing order and keeps its
 // first hit per criterion; the block minimum follows from a wave reduction
 // and one LDS exchange.
-__global__ void __launch_bounds__(256) k_find_rx(const srwd_trj_info* __restrict__ info, const double* samp,
+#define SRWD_RX_THREADS 1024
+__global__ void __launch_bounds__(SRWD_RX_THREADS) k_find_rx(const srwd_trj_info* __restrict__ info, const double* samp,
                                                  long long ldS, const double* mesh, double* out)
 {
     const int tr = blockIdx.x;
@@ -2018,7 +2038,7 @@ __global__ void __launch_bounds__(256) k_find_rx(const srwd_trj_info* __restrict
     const double sStart = I.sStart, sRange = (N - 1) * I.sStep, sEnd = sStart + sRange;
     const long long L = N - 1;
     const unsigned long long NONE = ~0ull;
-    __shared__ unsigned long long first[4][8];
+    __shared__ unsigned long long first[SRWD_RX_THREADS / 64][8];
     const double R0b = I.yObs - sEnd, R0f = I.yObs - sStart;
     double crd[4] = {xS, xE, zS, zE};
     double ref[8];
@@ -2052,7 +2072,7 @@ __global__ void __launch_bounds__(256) k_find_rx(const srwd_trj_info* __restrict
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int k = 0; k < 8; k++)
-            for (int q = 1; q < 4; q++) first[0][k] = first[q][k] < first[0][k] ? first[q][k] : first[0][k];
+            for (int q = 1; q < SRWD_RX_THREADS / 64; q++) first[0][k] = first[q][k] < first[0][k] ? first[q][k] : first[0][k];
     }
     if (threadIdx.x != 0) return;
     const double VL = 1.E+23;
@@ -2081,20 +2101,10 @@ __global__ void __launch_bounds__(256) k_find_rx(const srwd_trj_info* __restrict
 }
 
 extern "C" {
-int srwd_launch_nz(srwd_trj_info* dInfo, int nTraj, const double* dX, const double* dXp, const double* dY,
-                   const double* dYp, long long ldT, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_nz_flags, dim3(nTraj), dim3(256), 0, st, dInfo, dX, dXp, dY, dYp, ldT);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
-int srwd_launch_rx(const srwd_trj_info* dInfo, int nTraj, long long maxNp, const double* dX, const double* dY,
-                   const double* dIBx, const double* dIBz, long long ldT, double* dSamp, const double* dMesh,
+int srwd_launch_rx(const srwd_trj_info* dInfo, int nTraj, const double* dSamp, long long ldT, const double* dMesh,
                    double* dRx, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_rx_samples, dim3((unsigned)((maxNp + 255) / 256), nTraj), dim3(256), 0, st, dInfo, dX,
-                       dY, dIBx, dIBz, ldT, dSamp, ldT);
-    hipLaunchKernelGGL(k_find_rx, dim3(nTraj), dim3(256), 0, st, dInfo, dSamp, ldT, dMesh, dRx);
+    hipLaunchKernelGGL(k_find_rx, dim3(nTraj), dim3(SRWD_RX_THREADS), 0, st, dInfo, dSamp, ldT, dMesh, dRx);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 }

@@ -42,14 +42,14 @@ struct Arena {
 extern Arena* g_arena;   // non-null while a no-allocation call runs
 
 struct Buffers {
-    DBuf X, Xp, Y, Yp, IBx, IBz, Samp, Jobs, Fields, Info;
-    DBuf Rec, Chunk, Q, Edge, Mesh, Rx, Items, BlockItem, RowTraj, RowE, RowN, A, Part, Warn;
-    DBuf Cond, FpList, FpCount;   // condition check of the FP32 sums and its FP64 recomputation list
+    DBuf X, Xp, Y, Yp, IBx, IBz, Samp;
+    DBuf UpTrj, UpSr;             // setup data of an SR call: trajectories; requests, items and launch lists
+    DBuf Rec, Chunk, Q, Edge, A, Part;
+    DBuf Cond, FpList;            // condition check of the FP32 sums and its FP64 recomputation list
     DBuf Mrec;                    // integration-point records of the mesh kernel
     DBuf T64;                     // FP64 trajectory values per integration point (FP64 recomputation)
-    DBuf Req, Coord, BlkReq, Last;   // requests, observation coordinates, edge-derivative state
-    DBuf SrBlocks;                // SR launch lists {item, block}
-    DBuf TileBands, Patch, PatchCount;   // streamed rows: row bands per tile block, FP64 store records
+    DBuf Last;                    // edge-derivative state
+    DBuf Patch;                   // streamed rows: FP64 store records
     DBuf Ex, Ez;                  // field outputs
     DBuf W0, W1, W2, W3;          // propagation / accumulation work buffers
     DBuf Stokes, Draws, Wt, Net, Grad, Rep;
@@ -78,7 +78,7 @@ struct Context {
     size_t blockDoneCap = 0;
     unsigned streamEpoch = 0;
     hipEvent_t evTiles = nullptr;  // the streamed-rows tile kernel has finished
-    char* patchHost = nullptr;    // pinned: FP64 store count, then the store records
+    char* patchHost = nullptr;    // pinned: FP64 store records
     bool lastStreamFallback = false;
     bool lastStreamed = false;    // the last single-request call streamed rows without falling back
     bool trajSerial = false;      // test switch: serial RK4 kernel instead of the parallel one
@@ -94,7 +94,6 @@ struct Context {
     int nFftCalls = 0;
     double lastRsMs = 0, lastRsBytes = 0;   // last resampling of a propagation
     double lastPropDevMs = 0;               // device part of the last propagation (after upload, before download)
-    int* warnHost = nullptr;                // pinned: termination warning of the last SR pass
     // Streamed download of field results: a second stream copies finished
     // row bands into pinned staging while the next band is computed; the
     // calling thread moves them on into the caller's arrays.
@@ -109,7 +108,9 @@ struct Context {
     size_t momPinBytes = 0;
     std::vector<hipEvent_t> bandEv;         // per band: computed, downloaded, SR start, SR end
     int nTimePairs = 0;                     // timed SR launches of the last pass (bandEv[4b+2], [4b+3])
-    int* fpCountHost = nullptr;             // pinned: points recomputed in FP64, per band (at most 64 bands)
+    int* fpCountHost = nullptr;             // pinned: warning, FP64 stores, points recomputed in FP64 per band (at most 62)
+    char* geo = nullptr;                    // pinned: trajectory infos and radius results of an SR call
+    size_t geoBytes = 0;
     int fpBands = 0;
     long long lastFp64Points = 0;           // points of the last SR pass recomputed in FP64
     double condTol = 1e-4;                  // condition check of the FP32 sums (0: off)
@@ -169,7 +170,9 @@ struct HostOut {
 int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, float* dEx, float* dEz,
            const std::vector<long long>& outOff, std::vector<SrResult>& res, int termin,
            bool defer = false, bool geomOnly = false, const HostOut* hostOut = nullptr);
-// Pinned staging of at least `bytes` (grow-only); nullptr on failure.
+// Grow-only pinned buffer p of `have` bytes made at least `bytes` large, and
+// the staging of downloads; nullptr on failure.
+char* grow_pinned(char*& p, size_t& have, size_t bytes);
 char* pinned_staging(size_t bytes);
 // Copies device memory to host memory through the pinned staging on the copy
 // stream, in pieces, after the work already queued on the compute stream.

@@ -168,15 +168,16 @@ inline long long srwd_traj_scratch(long long ld) { return 20 * srwd_pic_cap(ld) 
 int srwd_launch_traj(const srwd_traj_job* dJobs, const srwd_field* dFields, int nTraj, double* dX,
                      double* dXp, double* dY, double* dYp, double* dZ, long long ld, double* dScratch,
                      int singleHarmonic, hipStream_t st);
-int srwd_launch_nz(srwd_trj_info* dInfo, int nTraj, const double* dX, const double* dXp, const double* dY,
-                   const double* dYp, long long ldT, hipStream_t st);
-int srwd_launch_tables(const srwd_trj_info* dInfo, int nTraj, long long maxInt, const double* dX,
+// From the trajectories (leading dimension ldT): the zero-field flags of
+// dInfo (zero before), the integrals of the squared angles, the integration-
+// point tables, the edge data and the samples of the radius search (dSamp, 4
+// ldT doubles per trajectory).
+int srwd_launch_tables(srwd_trj_info* dInfo, int nTraj, const double* dX,
                        const double* dXp, const double* dY, const double* dYp, long long ldT,
                        double* dIBx, double* dIBz, srwd_rec* dRec, srwd_chunk* dChunk, double* dQ,
                        long long ldI, long long ldC, srwd_edge* dEdge, double* dT64, srwd_mrec* dMrec, long long ldM,
-                       hipStream_t st);
-int srwd_launch_rx(const srwd_trj_info* dInfo, int nTraj, long long maxNp, const double* dX, const double* dY,
-                   const double* dIBx, const double* dIBz, long long ldT, double* dSamp, const double* dMesh,
+                       double* dSamp, hipStream_t st);
+int srwd_launch_rx(const srwd_trj_info* dInfo, int nTraj, const double* dSamp, long long ldT, const double* dMesh,
                    double* dRx, hipStream_t st);
 int srwd_launch_phase_table(const double* dQ, long long ldI, const int* dRowTraj, const double* dRowE,
                             const long long* dRowN, int nRows, long long maxInt, float* dA, hipStream_t st);

@@ -48,10 +48,9 @@ int ensure_device()
     if (hipEventCreateWithFlags(&g_ctx.evFork, hipEventDisableTiming) != hipSuccess) return SRWL_AMD_ERR_GPU;
     if (hipEventCreateWithFlags(&g_ctx.evJoin, hipEventDisableTiming) != hipSuccess) return SRWL_AMD_ERR_GPU;
     if (hipEventCreateWithFlags(&g_ctx.evTiles, hipEventDisableTiming) != hipSuccess) return SRWL_AMD_ERR_GPU;
-    if (hipHostMalloc((void**)&g_ctx.warnHost, sizeof(int), hipHostMallocDefault) != hipSuccess) return SRWL_AMD_ERR_GPU;
     if (hipHostMalloc((void**)&g_ctx.fpCountHost, sizeof(int) * 64, hipHostMallocDefault) != hipSuccess)
         return SRWL_AMD_ERR_GPU;
-    *g_ctx.warnHost = 0;
+    g_ctx.fpCountHost[0] = 0;
     g_ctx.device = dev;
     g_ctx.ready = true;
     return 0;
@@ -205,6 +204,25 @@ static int h2d(void* dst, const void* src, size_t bytes, hipStream_t st)
     return hipMemcpyAsync(dst, g_ctx.up + at, bytes, hipMemcpyHostToDevice, st) == hipSuccess ? 0 : SRWL_AMD_ERR_GPU;
 }
 
+// Setup data that one copy takes to the device: pieces at 256-byte offsets.
+struct UpBlob {
+    std::vector<char> h;
+    size_t add(const void* src, size_t bytes)
+    {
+        const size_t at = (h.size() + 255) & ~(size_t)255;
+        h.resize(at + bytes);
+        if (bytes) std::memcpy(h.data() + at, src, bytes);
+        return at;
+    }
+    template <typename T> size_t add(const std::vector<T>& v) { return add(v.data(), sizeof(T) * v.size()); }
+    size_t zeros(size_t bytes)
+    {
+        const size_t at = add(nullptr, 0);
+        h.resize(at + bytes, 0);
+        return at;
+    }
+};
+
 // Tiles of the mesh kernel over nx x nz computed points.
 static int mesh_tiles(int nx, int nz)
 {
@@ -310,15 +328,25 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     double* dY = (double*)B.Y.get(trjBytes); double* dYp = (double*)B.Yp.get(trjBytes);
     double* dIBx = (double*)B.IBx.get(trjBytes); double* dIBz = (double*)B.IBz.get(trjBytes);
     double* dSamp = (double*)B.Samp.get(4 * trjBytes);
-    srwd_traj_job* dJobs = (srwd_traj_job*)B.Jobs.get(sizeof(srwd_traj_job) * nT);
-    srwd_field* dFields = (srwd_field*)B.Fields.get(sizeof(srwd_field) * std::max<size_t>(fields.size(), 1));
-    srwd_trj_info* dInfo = (srwd_trj_info*)B.Info.get(sizeof(srwd_trj_info) * nT);
-    if (!dX || !dXp || !dY || !dYp || !dIBx || !dIBz || !dSamp || !dJobs || !dFields || !dInfo)
-        return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
-    if (int e_ = h2d(dJobs, tj.data(), sizeof(srwd_traj_job) * nT, st)) return e_;
-    if (!fields.empty())
-        if (int e_ = h2d(dFields, fields.data(), sizeof(srwd_field) * fields.size(), st)) return e_;
-    if (int e_ = h2d(dInfo, info.data(), sizeof(srwd_trj_info) * nT, st)) return e_;
+    std::vector<double> meshLim(4 * nT);
+    for (int j = 0; j < nT; j++) {
+        const SRWLRadMesh& m = jobs[j].mesh;
+        double xStep = m.nx > 1 ? (m.xFin - m.xStart) / (m.nx - 1) : 0;
+        double zStep = m.ny > 1 ? (m.yFin - m.yStart) / (m.ny - 1) : 0;
+        meshLim[4 * j] = m.xStart; meshLim[4 * j + 1] = m.xStart + (m.nx - 1) * xStep;
+        meshLim[4 * j + 2] = m.yStart; meshLim[4 * j + 3] = m.yStart + (m.ny - 1) * zStep;
+    }
+    UpBlob up;
+    const size_t oJobs = up.add(tj), oFields = up.add(fields), oMesh = up.add(meshLim), oInfo = up.add(info);
+    const size_t oRx = up.zeros(sizeof(double) * 4 * nT);   // results, read back together with the infos
+    char* dUp = (char*)B.UpTrj.get(up.h.size());
+    if (!dX || !dXp || !dY || !dYp || !dIBx || !dIBz || !dSamp || !dUp) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+    srwd_traj_job* dJobs = (srwd_traj_job*)(dUp + oJobs);
+    srwd_field* dFields = (srwd_field*)(dUp + oFields);
+    double* dMesh = (double*)(dUp + oMesh);
+    srwd_trj_info* dInfo = (srwd_trj_info*)(dUp + oInfo);
+    double* dRx = (double*)(dUp + oRx);
+    if (int e_ = h2d(dUp, up.h.data(), up.h.size(), st)) return e_;
     bool anyRK = false;
     for (int j = 0; j < nT; j++) {
         if (jobs[j].userTrj) {
@@ -350,7 +378,6 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             if (int e_ = h2d(dYp + j * ldT, u->arYp, b, st)) return e_;
         }
     }
-    if (srwd_launch_nz(dInfo, nT, dX, dXp, dY, dYp, ldT, st)) return SRWL_AMD_ERR_GPU;
     // --- tables ------------------------------------------------------------
     long long maxInt = 0;
     for (auto& I : info) maxInt = std::max(maxInt, I.nInt);
@@ -360,30 +387,28 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     srwd_chunk* dChunk = (srwd_chunk*)B.Chunk.get(sizeof(srwd_chunk) * (size_t)ldC * nT);
     double* dQ = (double*)B.Q.get(sizeof(double) * (size_t)ldI * nT);
     srwd_edge* dEdge = (srwd_edge*)B.Edge.get(sizeof(srwd_edge) * nT);
-    double* dMesh = (double*)B.Mesh.get(sizeof(double) * 4 * nT);
-    double* dRx = (double*)B.Rx.get(sizeof(double) * 4 * nT);
     double* dT64 = g_ctx.condTol > 0 ? (double*)B.T64.get(sizeof(double) * SRWD_T64 * (size_t)ldI * nT) : nullptr;
     const long long ldM = srwd_mesh_ld(maxInt);
     srwd_mrec* dMrec = (srwd_mrec*)B.Mrec.get(sizeof(srwd_mrec) * 2 * (size_t)ldM * nT);
-    if (!dRec || !dChunk || !dQ || !dEdge || !dMesh || !dRx || !dMrec || (g_ctx.condTol > 0 && !dT64))
+    double* dCond = (double*)B.Cond.get(sizeof(double) * 7 * nT);
+    if (!dRec || !dChunk || !dQ || !dEdge || !dMrec || !dCond || (g_ctx.condTol > 0 && !dT64))
         return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
-    if (srwd_launch_tables(dInfo, nT, maxInt, dX, dXp, dY, dYp, ldT, dIBx, dIBz, dRec, dChunk, dQ, ldI, ldC,
-                           dEdge, dT64, dMrec, ldM, st))
+    if (srwd_launch_tables(dInfo, nT, dX, dXp, dY, dYp, ldT, dIBx, dIBz, dRec, dChunk, dQ, ldI, ldC,
+                           dEdge, dT64, dMrec, ldM, dSamp, st))
         return SRWL_AMD_ERR_GPU;
-    std::vector<double> meshLim(4 * nT);
-    for (int j = 0; j < nT; j++) {
-        const SRWLRadMesh& m = jobs[j].mesh;
-        double xStep = m.nx > 1 ? (m.xFin - m.xStart) / (m.nx - 1) : 0;
-        double zStep = m.ny > 1 ? (m.yFin - m.yStart) / (m.ny - 1) : 0;
-        meshLim[4 * j] = m.xStart; meshLim[4 * j + 1] = m.xStart + (m.nx - 1) * xStep;
-        meshLim[4 * j + 2] = m.yStart; meshLim[4 * j + 3] = m.yStart + (m.ny - 1) * zStep;
-    }
-    if (int e_ = h2d(dMesh, meshLim.data(), sizeof(double) * 4 * nT, st)) return e_;
-    if (srwd_launch_rx(dInfo, nT, ldT, dX, dY, dIBx, dIBz, ldT, dSamp, dMesh, dRx, st)) return SRWL_AMD_ERR_GPU;
-    std::vector<double> rx(4 * nT);
-    HIPCHK(hipMemcpyAsync(rx.data(), dRx, sizeof(double) * 4 * nT, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(info.data(), dInfo, sizeof(srwd_trj_info) * nT, hipMemcpyDeviceToHost, st));
+    double* dScale = dCond + 5 * nT;   // inverse amplitude scales of the mesh records, 2 per trajectory
+    if (srwd_launch_cond_sums(dInfo, nT, dRec, ldI, dCond, dMrec, ldM, dMesh, dScale, st)) return SRWL_AMD_ERR_GPU;
+    if (srwd_launch_rx(dInfo, nT, dSamp, ldT, dMesh, dRx, st)) return SRWL_AMD_ERR_GPU;
+    // infos (zero-field flags) and radii in one copy, into pinned memory
+    // (a no-allocation call has none: pageable memory)
+    const size_t geoBytes = up.h.size() - oInfo;
+    char* geo = g_arena ? nullptr : grow_pinned(g_ctx.geo, g_ctx.geoBytes, geoBytes);
+    if (!g_arena && !geo) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+    if (!geo) geo = up.h.data() + oInfo;
+    HIPCHK(hipMemcpyAsync(geo, dInfo, geoBytes, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
+    std::memcpy(info.data(), geo, sizeof(srwd_trj_info) * nT);
+    const double* rx = (const double*)(geo + (oRx - oInfo));
     for (int j = 0; j < nT; j++) {
         res[j].Robs = rx[4 * j]; res[j].RobsErr = rx[4 * j + 1];
         res[j].xc = rx[4 * j + 2]; res[j].zc = rx[4 * j + 3];
@@ -418,22 +443,30 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             blkReq.insert(blkReq.end(), (size_t)nb, j);
         }
     }
-    srwd_req* dReq = (srwd_req*)B.Req.get(sizeof(srwd_req) * nT);
-    double* dCoord = (double*)B.Coord.get(sizeof(double) * std::max<size_t>(1, coord.size()));
     long long nEdgeBlk = (long long)blkReq.size();
-    int* dBlkReq = nEdgeBlk ? (int*)B.BlkReq.get(sizeof(int) * (size_t)nEdgeBlk) : nullptr;
     long long* dLast = nEdgeBlk ? (long long*)B.Last.get(sizeof(long long) * 2 * (size_t)nEdgeBlk) : nullptr;
-    if (!dReq || !dCoord || (nEdgeBlk && (!dBlkReq || !dLast))) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
-    if (int e_ = h2d(dReq, reqs.data(), sizeof(srwd_req) * nT, st)) return e_;
-    if (!coord.empty())
-        if (int e_ = h2d(dCoord, coord.data(), sizeof(double) * coord.size(), st)) return e_;
-    if (nEdgeBlk) {
-        if (int e_ = h2d(dBlkReq, blkReq.data(), sizeof(int) * (size_t)nEdgeBlk, st)) return e_;
-        if (srwd_launch_edge_state(dReq, nT, dBlkReq, nEdgeBlk, dInfo, dEdge, dCoord, termin, dLast, st))
+    if (nEdgeBlk && !dLast) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+    UpBlob us;
+    const size_t oReq = us.add(reqs), oCoord = us.add(coord), oBlkReq = us.add(blkReq);
+    srwd_req* dReq = nullptr;
+    double* dCoord = nullptr;
+    char* dUs = nullptr;
+    // uploads the setup data gathered so far and queues the edge-derivative state
+    auto upload_requests = [&]() -> int {
+        dUs = (char*)B.UpSr.get(us.h.size());
+        if (!dUs) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+        dReq = (srwd_req*)(dUs + oReq);
+        dCoord = (double*)(dUs + oCoord);
+        if (int e_ = h2d(dUs, us.h.data(), us.h.size(), st)) return e_;
+        if (nEdgeBlk && srwd_launch_edge_state(dReq, nT, (const int*)(dUs + oBlkReq), nEdgeBlk, dInfo, dEdge, dCoord,
+                                               termin, dLast, st))
             return SRWL_AMD_ERR_GPU;
-    }
+        return 0;
+    };
     if (jobs[0].meth == 1) {
         for (auto& J : jobs) if (J.meth != 1) return SRWL_AMD_ERR_BATCH;
+        rc = upload_requests();
+        if (rc) return rc;
         if (g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev0, st));
         rc = sr_auto_run(jobs, info, dInfo, dX, dY, dIBx, dIBz, ldT, dEdge, termin, dEx, dEz, outOff, res, dReq, dCoord,
                          dLast);
@@ -449,7 +482,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         long long ev = 0;
         for (int L : g_ctx.autoLevels) ev += 4LL * (1LL << L) + 1;
         g_ctx.pendingEvals = ev;
-        *g_ctx.warnHost = 0;
+        g_ctx.fpCountHost[0] = 0;
         if (defer) return 0;
         HIPCHK(hipStreamSynchronize(st));
         sr_complete(res);
@@ -660,45 +693,36 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         nSplit = (int)std::min<long long>(std::max<long long>(1, (wgTarget + bandWG - 1) / bandWG), minChunks);
     }
     if (g_ctx.forceSplit > 0) nSplit = (int)std::min<long long>(g_ctx.forceSplit, minChunks);
-    srwd_item* dItems = (srwd_item*)B.Items.get(sizeof(srwd_item) * nItems);
-    int* dBlockItem = (int*)B.BlockItem.get(sizeof(int) * nBlocks);
     std::vector<int2> srLists;   // finalize lists, then the lists of the sums
     for (auto* l : {&tileBlocks, &restBlocks, &srTileBlocks, &srRestBlocks, &meshTiles})
         srLists.insert(srLists.end(), l->begin(), l->end());
-    int2* dSrBlocks = (int2*)B.SrBlocks.get(sizeof(int2) * srLists.size());
-    int* dRowTraj = (int*)B.RowTraj.get(sizeof(int) * nRows);
-    double* dRowE = (double*)B.RowE.get(sizeof(double) * nRows);
-    long long* dRowN = (long long*)B.RowN.get(sizeof(long long) * nRows);
+    const size_t oItems = us.add(items), oBlockItem = us.add(blockItem), oLists = us.add(srLists);
+    const size_t oRowTraj = us.add(rowTraj), oRowE = us.add(rowE), oRowN = us.add(rowN);
+    // warning, FP64 stores recorded for the host, FP64 points per band: zero, read back in one copy
+    const size_t oCounts = us.zeros(sizeof(int) * (2 + (size_t)nBands));
     float* dA = (float*)B.A.get(sizeof(float) * (size_t)ldI * nRows);
     double* dPart = (double*)B.Part.get(sizeof(double) * 4 * (size_t)nSplit * nPointsPad);
-    int* dWarn = (int*)B.Warn.get(sizeof(int));
     // condition check of the FP32 sums and the FP64 recomputation list (one band at a time)
     int maxBandBlocks = 0;
     for (int b = 0; b < nBands; b++) maxBandBlocks = std::max(maxBandBlocks, bandBlock0[b + 1] - bandBlock0[b]);
-    double* dCond = (double*)B.Cond.get(sizeof(double) * 7 * nT);
-    double* dScale = dCond + 5 * nT;   // inverse amplitude scales of the mesh records, 2 per trajectory
     // one list per compute stream: consecutive bands run on alternate streams
     const int nLists = nBands > 1 ? 2 : 1;
     int* dFpList = (int*)B.FpList.get(sizeof(int) * 256 * (size_t)maxBandBlocks * nLists);
-    int* dFpCount = (int*)B.FpCount.get(sizeof(int) * (size_t)nBands);
-    if (!dItems || !dBlockItem || !dSrBlocks || !dRowTraj || !dRowE || !dRowN || !dA || !dPart || !dWarn || !dCond || !dFpList ||
-        !dFpCount)
-        return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
-    if (int e_ = h2d(dItems, items.data(), sizeof(srwd_item) * nItems, st)) return e_;
-    if (int e_ = h2d(dBlockItem, blockItem.data(), sizeof(int) * nBlocks, st)) return e_;
-    int2* dTileBlocks = dSrBlocks;
+    if (!dA || !dPart || !dFpList) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+    rc = upload_requests();
+    if (rc) return rc;
+    srwd_item* dItems = (srwd_item*)(dUs + oItems);
+    int* dBlockItem = (int*)(dUs + oBlockItem);
+    int* dWarn = (int*)(dUs + oCounts);
+    int* dPatchCount = dWarn + 1;
+    int* dFpCount = dWarn + 2;
+    int2* dTileBlocks = (int2*)(dUs + oLists);
     int2* dRestBlocks = dTileBlocks + tileBlocks.size();
     int2* dSrTile = dRestBlocks + restBlocks.size();
     int2* dSrRest = dSrTile + srTileBlocks.size();
     int2* dMeshTiles = dSrRest + srRestBlocks.size();
-    if (int e_ = h2d(dSrBlocks, srLists.data(), sizeof(int2) * srLists.size(), st)) return e_;
-    if (int e_ = h2d(dRowTraj, rowTraj.data(), sizeof(int) * nRows, st)) return e_;
-    if (int e_ = h2d(dRowE, rowE.data(), sizeof(double) * nRows, st)) return e_;
-    if (int e_ = h2d(dRowN, rowN.data(), sizeof(long long) * nRows, st)) return e_;
-    HIPCHK(hipMemsetAsync(dWarn, 0, sizeof(int), st));
-    if (nRows > 0 && srwd_launch_phase_table(dQ, ldI, dRowTraj, dRowE, dRowN, nRows, maxInt, dA, st)) return SRWL_AMD_ERR_GPU;
-    if (srwd_launch_cond_sums(dInfo, nT, dRec, ldI, dCond, dMrec, ldM, dMesh, dScale, st)) return SRWL_AMD_ERR_GPU;
-    HIPCHK(hipMemsetAsync(dFpCount, 0, sizeof(int) * (size_t)nBands, st));
+    if (nRows > 0 && srwd_launch_phase_table(dQ, ldI, (const int*)(dUs + oRowTraj), (const double*)(dUs + oRowE),
+                                             (const long long*)(dUs + oRowN), nRows, maxInt, dA, st)) return SRWL_AMD_ERR_GPU;
     g_ctx.lastSrBlocks = nBlocks;
     g_ctx.lastSrSplit = nSplit;
     // events of a banded pass: per band a timing pair around the SR launch,
@@ -763,15 +787,13 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         // flags of this call carry its own epoch (never 0), so they need no clearing
         const unsigned epoch = ++g_ctx.streamEpoch ? g_ctx.streamEpoch : ++g_ctx.streamEpoch;
         if (!g_ctx.patchHost &&
-            hipHostMalloc((void**)&g_ctx.patchHost, sizeof(srwd_patch) * SRWL_AMD_PATCH_CAP + 256,
+            hipHostMalloc((void**)&g_ctx.patchHost, sizeof(srwd_patch) * SRWL_AMD_PATCH_CAP,
                           hipHostMallocDefault) != hipSuccess) {
             g_ctx.patchHost = nullptr;
             return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
         }
         srwd_patch* dPatch = (srwd_patch*)B.Patch.get(sizeof(srwd_patch) * SRWL_AMD_PATCH_CAP);
-        int* dPatchCount = (int*)B.PatchCount.get(sizeof(int));
-        if (!dPatch || !dPatchCount) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
-        HIPCHK(hipMemsetAsync(dPatchCount, 0, sizeof(int), st));
+        if (!dPatch) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
         volatile unsigned* done = g_ctx.blockDone;
         while (g_ctx.bandEv.size() < 4 * (size_t)nDl) {
             hipEvent_t e;
@@ -842,9 +864,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             srwd_launch_sr_fp64(dItems, dBlockItem, dInfo, dEdge, termin, dT64, ldI, dEx, dEz, dWarn, dFpList,
                                 dFpCount, dReq, dCoord, dLast, dPart, dPatch, dPatchCount, SRWL_AMD_PATCH_CAP, st))
             return SRWL_AMD_ERR_GPU;
-        HIPCHK(hipMemcpyAsync(g_ctx.warnHost, dWarn, sizeof(int), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(g_ctx.fpCountHost, dFpCount, sizeof(int), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(g_ctx.patchHost, dPatchCount, sizeof(int), hipMemcpyDeviceToHost, st));
+        HIPCHK(hipMemcpyAsync(g_ctx.fpCountHost, dWarn, sizeof(int) * 3, hipMemcpyDeviceToHost, st));
         g_ctx.fpBands = 1;
         long long evs = 0;
         for (auto& it : items) evs += (long long)it.npts * info[it.traj].nInt;
@@ -895,7 +915,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         }
         (void)hipGetLastError();   // the queries' "not ready"
         HIPCHK(hipStreamSynchronize(st));
-        const int nPatch = *(volatile int*)g_ctx.patchHost;
+        const int nPatch = ((volatile int*)g_ctx.fpCountHost)[1];
         g_ctx.lastStreamFallback = late || nPatch > SRWL_AMD_PATCH_CAP;
         g_ctx.lastStreamed = !g_ctx.lastStreamFallback;
         if (g_ctx.lastStreamFallback) {
@@ -907,7 +927,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             if (rc) return rc;
         } else {
             // the FP64-recomputed values over what the bands carried
-            srwd_patch* P = (srwd_patch*)(g_ctx.patchHost + 256);
+            srwd_patch* P = (srwd_patch*)g_ctx.patchHost;
             if (nPatch > 0)
                 HIPCHK(hipMemcpy(P, dPatch, sizeof(srwd_patch) * (size_t)nPatch, hipMemcpyDeviceToHost));
             float2* hx = (float2*)hostOut->ex;
@@ -989,8 +1009,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         HIPCHK(hipStreamWaitEvent(st, g_ctx.evJoin, 0));
     }
     // the warning flag and the FP64 point counts are read back with the caller's final synchronisation
-    HIPCHK(hipMemcpyAsync(g_ctx.warnHost, dWarn, sizeof(int), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(g_ctx.fpCountHost, dFpCount, sizeof(int) * (size_t)nBands, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(g_ctx.fpCountHost, dWarn, sizeof(int) * (2 + (size_t)nBands), hipMemcpyDeviceToHost, st));
     g_ctx.fpBands = nBands;
     long long ev = 0;
     for (auto& it : items) ev += (long long)it.npts * info[it.traj].nInt;
@@ -1025,20 +1044,22 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     return 0;
 }
 
-char* pinned_staging(size_t bytes)
+char* grow_pinned(char*& p, size_t& have, size_t bytes)
 {
-    if (bytes > g_ctx.pinBytes) {
-        if (g_ctx.pin) (void)hipHostFree(g_ctx.pin);
-        g_ctx.pin = nullptr;
-        g_ctx.pinBytes = 0;
-        if (hipHostMalloc((void**)&g_ctx.pin, bytes, hipHostMallocDefault) != hipSuccess) {
-            g_ctx.pin = nullptr;
+    if (bytes > have) {
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        have = 0;
+        if (hipHostMalloc((void**)&p, bytes, hipHostMallocDefault) != hipSuccess) {
+            p = nullptr;
             return nullptr;
         }
-        g_ctx.pinBytes = bytes;
+        have = bytes;
     }
-    return g_ctx.pin;
+    return p;
 }
+
+char* pinned_staging(size_t bytes) { return grow_pinned(g_ctx.pin, g_ctx.pinBytes, bytes); }
 
 namespace {
 // A copy whose stores bypass the caches (16-byte streaming stores once the
@@ -1252,10 +1273,10 @@ void sr_complete(std::vector<SrResult>& res)
         g_ctx.sumSrEvals += (double)g_ctx.pendingEvals;
         g_ctx.nSrCalls += 1;
     }
-    if (*g_ctx.warnHost)
+    if (g_ctx.fpCountHost[0])
         for (auto& r : res) if (!r.warn) r.warn = SRWL_WARN_BAD_RAD_INT_TERMINATIONS;
     long long fp = 0;
-    for (int b = 0; b < g_ctx.fpBands; b++) fp += g_ctx.fpCountHost[b];
+    for (int b = 0; b < g_ctx.fpBands; b++) fp += g_ctx.fpCountHost[2 + b];
     g_ctx.lastFp64Points = fp;
     g_ctx.fpBands = 0;
 }
@@ -1396,27 +1417,38 @@ SRWL_EXPORT int srwlCalcPartTraj(SRWLPrtTrj* pTrj, SRWLMagFldC* pMagFld, double*
     J.ctStart = pTrj->ctStart; J.ctEnd = pTrj->ctEnd; J.np = pTrj->np; J.field = 0;
     hipStream_t st = g_ctx.stream;
     Buffers& B = g_ctx.buf;
-    size_t b = sizeof(double) * pTrj->np;
-    double* dX = (double*)B.X.get(b); double* dXp = (double*)B.Xp.get(b);
-    double* dY = (double*)B.Y.get(b); double* dYp = (double*)B.Yp.get(b); double* dZ = (double*)B.IBx.get(b);
-    srwd_traj_job* dJ = (srwd_traj_job*)B.Jobs.get(sizeof(J));
-    srwd_field* dF = (srwd_field*)B.Fields.get(sizeof(f));
-    if (!dX || !dXp || !dY || !dYp || !dZ || !dJ || !dF) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
-    HIPCHK(hipMemcpyAsync(dJ, &J, sizeof(J), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dF, &f, sizeof(f), hipMemcpyHostToDevice, st));
+    const size_t b = sizeof(double) * pTrj->np;
+    // the five components side by side, read back in one copy through the
+    // pinned staging
+    double* dX = (double*)B.X.get(5 * b);
+    if (!dX) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+    double *dXp = dX + pTrj->np, *dY = dXp + pTrj->np, *dYp = dY + pTrj->np, *dZ = dYp + pTrj->np;
+    UpBlob up;
+    const size_t oJob = up.add(&J, sizeof(J)), oField = up.add(&f, sizeof(f));
+    char* dUp = (char*)B.UpTrj.get(up.h.size());
+    char* pin = pinned_staging(5 * b);
+    if (!dUp || !pin) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+    if (g_ctx.upUsed) {   // the upload staging is reused once its copies are done
+        HIPCHK(hipStreamSynchronize(st));
+        g_ctx.upUsed = 0;
+    }
+    if (int e_ = h2d(dUp, up.h.data(), up.h.size(), st)) return e_;
     double* dPic = nullptr;
     if (!g_ctx.trajSerial) {
         dPic = (double*)B.Pic.get(sizeof(double) * (size_t)srwd_traj_scratch(pTrj->np));
         if (!dPic) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
     }
     int one = (f.n == 1 && f.u[0].nh == 1);
-    if (srwd_launch_traj(dJ, dF, 1, dX, dXp, dY, dYp, dZ, pTrj->np, dPic, one, st)) return SRWL_AMD_ERR_GPU;
-    HIPCHK(hipMemcpyAsync(pTrj->arX, dX, b, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(pTrj->arXp, dXp, b, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(pTrj->arY, dY, b, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(pTrj->arYp, dYp, b, hipMemcpyDeviceToHost, st));
-    if (pTrj->arZ) HIPCHK(hipMemcpyAsync(pTrj->arZ, dZ, b, hipMemcpyDeviceToHost, st));
+    if (srwd_launch_traj((srwd_traj_job*)(dUp + oJob), (srwd_field*)(dUp + oField), 1, dX, dXp, dY, dYp, dZ, pTrj->np,
+                         dPic, one, st))
+        return SRWL_AMD_ERR_GPU;
+    HIPCHK(hipMemcpyAsync(pin, dX, 5 * b, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
+    std::memcpy(pTrj->arX, pin, b);
+    std::memcpy(pTrj->arXp, pin + b, b);
+    std::memcpy(pTrj->arY, pin + 2 * b, b);
+    std::memcpy(pTrj->arYp, pin + 3 * b, b);
+    if (pTrj->arZ) std::memcpy(pTrj->arZ, pin + 4 * b, b);
     if (pTrj->arZp) {
         // srgtrjdt.cpp:150: longitudinal relative velocity from the transverse ones
         double gEm2 = 1. / g / g;
