@@ -58,6 +58,24 @@ int device_moments(const std::vector<srwm_mslice>& sl, std::vector<double>& sums
     return 0;
 }
 
+int device_moments_queue(const std::vector<srwm_mslice>& slices, bool lanesOverSlices, MomQueued& q)
+{
+    const int n = (int)slices.size();
+    // pinned: slice table, then 24 sums per slice
+    const size_t slBytes = ((sizeof(srwm_mslice) * n + 255) / 256) * 256;
+    if (!grow_pinned(g_ctx.momPin, g_ctx.momPinBytes, slBytes + sizeof(double) * 24 * n))
+        return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+    srwm_mslice* sl = (srwm_mslice*)g_ctx.momPin;
+    q.sums = (double*)(g_ctx.momPin + slBytes);
+    int nxMax = 1, nzMax = 1;
+    for (int k = 0; k < n; k++) {
+        sl[k] = slices[k];
+        nxMax = std::max(nxMax, sl[k].nx);
+        nzMax = std::max(nzMax, sl[k].nz);
+    }
+    return queue_sums(sl, n, nxMax, nzMax, lanesOverSlices, q.sums, nullptr);
+}
+
 int wfr_moments_queue(const SRWLWfr& w, const float2* dEx, const float2* dEz, long long perE, long long perX,
                       long long perZ, MomQueued& q)
 {
@@ -65,30 +83,10 @@ int wfr_moments_queue(const SRWLWfr& w, const float2* dEx, const float2* dEz, lo
     if (w.mesh.nx <= 1 && w.mesh.ny <= 1) return 0;
     int rc = ensure_device();
     if (rc) return rc;
-    int n = (int)w.mesh.ne;
-    // pinned: slice table, then 24 sums per slice
-    size_t slBytes = ((sizeof(srwm_mslice) * n + 255) / 256) * 256;
-    size_t bytes = slBytes + sizeof(double) * 24 * n;
-    if (bytes > g_ctx.momPinBytes) {
-        if (g_ctx.momPin) (void)hipHostFree(g_ctx.momPin);
-        g_ctx.momPin = nullptr;
-        g_ctx.momPinBytes = 0;
-        if (hipHostMalloc((void**)&g_ctx.momPin, bytes, hipHostMallocDefault) != hipSuccess) {
-            g_ctx.momPin = nullptr;
-            return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
-        }
-        g_ctx.momPinBytes = bytes;
-    }
-    srwm_mslice* sl = (srwm_mslice*)g_ctx.momPin;
-    q.sums = (double*)(g_ctx.momPin + slBytes);
-    int nxMax = 1, nzMax = 1;
-    for (long ie = 0; ie < n; ie++) {
-        sl[ie] = wfr_slice(w, dEx, dEz, perE, perX, perZ, ie);
-        nxMax = std::max(nxMax, sl[ie].nx);
-        nzMax = std::max(nzMax, sl[ie].nz);
-    }
-    q.sl.assign(sl, sl + n);
-    rc = queue_sums(sl, n, nxMax, nzMax, perE == 1 && n > 1, q.sums, nullptr);
+    const int n = (int)w.mesh.ne;
+    q.sl.clear();
+    for (long ie = 0; ie < n; ie++) q.sl.push_back(wfr_slice(w, dEx, dEz, perE, perX, perZ, ie));
+    rc = device_moments_queue(q.sl, perE == 1 && n > 1, q);
     if (rc) return rc;
     q.n = n;
     q.hasX = dEx != nullptr;

@@ -410,13 +410,12 @@ SRWL_EXPORT int srwlPropagElecField(SRWLWfr* pWfr, SRWLOptC* pOpt, int nInt, cha
     float2* dS = (float2*)bufCur->get(sizeof(float2) * 2 * n);
     srwf_slice* dSp = (srwf_slice*)g_ctx.buf.W2.get(sizeof(srwf_slice) * 2 * ne);
     if (!dIn || !dS || !dSp) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
-    HIPCHK(hipMemcpyAsync(dIn, pWfr->arEx, sizeof(float2) * n, hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dIn + n, pWfr->arEy, sizeof(float2) * n, hipMemcpyHostToDevice, st));
     // slice-major layout: slice (2*ie + comp) holds [iy][ix]
-    if (ne == 1) {
-        for (int c = 0; c < 2; c++)
-            HIPCHK(hipMemcpyAsync(dS + c * nxy, dIn + c * n, sizeof(float2) * nxy, hipMemcpyDeviceToDevice, st));
-    } else {
+    float2* dUp = ne == 1 ? dS : dIn;
+    const XferSeg in[2] = {{pWfr->arEx, dUp, sizeof(float2) * (size_t)n}, {pWfr->arEy, dUp + n, sizeof(float2) * (size_t)n}};
+    rc = upload_segs(in, 2);
+    if (rc) return rc;
+    if (ne > 1) {
         if (srwf_launch_slices(dIn, dIn + n, dS, (int)ne, nxy, 1, st)) return SRWL_AMD_ERR_GPU;
     }
     if (g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev2, st));
@@ -615,13 +614,11 @@ SRWL_EXPORT int srwlPropagElecField(SRWLWfr* pWfr, SRWLOptC* pOpt, int nInt, cha
         if ((*g_wfrModif)(2, pWfr, 0)) return SRWL_WFR_EXT_MODIF_FAILED;
         if (pWfr->arEx == nullptr || pWfr->arEy == nullptr) return SRWL_WFR_EXT_MODIF_FAILED;
     }
-    if (ne == 1) {
-        HIPCHK(hipMemcpyAsync(pWfr->arEx, dS, sizeof(float2) * nxy, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(pWfr->arEy, dS + nxy, sizeof(float2) * nxy, hipMemcpyDeviceToHost, st));
-    } else {
-        HIPCHK(hipMemcpyAsync(pWfr->arEx, dIn, sizeof(float2) * n, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(pWfr->arEy, dIn + n, sizeof(float2) * n, hipMemcpyDeviceToHost, st));
-    }
+    const float2* dOut = ne == 1 ? dS : dIn;
+    const XferSeg out[2] = {{pWfr->arEx, (void*)dOut, sizeof(float2) * (size_t)n},
+                            {pWfr->arEy, (void*)(dOut + n), sizeof(float2) * (size_t)n}};
+    rc = download_segs(out, 2);
+    if (rc) return rc;
     HIPCHK(hipStreamSynchronize(st));
     if (g_ctx.timing) {
         float ms = 0;
@@ -666,7 +663,9 @@ SRWL_EXPORT int srwlUtiFFT(char* pcData, char typeData, double* arMesh, int nMes
     S.sh1y = shZ ? t0s * z0 : 0.;
     S.ny = (int)nz;
     HIPCHK(hipMemcpyAsync(dSp, &S, sizeof(S), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(d, pcData, sizeof(float2) * nxy, hipMemcpyHostToDevice, st));
+    const XferSeg in{pcData, d, sizeof(float2) * (size_t)nxy};
+    rc = upload_segs(&in, 1);
+    if (rc) return rc;
     int inv = dir > 0 ? 0 : 1;
     if (p2) {
         const float2* twx = twiddles(lx);
@@ -687,8 +686,8 @@ SRWL_EXPORT int srwlUtiFFT(char* pcData, char typeData, double* arMesh, int nMes
         if (srwf_launch_gtranspose(d, t, (int)nz, (int)nx, nxy, 1, st)) return SRWL_AMD_ERR_GPU;
         if (srwf_launch_gcols(t, nxy, 1, dSp, twz, pz, (int)nx, 2, inv, o, st)) return SRWL_AMD_ERR_GPU;
     }
-    HIPCHK(hipMemcpyAsync(pcData, o, sizeof(float2) * nxy, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    rc = download(pcData, o, sizeof(float2) * (size_t)nxy);
+    if (rc) return rc;
     arMesh[0] = xStartTr; arMesh[1] = xStepTr; arMesh[3] = zStartTr; arMesh[4] = zStepTr;
     return 0;
 }
@@ -793,14 +792,16 @@ SRWL_EXPORT int srwlCalcIntFromElecField(char* pInt, SRWLWfr* pWfr, char pol, ch
     if (!d || !o || !rows) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
     float2* dx = pWfr->arEx ? d : nullptr;
     float2* dz = pWfr->arEy ? d + n : nullptr;
-    if (dx) HIPCHK(hipMemcpyAsync(dx, pWfr->arEx, sizeof(float2) * n, hipMemcpyHostToDevice, st));
-    if (dz) HIPCHK(hipMemcpyAsync(dz, pWfr->arEy, sizeof(float2) * n, hipMemcpyHostToDevice, st));
+    XferSeg in[3];
+    int nIn = 0;
+    if (dx) in[nIn++] = XferSeg{pWfr->arEx, dx, sizeof(float2) * (size_t)n};
+    if (dz) in[nIn++] = XferSeg{pWfr->arEy, dz, sizeof(float2) * (size_t)n};
     // the averaging and sum modes update the caller's previous values
-    if (P.iter != 0.) HIPCHK(hipMemcpyAsync(o, pInt, outBytes, hipMemcpyHostToDevice, st));
+    if (P.iter != 0.) in[nIn++] = XferSeg{pInt, o, outBytes};
+    rc = upload_segs(in, nIn);
+    if (rc) return rc;
     if (srwx_launch_extract(dx, dz, P, o, rows, st)) return SRWL_AMD_ERR_GPU;
-    HIPCHK(hipMemcpyAsync(pInt, o, what == 4 ? sizeof(float) * P.ne : outBytes, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    return 0;
+    return download(pInt, o, what == 4 ? sizeof(float) * (size_t)P.ne : outBytes);
 }
 
 }  // extern "C"

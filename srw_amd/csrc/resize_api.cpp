@@ -185,8 +185,9 @@ SRWL_EXPORT int srwlResizeElecField(SRWLWfr* pWfr, char type, double* par)
     float2* dO = (float2*)g_ctx.buf.RsO.get(sizeof(float2) * 2 * nOld);
     float2* dN = (float2*)g_ctx.buf.RsN.get(sizeof(float2) * 2 * nNew);
     if (!dO || !dN) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
-    HIPCHK(hipMemcpyAsync(dO, pWfr->arEx, sizeof(float2) * nOld, hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dO + nOld, pWfr->arEy, sizeof(float2) * nOld, hipMemcpyHostToDevice, st));
+    const XferSeg in[2] = {{pWfr->arEx, dO, sizeof(float2) * (size_t)nOld}, {pWfr->arEy, dO + nOld, sizeof(float2) * (size_t)nOld}};
+    rc = upload_segs(in, 2);
+    if (rc) return rc;
     srwr_layout lo = {ne, ne * pWfr->mesh.nx, 1};
     srwr_layout ln = {ne, ne * P.x.n, 1};
     rc = device_resize(*pWfr, P, dO, dO + nOld, lo, dN, dN + nNew, ln, st);
@@ -194,8 +195,9 @@ SRWL_EXPORT int srwlResizeElecField(SRWLWfr* pWfr, char type, double* par)
     HIPCHK(hipStreamSynchronize(st));
     rc = realloc_wfr_arrays(*pWfr, P);
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(pWfr->arEx, dN, sizeof(float2) * nNew, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(pWfr->arEy, dN + nNew, sizeof(float2) * nNew, hipMemcpyDeviceToHost, st));
+    const XferSeg out[2] = {{pWfr->arEx, dN, sizeof(float2) * (size_t)nNew}, {pWfr->arEy, dN + nNew, sizeof(float2) * (size_t)nNew}};
+    rc = download_segs(out, 2);
+    if (rc) return rc;
     HIPCHK(hipStreamSynchronize(st));
     return 0;
 }
@@ -276,8 +278,9 @@ SRWL_EXPORT int srwlResizeElecFieldMesh(SRWLWfr* pWfr, SRWLRadMesh* pMesh, doubl
     float2* dO = (float2*)g_ctx.buf.RsO.get(sizeof(float2) * 2 * nOld);
     float2* dN = (float2*)g_ctx.buf.RsN.get(sizeof(float2) * 2 * nNew);
     if (!dO || !dN) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
-    HIPCHK(hipMemcpyAsync(dO, pWfr->arEx, sizeof(float2) * nOld, hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dO + nOld, pWfr->arEy, sizeof(float2) * nOld, hipMemcpyHostToDevice, st));
+    const XferSeg in[2] = {{pWfr->arEx, dO, sizeof(float2) * (size_t)nOld}, {pWfr->arEy, dO + nOld, sizeof(float2) * (size_t)nOld}};
+    rc = upload_segs(in, 2);
+    if (rc) return rc;
     srwr_layout lo = {ne, ne * nx, 1};
     srwr_layout ln = {ne, ne * (long long)mn.nx, 1};
     rc = device_resize(*pWfr, P, dO, dO + nOld, lo, dN, dN + nNew, ln, st);
@@ -285,8 +288,9 @@ SRWL_EXPORT int srwlResizeElecFieldMesh(SRWLWfr* pWfr, SRWLRadMesh* pMesh, doubl
     HIPCHK(hipStreamSynchronize(st));
     rc = realloc_wfr_arrays(*pWfr, P);
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(pWfr->arEx, dN, sizeof(float2) * nNew, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(pWfr->arEy, dN + nNew, sizeof(float2) * nNew, hipMemcpyDeviceToHost, st));
+    const XferSeg out[2] = {{pWfr->arEx, dN, sizeof(float2) * (size_t)nNew}, {pWfr->arEy, dN + nNew, sizeof(float2) * (size_t)nNew}};
+    rc = download_segs(out, 2);
+    if (rc) return rc;
     HIPCHK(hipStreamSynchronize(st));
     return 0;
 }

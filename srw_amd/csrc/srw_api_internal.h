@@ -34,6 +34,8 @@ struct Arena {
 // Most row bands of one request (the FP64 counts of the bands are read back
 // through a pinned array of 64).
 #define SRWL_AMD_MAX_BANDS 32
+// Pieces of a staged host transfer in flight.
+#define SRWL_AMD_XFER_SLOTS 8
 // FP64 store records a streamed-rows call patches into the caller's arrays
 // (more: the whole field is downloaded again), and the longest the host
 // waits for the blocks' flags before it falls back to a plain download.
@@ -100,6 +102,7 @@ struct Context {
     hipStream_t copyStream = nullptr;
     hipStream_t stream2 = nullptr;          // second compute stream: alternate row bands overlap their tails
     hipEvent_t evFork = nullptr, evJoin = nullptr;
+    hipEvent_t evXfer[SRWL_AMD_XFER_SLOTS] = {};   // pieces of a staged transfer
     char* pin = nullptr;                    // pinned staging (grow-only)
     size_t pinBytes = 0;
     char* up = nullptr;           // pinned staging of setup uploads (bump allocated per SR call)
@@ -174,8 +177,19 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
 // the staging of downloads; nullptr on failure.
 char* grow_pinned(char*& p, size_t& have, size_t bytes);
 char* pinned_staging(size_t bytes);
-// Copies device memory to host memory through the pinned staging on the copy
-// stream, in pieces, after the work already queued on the compute stream.
+// Copies between device memory and the caller's (pageable) arrays through the
+// pinned staging, in pieces, the DMA of one piece beside the host copy of
+// another.  download_segs returns when the arrays hold the data: the copies run
+// on the copy stream after event `after`, or after the work already queued on
+// the compute stream when it is nullptr.  upload_segs returns when the arrays
+// have been read; the copies are queued on the compute stream.
+struct XferSeg {
+    void* host;
+    void* dev;
+    size_t n;
+};
+int download_segs(const XferSeg* seg, int nSeg, hipEvent_t after = nullptr);
+int upload_segs(const XferSeg* seg, int nSeg);
 int download(void* dst, const void* src, size_t bytes);
 // Host memcpy split over a pool of threads (large copies out of pinned
 // memory): one range, or several ranges as one job.
@@ -219,6 +233,8 @@ struct MomQueued {
 };
 int wfr_moments_queue(const SRWLWfr& w, const float2* dEx, const float2* dEz, long long perE, long long perX,
                       long long perZ, MomQueued& q);
+// The same for any slices: the kernels and the read-back of q.sums queued.
+int device_moments_queue(const std::vector<srwm_mslice>& slices, bool lanesOverSlices, MomQueued& q);
 void wfr_moments_collect(const MomQueued& q, double* momX, double* momZ);
 srwm_mslice wfr_slice(const SRWLWfr& w, const float2* dEx, const float2* dEz, long long perE, long long perX,
                       long long perZ, long ie);

@@ -21,6 +21,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -48,6 +49,8 @@ int ensure_device()
     if (hipEventCreateWithFlags(&g_ctx.evFork, hipEventDisableTiming) != hipSuccess) return SRWL_AMD_ERR_GPU;
     if (hipEventCreateWithFlags(&g_ctx.evJoin, hipEventDisableTiming) != hipSuccess) return SRWL_AMD_ERR_GPU;
     if (hipEventCreateWithFlags(&g_ctx.evTiles, hipEventDisableTiming) != hipSuccess) return SRWL_AMD_ERR_GPU;
+    for (hipEvent_t& e : g_ctx.evXfer)
+        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return SRWL_AMD_ERR_GPU;
     if (hipHostMalloc((void**)&g_ctx.fpCountHost, sizeof(int) * 64, hipHostMallocDefault) != hipSuccess)
         return SRWL_AMD_ERR_GPU;
     g_ctx.fpCountHost[0] = 0;
@@ -250,6 +253,19 @@ static int mesh_split(long long nTiles, long long nUnits, long long nPts)
         if (t < bestT * 0.98) { bestT = t; best = (int)n; }
     }
     return best;
+}
+
+// A field in one piece into the caller's arrays, behind the work queued so far;
+// the caller's further device work is queued first and runs beside the copies.
+static int field_to_host(const HostOut& out, float* dEx, float* dEz, size_t bytes, const std::vector<SrResult>& res)
+{
+    HIPCHK(hipEventRecord(g_ctx.evFork, g_ctx.stream));
+    if (out.queueMore) {
+        const int rc = out.queueMore(out.queueCtx, res);
+        if (rc) return rc;
+    }
+    const XferSeg seg[2] = {{out.ex, dEx, bytes}, {out.ez, dEz, bytes}};
+    return download_segs(seg, 2, g_ctx.evFork);
 }
 
 // Runs the single-electron SR computation for a set of requests.  Outputs
@@ -475,8 +491,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         if (hostOut) {
             const SRWLRadMesh& m = jobs[0].mesh;
             size_t n = sizeof(float) * 2 * (size_t)m.ne * m.nx * m.ny;
-            rc = download(hostOut->ex, dEx, n);
-            if (!rc) rc = download(hostOut->ez, dEz, n);
+            rc = field_to_host(*hostOut, dEx, dEz, n, res);
             if (rc) return rc;
         }
         long long ev = 0;
@@ -922,8 +937,8 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             // flags not all seen, or more FP64 stores than the patch area
             // holds: the whole field, now final, the plain way
             HIPCHK(hipStreamSynchronize(g_ctx.copyStream));
-            rc = download(hostOut->ex, dEx, compBytes);
-            if (!rc) rc = download(hostOut->ez, dEz, compBytes);
+            const XferSeg seg[2] = {{hostOut->ex, dEx, compBytes}, {hostOut->ez, dEz, compBytes}};
+            rc = download_segs(seg, 2);
             if (rc) return rc;
         } else {
             // the FP64-recomputed values over what the bands carried
@@ -1033,9 +1048,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         HIPCHK(hipMemcpyAsync(hostOut->ex, dEx, compBytes, hipMemcpyDeviceToHost, st));
         HIPCHK(hipMemcpyAsync(hostOut->ez, dEz, compBytes, hipMemcpyDeviceToHost, st));
     } else if (hostOut) {
-        size_t n = compBytes;
-        rc = download(hostOut->ex, dEx, n);
-        if (!rc) rc = download(hostOut->ez, dEz, n);
+        rc = field_to_host(*hostOut, dEx, dEz, compBytes, res);
         if (rc) return rc;
     }
     if (defer) return 0;
@@ -1088,11 +1101,16 @@ void copy_stream(void* dst, const void* src, size_t n)
     _mm_sfence();
 }
 
-// Host copies out of the pinned staging: a pool of worker threads started on
-// first use and kept for the life of the process (starting threads per copy
+// Host copies to and from the pinned staging: a pool of worker threads started
+// on first use and kept for the life of the process (starting threads per copy
 // costs more than a small band's copy).  A job is a list of ranges cut into
-// 1 MiB pieces that the workers and the calling thread take in turn.  A forked
-// child, which has none of the workers, copies on its own thread.
+// pieces that the workers and the calling thread take in turn; the caller
+// leaves when every piece is copied, without waiting for workers that woke too
+// late to take one (each holds its job's list by itself).  After a job a worker
+// looks for the next one for some tens of microseconds before it sleeps: a
+// staged transfer is a run of jobs about that far apart, and waking a thread
+// takes as long.  A forked child, which has none of the workers, copies on its
+// own thread.
 class CopyPool {
 public:
     explicit CopyPool(unsigned nWorkers) : pid_(getpid())
@@ -1104,56 +1122,57 @@ public:
     {
         size_t total = 0;
         for (int k = 0; k < nSeg; k++) total += seg[k].n;
-        if (workers_ == 0 || total <= kPiece || getpid() != pid_) {
+        if (workers_ == 0 || total <= 2 * kPiece || getpid() != pid_) {
             for (int k = 0; k < nSeg; k++) copy_stream(seg[k].dst, seg[k].src, seg[k].n);
             return;
         }
-        std::lock_guard<std::mutex> one(job_);   // one job at a time
-        pieces_.clear();
+        auto job = std::make_shared<Job>();
         for (int k = 0; k < nSeg; k++)
             for (size_t o = 0; o < seg[k].n; o += kPiece)
-                pieces_.push_back(CopySeg{(char*)seg[k].dst + o, (const char*)seg[k].src + o,
-                                          std::min(kPiece, seg[k].n - o)});
-        next_.store(0);
+                job->p.push_back(CopySeg{(char*)seg[k].dst + o, (const char*)seg[k].src + o,
+                                         std::min(kPiece, seg[k].n - o)});
         {
             std::lock_guard<std::mutex> l(m_);
-            pending_ = workers_;
-            gen_++;
+            job_ = job;
+            gen_.fetch_add(1);
         }
         cv_.notify_all();
-        run();
-        std::unique_lock<std::mutex> l(m_);
-        cvDone_.wait(l, [&] { return pending_ == 0; });
+        run(*job);
+        while (job->done.load() < job->p.size()) _mm_pause();
     }
 
 private:
-    static constexpr size_t kPiece = 1 << 20;
-    void run()
+    struct Job {
+        std::vector<CopySeg> p;
+        std::atomic<size_t> next{0}, done{0};
+    };
+    static constexpr size_t kPiece = 256 << 10;
+    static void run(Job& j)
     {
-        for (size_t k; (k = next_.fetch_add(1)) < pieces_.size();)
-            copy_stream(pieces_[k].dst, pieces_[k].src, pieces_[k].n);
+        for (size_t k; (k = j.next.fetch_add(1)) < j.p.size(); j.done.fetch_add(1))
+            copy_stream(j.p[k].dst, j.p[k].src, j.p[k].n);
     }
     void worker()
     {
         unsigned seen = 0;
         for (;;) {
+            for (int i = 0; i < 2000 && gen_.load() == seen; i++) _mm_pause();
+            std::shared_ptr<Job> job;
             {
                 std::unique_lock<std::mutex> l(m_);
-                cv_.wait(l, [&] { return gen_ != seen; });
-                seen = gen_;
+                cv_.wait(l, [&] { return gen_.load() != seen; });
+                seen = gen_.load();
+                job = job_;
             }
-            run();
-            std::lock_guard<std::mutex> l(m_);
-            if (--pending_ == 0) cvDone_.notify_one();
+            run(*job);
         }
     }
     pid_t pid_;
     unsigned workers_ = 0;
-    std::mutex job_, m_;
-    std::condition_variable cv_, cvDone_;
-    std::vector<CopySeg> pieces_;
-    std::atomic<size_t> next_{0};
-    unsigned pending_ = 0, gen_ = 0;
+    std::mutex m_;
+    std::condition_variable cv_;
+    std::shared_ptr<Job> job_;
+    std::atomic<unsigned> gen_{0};
 };
 
 CopyPool& copy_pool()
@@ -1173,39 +1192,71 @@ void par_memcpy(void* dst, const void* src, size_t bytes)
     par_memcpy(&s, 1);
 }
 
-int download(void* dst, const void* src, size_t bytes)
+namespace {
+// Pieces of a list of transfers: an eighth of the whole, between 256 KB (a
+// DMA's fixed cost is about 10 us, the time of 512 KB) and 4 MB.
+struct XferPieces {
+    std::vector<XferSeg> p;
+    size_t piece = 0;
+    XferPieces(const XferSeg* seg, int nSeg)
+    {
+        size_t total = 0;
+        for (int k = 0; k < nSeg; k++) total += seg[k].n;
+        piece = std::min<size_t>(4 << 20, std::max<size_t>(256 << 10, (total / SRWL_AMD_XFER_SLOTS + 4095) & ~(size_t)4095));
+        for (int k = 0; k < nSeg; k++)
+            for (size_t o = 0; o < seg[k].n; o += piece)
+                p.push_back(XferSeg{(char*)seg[k].host + o, (char*)seg[k].dev + o, std::min(piece, seg[k].n - o)});
+    }
+    size_t staging() const { return piece * std::min<size_t>(p.size(), SRWL_AMD_XFER_SLOTS); }
+};
+}  // namespace
+
+int download_segs(const XferSeg* seg, int nSeg, hipEvent_t after)
 {
-    // pieces of up to 32 MiB through the pinned staging: the DMA of piece k + 1
-    // overlaps the host copy of piece k
-    const size_t piece = 32 << 20;
-    size_t np = (bytes + piece - 1) / piece;
-    char* pin = pinned_staging(std::min(bytes, 2 * piece));
+    const XferPieces X(seg, nSeg);
+    if (X.p.empty()) return 0;
+    char* pin = pinned_staging(X.staging());
     if (!pin) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
-    while (g_ctx.bandEv.size() < 4) {
-        hipEvent_t e;
-        HIPCHK(hipEventCreate(&e));
-        g_ctx.bandEv.push_back(e);
+    if (!after) {
+        after = g_ctx.evFork;
+        HIPCHK(hipEventRecord(after, g_ctx.stream));
     }
-    HIPCHK(hipEventRecord(g_ctx.bandEv[0], g_ctx.stream));
-    HIPCHK(hipStreamWaitEvent(g_ctx.copyStream, g_ctx.bandEv[0], 0));
-    for (size_t k = 0; k < np; k++) {
-        size_t o = k * piece, n = std::min(piece, bytes - o);
-        char* stage = pin + (k & 1) * piece;
-        if (k >= 2) HIPCHK(hipEventSynchronize(g_ctx.bandEv[2 + (k & 1)]));   // stage free again
-        HIPCHK(hipMemcpyAsync(stage, (const char*)src + o, n, hipMemcpyDeviceToHost, g_ctx.copyStream));
-        HIPCHK(hipEventRecord(g_ctx.bandEv[2 + (k & 1)], g_ctx.copyStream));
-        if (k >= 1) {
-            size_t op = (k - 1) * piece, npv = std::min(piece, bytes - op);
-            HIPCHK(hipEventSynchronize(g_ctx.bandEv[2 + ((k - 1) & 1)]));
-            par_memcpy((char*)dst + op, pin + ((k - 1) & 1) * piece, npv);
+    HIPCHK(hipStreamWaitEvent(g_ctx.copyStream, after, 0));
+    const size_t S = SRWL_AMD_XFER_SLOTS, np = X.p.size();
+    for (size_t k = 0, next = 0; k < np; k++) {
+        for (; next < np && next < k + S; next++) {   // slot of piece k - 1 is free again
+            HIPCHK(hipMemcpyAsync(pin + (next % S) * X.piece, X.p[next].dev, X.p[next].n, hipMemcpyDeviceToHost,
+                                  g_ctx.copyStream));
+            HIPCHK(hipEventRecord(g_ctx.evXfer[next % S], g_ctx.copyStream));
         }
-    }
-    if (np > 0) {
-        size_t k = np - 1, o = k * piece, n = std::min(piece, bytes - o);
-        HIPCHK(hipEventSynchronize(g_ctx.bandEv[2 + (k & 1)]));
-        par_memcpy((char*)dst + o, pin + (k & 1) * piece, n);
+        HIPCHK(hipEventSynchronize(g_ctx.evXfer[k % S]));
+        par_memcpy(X.p[k].host, pin + (k % S) * X.piece, X.p[k].n);
     }
     return 0;
+}
+
+int upload_segs(const XferSeg* seg, int nSeg)
+{
+    const XferPieces X(seg, nSeg);
+    if (X.p.empty()) return 0;
+    // an earlier upload may still read the staging
+    HIPCHK(hipStreamSynchronize(g_ctx.stream));
+    char* pin = pinned_staging(X.staging());
+    if (!pin) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+    const size_t S = SRWL_AMD_XFER_SLOTS, np = X.p.size();
+    for (size_t k = 0; k < np; k++) {
+        if (k >= S) HIPCHK(hipEventSynchronize(g_ctx.evXfer[k % S]));
+        par_memcpy(pin + (k % S) * X.piece, X.p[k].host, X.p[k].n);
+        HIPCHK(hipMemcpyAsync(X.p[k].dev, pin + (k % S) * X.piece, X.p[k].n, hipMemcpyHostToDevice, g_ctx.stream));
+        HIPCHK(hipEventRecord(g_ctx.evXfer[k % S], g_ctx.stream));
+    }
+    return 0;
+}
+
+int download(void* dst, const void* src, size_t bytes)
+{
+    const XferSeg s{dst, (void*)src, bytes};
+    return download_segs(&s, 1);
 }
 
 SrRegion sr_region(const SRWLRadMesh& m, const srwd_trj_info& I)
@@ -1599,6 +1650,7 @@ SRWL_EXPORT int srwlCalcElecFieldSRBatch(SRWLWfr** arWfr, SRWLMagFldC** arMagFld
     rc = sr_run(jobs, fields, dEx, dEz, off, res, termin, true);
     if (rc) return rc;
     int warn = 0;
+    std::vector<XferSeg> segs;
     std::vector<srwm_mslice> momSl;
     std::vector<std::pair<int, int>> momOwner;   // (request, energy) of each slice
     long long nAdj = 0;
@@ -1606,10 +1658,8 @@ SRWL_EXPORT int srwlCalcElecFieldSRBatch(SRWLWfr** arWfr, SRWLMagFldC** arMagFld
         SRWLWfr* w = arWfr[i];
         long long n = (long long)w->mesh.ne * w->mesh.nx * w->mesh.ny;
         if (!g_ctx.keepOnDevice) {
-            HIPCHK(hipMemcpyAsync(w->arEx, dEx + 2 * off[i], sizeof(float) * 2 * n, hipMemcpyDeviceToHost,
-                                  g_ctx.stream));
-            HIPCHK(hipMemcpyAsync(w->arEy, dEz + 2 * off[i], sizeof(float) * 2 * n, hipMemcpyDeviceToHost,
-                                  g_ctx.stream));
+            segs.push_back(XferSeg{w->arEx, dEx + 2 * off[i], sizeof(float) * 2 * (size_t)n});
+            segs.push_back(XferSeg{w->arEy, dEz + 2 * off[i], sizeof(float) * 2 * (size_t)n});
         }
         w->Rx = w->Ry = res[i].Robs; w->dRx = w->dRy = res[i].RobsErr;
         w->xc = res[i].xc; w->yc = res[i].zc;
@@ -1625,12 +1675,18 @@ SRWL_EXPORT int srwlCalcElecFieldSRBatch(SRWLWfr** arWfr, SRWLMagFldC** arMagFld
         w->avgPhotEn = 0.5 * (w->mesh.eStart + w->mesh.eFin);
         w->presCA = 0; w->presFT = 0;
     }
+    // all requests' slices in one device pass, queued before the fields travel
+    HIPCHK(hipEventRecord(g_ctx.evFork, g_ctx.stream));
+    MomQueued mq;
     if (!momSl.empty()) {
-        // all requests' slices in one device pass
-        std::vector<double> sums;
-        std::vector<int> lims;
-        rc = device_moments(momSl, sums, lims, 2 * nAdj > (long long)momSl.size());
+        rc = device_moments_queue(momSl, 2 * nAdj > (long long)momSl.size(), mq);
         if (rc) return rc;
+    }
+    rc = download_segs(segs.data(), (int)segs.size(), g_ctx.evFork);
+    if (rc) return rc;
+    HIPCHK(hipStreamSynchronize(g_ctx.stream));
+    if (!momSl.empty()) {
+        const double* sums = mq.sums;
         for (size_t k = 0; k < momSl.size(); k++) {
             SRWLWfr* w = arWfr[momOwner[k].first];
             int ie = momOwner[k].second;
@@ -1638,7 +1694,6 @@ SRWL_EXPORT int srwlCalcElecFieldSRBatch(SRWLWfr** arWfr, SRWLMagFldC** arMagFld
             if (w->arMomY) moments_from_sums(&sums[24 * k + 11], momSl[k], w->arMomY + 11 * ie);
         }
     }
-    HIPCHK(hipStreamSynchronize(g_ctx.stream));
     sr_complete(res);
     for (auto& r : res) if (r.warn) warn = r.warn;
     return warn;
