@@ -475,6 +475,7 @@ __device__ void picard_arrive(const rk_ctx& c, double* y, double h, long long n,
 // for ranges on one side of ct = 0.
 // ------------------------------------------------------------------------
 #define SRWD_SW_THREADS 256
+#define SRWD_SW_TEST 4       // first sweep that compares its points with the previous one's
 
 // Chain of one block of k_traj_init / k_traj_sweep: the upstream chain's
 // blocks come first, then the downstream chain's.
@@ -524,11 +525,34 @@ __device__ __forceinline__ sw_chain sw_setup(const srwd_traj_job& J, int b)
     return c;
 }
 
-// Scratch of one trajectory (srwd_traj_scratch doubles): the increments
-// [5][ld], the z positions [ld] when the caller takes none, the block totals
-// [2][2 sides][blocks][5]; at the end, clear of what k_traj_picard uses, the
-// sweeps' records [2 sides][SRWD_SW_MAX + 1][12]: 5 largest changes, 5 largest
-// magnitudes, 1 when the sweep ran; record 0 holds the chain's start point.
+// Wave sums of doubles by data-parallel-primitive moves (no LDS round trip):
+// inclusive scan over the 64 lanes; lane 63 ends with the wave's sum.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_zero(double x)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, ROWS, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ double wave_scan(double x)
+{
+    x += dpp_zero<0x111, 0xf>(x);   // row_shr 1, 2, 4, 8 within rows of 16
+    x += dpp_zero<0x112, 0xf>(x);
+    x += dpp_zero<0x114, 0xf>(x);
+    x += dpp_zero<0x118, 0xf>(x);
+    x += dpp_zero<0x142, 0xa>(x);   // row_bcast 15 into rows 1 and 3
+    x += dpp_zero<0x143, 0xc>(x);   // row_bcast 31 into rows 2 and 3
+    return x;
+}
+
+// Scratch of one trajectory (srwd_traj_scratch doubles): the increments'
+// inclusive sums within their block [5][ld], the z positions [ld] when the
+// caller takes none, the block totals [2][2 sides][blocks][5]; at the end,
+// clear of what k_traj_picard uses, the sweeps' records [2 sides][12]: the
+// chain's start point, its magnitudes, and in the last two places as integers
+// the sweep that found the chain converged (0: none) and per sweep two bits
+// (something moved, something not finite).
 struct sw_scratch {
     double *D, *Z, *tot, *rec;
     long long nb;
@@ -538,27 +562,18 @@ struct sw_scratch {
         Z = D + 5 * ld;
         tot = Z + ld;
         nb = ld / SRWD_SW_THREADS + 2;
-        rec = D + per - 2 * (SRWD_SW_MAX + 1) * 12;
+        rec = D + per - 2 * 12;
     }
     __device__ __forceinline__ double* total(int sweep, int side, long long b) const
     {
         return tot + (((sweep & 1) * 2 + side) * nb + b) * 5;
     }
-    __device__ __forceinline__ double* record(int side, int sweep) const { return rec + (side * (SRWD_SW_MAX + 1) + sweep) * 12; }
+    __device__ __forceinline__ double* start(int side) const { return rec + side * 12; }
+    __device__ __forceinline__ double* magnitude(int side) const { return rec + side * 12 + 5; }
+    __device__ __forceinline__ int* converged(int side) const { return (int*)(rec + side * 12 + 10); }
+    __device__ __forceinline__ unsigned* moved(int side) const { return (unsigned*)(rec + side * 12 + 11); }
 };
-
-// State of a chain after sweep k: 0 not run, 1 to be continued, 2 converged,
-// 3 not finite.
-__device__ __forceinline__ int sw_state(const double* r)
-{
-    if (r[10] != 1.) return 0;
-    bool done = true;
-    for (int k = 0; k < 5; k++) {
-        if (!isfinite(r[k])) return 3;
-        done = done && (r[k] <= 1e-15 * r[5 + k]);
-    }
-    return done ? 2 : 1;
-}
+static_assert(2 * SRWD_SW_MAX <= 32, "two bits per sweep");
 
 // Whether both chains of trajectory tr converged in the sweeps.
 __device__ __forceinline__ bool sw_converged(const srwd_traj_job& J, double* scratch, int tr, long long ld, long long per)
@@ -566,38 +581,31 @@ __device__ __forceinline__ bool sw_converged(const srwd_traj_job& J, double* scr
     bool has[2];
     if (!sw_spans_zero(J, has[0], has[1]) || J.np <= 1) return false;
     const sw_scratch S(scratch, tr, ld, per);
-    for (int side = 0; side < 2; side++) {
-        if (!has[side]) continue;
-        bool ok = false;
-        for (int k = 1; k <= SRWD_SW_MAX && !ok; k++) ok = sw_state(S.record(side, k)) == 2;
-        if (!ok) return false;
-    }
+    for (int side = 0; side < 2; side++)
+        if (has[side] && !*S.converged(side) && (*S.moved(side) >> (2 * SRWD_SW_MAX - 2) & 3)) return false;
     return true;
 }
 
-// Increment of point y (none for a chain's last point), stored with the
-// block's total.
+// Increment of point y (none for a chain's last point): its inclusive sum
+// within the block, and the block's total.
 template <int ONE>
 __device__ __forceinline__ void sw_increment(const rk_ctx& rk, const sw_chain& C, const sw_scratch& S, long long ld,
                                              long long j, const double* y, int sweep, double* lds)
 {
-    double D[5] = {0., 0., 0., 0., 0.};
-    if (j < C.n - 1) {
-        rk4_increment<ONE>(rk, y, C.h, D);
-        for (int k = 0; k < 5; k++) S.D[k * ld + C.step(j)] = D[k];
-    }
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    double D[5] = {0., 0., 0., 0., 0.};
+    if (j < C.n - 1) rk4_increment<ONE>(rk, y, C.h, D);
     for (int k = 0; k < 5; k++) {
-        double x = D[k];
-        for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-        if (lane == 0) lds[w * 5 + k] = x;
+        D[k] = wave_scan(D[k]);
+        if (lane == 63) lds[w * 5 + k] = D[k];
     }
     __syncthreads();
-    if (threadIdx.x < 5) {
-        double x = lds[threadIdx.x];
-        for (int q = 1; q < SRWD_SW_THREADS / 64; q++) x += lds[q * 5 + threadIdx.x];
-        S.total(sweep, C.side, C.blk)[threadIdx.x] = x;
+    for (int k = 0; k < 5; k++) {
+        for (int q = 0; q < w; q++) D[k] += lds[q * 5 + k];
+        if (j < C.n - 1) S.D[k * ld + C.step(j)] = D[k];
     }
+    if (threadIdx.x == SRWD_SW_THREADS - 1)
+        for (int k = 0; k < 5; k++) S.total(sweep, C.side, C.blk)[k] = D[k];
 }
 
 // Sweep 0: the chain's start point (one RK4 step from ct = 0 where the grid
@@ -614,8 +622,7 @@ __global__ void __launch_bounds__(SRWD_SW_THREADS) k_traj_init(const srwd_traj_j
     const srwd_traj_job J = jobs[tr];
     const sw_scratch S(scratch, tr, ld, per);
     if (blockIdx.x == 0 && threadIdx.x < 2)
-        for (int k = 1; k <= SRWD_SW_MAX; k++)
-            for (int q = 0; q < 12; q++) S.record(threadIdx.x, k)[q] = 0.;
+        for (int q = 5; q < 12; q++) S.start(threadIdx.x)[q] = 0.;
     const sw_chain C = sw_setup(J, blockIdx.x);
     if (!C.live) return;
     rk_ctx rk;
@@ -627,7 +634,7 @@ __global__ void __launch_bounds__(SRWD_SW_THREADS) k_traj_init(const srwd_traj_j
         rk4_increment<ONE>(rk, y0, C.s0, D);
         for (int k = 0; k < 5; k++) y0[k] += D[k];
     }
-    if (C.blk == 0 && threadIdx.x < 5) S.record(C.side, 0)[threadIdx.x] = y0[threadIdx.x];
+    if (C.blk == 0 && threadIdx.x < 5) S.start(C.side)[threadIdx.x] = y0[threadIdx.x];
     rk_deriv_t<ONE>(rk, y0, d0);
     d0[1] = d0[3] = 0.;
     const long long j = (long long)C.blk * SRWD_SW_THREADS + threadIdx.x;
@@ -647,69 +654,76 @@ __global__ void __launch_bounds__(SRWD_SW_THREADS) k_traj_sweep(const srwd_traj_
                                                                  long long ld, double* scratch, long long per, int sweep)
 {
     const int NW = SRWD_SW_THREADS / 64;
-    __shared__ double lds[10 * NW], ldsT[5 * NW], ldsI[5 * NW];
+    __shared__ double lds[5 * NW], ldsT[5 * NW], ldsM[5 * NW];
     const int tr = blockIdx.y;
     const srwd_traj_job J = jobs[tr];
     const sw_scratch S(scratch, tr, ld, per);
     const sw_chain C = sw_setup(J, blockIdx.x);
-    if (!C.live || (sweep > 1 && sw_state(S.record(C.side, sweep - 1)) != 1)) return;
+    if (!C.live || *S.converged(C.side)) return;
+    // sweeps before SRWD_SW_TEST do not compare: the magnitudes that the
+    // comparison uses are taken in the sweep before it
+    const unsigned mv = sweep > SRWD_SW_TEST ? *S.moved(C.side) >> (2 * sweep - 4) & 3 : 1u;
+    if (mv != 1u) {
+        // the previous sweep moved nothing: the points are final (or, with
+        // something not finite, left to k_traj_picard)
+        if (threadIdx.x == 0 && C.blk == 0) {
+            if (mv == 0) *S.converged(C.side) = sweep - 1;
+            else atomicOr(S.moved(C.side), 3u << (2 * SRWD_SW_MAX - 2) | 3u << (2 * sweep - 2));
+        }
+        return;
+    }
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const long long j = (long long)C.blk * SRWD_SW_THREADS + threadIdx.x, at = C.base + C.dir * j;
-    // totals of the blocks before this one, and the exclusive scan within it
-    double y[5], pre[5] = {0., 0., 0., 0., 0.};
+    double* P[5] = {X + tr * ld, Xp + tr * ld, Y + tr * ld, Yp + tr * ld, Z ? Z + tr * ld : S.Z};
+    // the increments before point j: the totals of the blocks before this one
+    // and the sum within the block up to step j - 1
+    double y[5], old[5], pre[5] = {0., 0., 0., 0., 0.};
+    for (int k = 0; k < 5; k++) {
+        y[k] = threadIdx.x && j < C.n ? S.D[k * ld + C.step(j - 1)] : 0.;
+        old[k] = j < C.n ? P[k][at] : 0.;
+    }
     for (int b = threadIdx.x; b < C.blk; b += SRWD_SW_THREADS) {
         const double* t = S.total(sweep - 1, C.side, b);
         for (int k = 0; k < 5; k++) pre[k] += t[k];
     }
     for (int k = 0; k < 5; k++) {
-        const double D = j < C.n - 1 ? S.D[k * ld + C.step(j)] : 0.;
-        double x = D, t = pre[k];
-        for (int off = 1; off < 64; off <<= 1) {
-            const double u = __shfl_up(x, off, 64);
-            if (lane >= off) x += u;
-        }
-        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
-        if (lane == 63) ldsI[w * 5 + k] = x;
-        if (lane == 0) ldsT[w * 5 + k] = t;
-        const double e = __shfl_up(x, 1, 64);
-        y[k] = lane ? e : 0.;
-    }
-    __syncthreads();
-    const double* y0 = S.record(C.side, 0);
-    for (int k = 0; k < 5; k++) {
-        double t = ldsT[k];
-        for (int q = 1; q < NW; q++) t += ldsT[q * 5 + k];
-        for (int q = 0; q < w; q++) t += ldsI[q * 5 + k];
-        y[k] = y0[k] + (t + y[k]);
-    }
-    double m[10] = {0., 0., 0., 0., 0., 0., 0., 0., 0., 0.};
-    if (j < C.n) {
-        double* P[5] = {X + tr * ld, Xp + tr * ld, Y + tr * ld, Yp + tr * ld, Z ? Z + tr * ld : S.Z};
-        for (int k = 0; k < 5; k++) {
-            const double dv = fabs(y[k] - P[k][at]);
-            m[k] = isfinite(dv) ? dv : INFINITY;
-            m[5 + k] = fabs(y[k]);
-            P[k][at] = y[k];
-        }
-    }
-    for (int k = 0; k < 10; k++) {
-        double x = m[k];
-        for (int off = 32; off > 0; off >>= 1) x = fmax(x, __shfl_xor(x, off, 64));
-        if (lane == 0) lds[w * 10 + k] = x;
+        const double t = wave_scan(pre[k]);
+        if (lane == 63) ldsT[w * 5 + k] = t;
     }
     rk_ctx rk;
     rk_ctx_setup(rk, J, fields);
     __syncthreads();
-    double* R = S.record(C.side, sweep);
-    if (threadIdx.x < 10) {
-        double x = lds[threadIdx.x];
-        for (int q = 1; q < NW; q++) x = fmax(x, lds[q * 10 + threadIdx.x]);
-        // non-negative doubles order as their bit patterns
-        atomicMax((unsigned long long*)R + threadIdx.x, (unsigned long long)__double_as_longlong(x));
+    const double *y0 = S.start(C.side), *mag = S.magnitude(C.side);
+    bool moved = false, bad = false;
+    for (int k = 0; k < 5; k++) {
+        double t = ldsT[k];
+        for (int q = 1; q < NW; q++) t += ldsT[q * 5 + k];
+        y[k] = y0[k] + (t + y[k]);
+        if (j < C.n) {
+            const double dv = fabs(y[k] - old[k]);
+            moved = moved || dv > 1e-15 * mag[k];
+            bad = bad || !isfinite(dv);
+            P[k][at] = y[k];
+        }
     }
-    if (C.blk == 0 && threadIdx.x == 10) R[10] = 1.;
-    __syncthreads();
-    sw_increment<ONE>(rk, C, S, ld, j, y, sweep, ldsI);
+    if (sweep == SRWD_SW_TEST - 1) {
+        for (int k = 0; k < 5; k++) {
+            double x = j < C.n ? fabs(y[k]) : 0.;
+            for (int off = 32; off > 0; off >>= 1) x = fmax(x, __shfl_xor(x, off, 64));
+            if (lane == 0) ldsM[w * 5 + k] = x;
+        }
+        __syncthreads();
+        if (threadIdx.x < 5) {
+            double x = ldsM[threadIdx.x];
+            for (int q = 1; q < NW; q++) x = fmax(x, ldsM[q * 5 + threadIdx.x]);
+            // non-negative doubles order as their bit patterns
+            atomicMax((unsigned long long*)S.magnitude(C.side) + threadIdx.x, (unsigned long long)__double_as_longlong(x));
+        }
+    } else if (sweep >= SRWD_SW_TEST) {
+        const unsigned f = __any(bad) ? 3u : (__any(moved) ? 1u : 0u);
+        if (f && lane == 0) atomicOr(S.moved(C.side), f << (2 * sweep - 2));
+    }
+    sw_increment<ONE>(rk, C, S, ld, j, y, sweep, lds);
 }
 
 // Same trajectory as k_traj_rk4 (srgtrjdt.cpp:90-340), each chain solved by

@@ -160,7 +160,7 @@ inline long long srwd_pic_cap(long long ld) { return ((ld - 1 + 511) / 512) * 51
 // converge in 7-8).
 #define SRWD_SW_MAX 11
 // Scratch of the parallel-in-s RK4, in doubles per trajectory.
-inline long long srwd_traj_scratch(long long ld) { return 20 * srwd_pic_cap(ld) + 2 * (SRWD_SW_MAX + 1) * 12; }
+inline long long srwd_traj_scratch(long long ld) { return 20 * srwd_pic_cap(ld) + 2 * 12; }
 
 // dScratch (srwd_traj_scratch(ld) doubles per trajectory) selects the
 // parallel-in-s solver; nullptr runs the serial kernel.
