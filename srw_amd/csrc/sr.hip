@@ -944,11 +944,18 @@ __device__ __forceinline__ double int_point_s(const srwd_trj_info& I, long long 
 }
 
 // Edge data at the integration limits (srtrjdat.h:1006-1034), end 0 or 1.
+// Outside the magnet the field and its slope there are the rounding of the
+// interpolation's higher derivatives (about 1e-13 T and 5e-10 T/m, decided by
+// the low bits of the positions), which moves fields of low photon energies by
+// 1e-4: a field below 1e-10 T, the reference's own limit of a field-free edge
+// (srtrjdat.h:119), is taken as zero.
 __device__ __forceinline__ void sr_edge(const srwd_trj_info& I, const double* cx, const double* cz, const double* ix,
                                         const double* iz, int end, srwd_edge& E)
 {
     const double s = end ? I.sIntegFin : I.sIntegStart;
-    const trj_pt px = eval_plane(I, cx, ix, -1. / I.betaNorm, s, true), pz = eval_plane(I, cz, iz, 1. / I.betaNorm, s, true);
+    trj_pt px = eval_plane(I, cx, ix, -1. / I.betaNorm, s, true), pz = eval_plane(I, cz, iz, 1. / I.betaNorm, s, true);
+    if (fabs(px.b) < 1.E-10) px.b = px.dbds = 0.;
+    if (fabs(pz.b) < 1.E-10) pz.b = pz.dbds = 0.;
     double* v = E.v[end];
     v[0] = px.dbds; v[1] = px.b; v[2] = px.bt; v[3] = px.crd; v[4] = px.ib;
     v[5] = pz.dbds; v[6] = pz.b; v[7] = pz.bt; v[8] = pz.crd; v[9] = pz.ib;
@@ -1565,7 +1572,7 @@ __global__ void __launch_bounds__(SRWD_CS_THREADS) k_cond_sums(const srwd_trj_in
 // energy t % g of point t / g of the part, so that a wave stores runs of g
 // consecutive energies (the field is stored photon energy fastest).
 __global__ void __launch_bounds__(256) k_sr_finalize(const srwd_item* __restrict__ items,
-                                                     const int2* __restrict__ entries, int g,
+                                                     const int2* __restrict__ entries, int nbU, int g,
                                                      const srwd_trj_info* __restrict__ info,
                                                      const srwd_edge* __restrict__ edges, int termin,
                                                      const double* __restrict__ part, int nSplit,
@@ -1575,7 +1582,7 @@ __global__ void __launch_bounds__(256) k_sr_finalize(const srwd_item* __restrict
                                                      const double* __restrict__ coord,
                                                      const long long* __restrict__ last)
 {
-    const int2 bk = entries[blockIdx.x / g];
+    const int2 bk = entries ? entries[blockIdx.x / g] : make_int2(blockIdx.x / nbU, blockIdx.x % nbU);
     const int q = blockIdx.x % g, e = threadIdx.x % g;
     const int p = q * (256 / g) + threadIdx.x / g;   // point of the 256-point block
     const srwd_item& IT = items[bk.x + e];
@@ -1675,7 +1682,7 @@ __device__ __forceinline__ const double* wave_first_ptr(const double* p)
 //   over the trajectory: one wave per point, the integration points split
 //   over its lanes.
 __global__ void __launch_bounds__(256) k_sr_fp64(const srwd_item* __restrict__ items,
-                                                 const int* __restrict__ blockItem,
+                                                 const int* __restrict__ blockItem, int nbU,
                                                  const srwd_trj_info* __restrict__ info,
                                                  const srwd_edge* __restrict__ edges, int termin,
                                                  const double* __restrict__ T64, long long ldI, float2* Ex,
@@ -1692,7 +1699,7 @@ __global__ void __launch_bounds__(256) k_sr_fp64(const srwd_item* __restrict__ i
         for (int q = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); q < count; q += nWaves) {
             const int entry = fpList[q];
             const int blk = entry >> 8, thr = entry & 255;
-            const srwd_item& IT = items[blockItem[blk]];
+            const srwd_item& IT = items[blockItem ? blockItem[blk] : blk / nbU];
             const int local = (blk - IT.blockBase) * 256 + thr;
             const srwd_trj_info I = info[IT.traj];
             int ix = local % IT.nxc, iz = IT.iz0 + local / IT.nxc;
@@ -1718,7 +1725,7 @@ __global__ void __launch_bounds__(256) k_sr_fp64(const srwd_item* __restrict__ i
             if (q < count) {
                 const int entry = fpList[q];
                 const int blk = entry >> 8, thr = entry & 255;
-                const srwd_item& IT = items[blockItem[blk]];
+                const srwd_item& IT = items[blockItem ? blockItem[blk] : blk / nbU];
                 const int local = (blk - IT.blockBase) * 256 + thr;
                 const srwd_trj_info I = info[IT.traj];
                 int ix = local % IT.nxc, iz = IT.iz0 + local / IT.nxc;
@@ -1743,7 +1750,7 @@ __global__ void __launch_bounds__(256) k_sr_fp64(const srwd_item* __restrict__ i
     for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < count; q += gridDim.x * blockDim.x) {
         const int entry = fpList[q];
         const int blk = entry >> 8, thr = entry & 255;
-        const srwd_item& IT = items[blockItem[blk]];
+        const srwd_item& IT = items[blockItem ? blockItem[blk] : blk / nbU];
         const int local = (blk - IT.blockBase) * 256 + thr;
         const srwd_trj_info I = info[IT.traj];
         int ix = local % IT.nxc, iz = IT.iz0 + local / IT.nxc;
@@ -1763,7 +1770,7 @@ __global__ void __launch_bounds__(256) k_sr_fp64(const srwd_item* __restrict__ i
 // A wave whose points span trajectories reads per lane.  Kept apart from the
 // terminating terms of k_sr_fp64 so that it runs with few registers.
 __global__ void __launch_bounds__(256) k_sr_fp64_sums(const srwd_item* __restrict__ items,
-                                                      const int* __restrict__ blockItem,
+                                                      const int* __restrict__ blockItem, int nbU,
                                                       const srwd_trj_info* __restrict__ info,
                                                       const double* __restrict__ T64, long long ldI,
                                                       const int* __restrict__ fpList,
@@ -1780,7 +1787,7 @@ __global__ void __launch_bounds__(256) k_sr_fp64_sums(const srwd_item* __restric
         if (q < count) {
             const int entry = fpList[q];
             const int blk = entry >> 8, thr = entry & 255;
-            const srwd_item& IT = items[blockItem[blk]];
+            const srwd_item& IT = items[blockItem ? blockItem[blk] : blk / nbU];
             const int local = (blk - IT.blockBase) * 256 + thr;
             const int traj = IT.traj;
             int ix = local % IT.nxc, iz = IT.iz0 + local / IT.nxc;
@@ -1812,14 +1819,14 @@ __global__ void __launch_bounds__(256) k_sr_fp64_sums(const srwd_item* __restric
 // k_edge_blocks: per block of SRWD_EDGE_BLOCK points and edge, the last
 // accepted point of the block (-1: none).
 __global__ void __launch_bounds__(SRWD_EDGE_BLOCK) k_edge_blocks(const srwd_req* __restrict__ reqs,
-                                                                 const int* __restrict__ blkReq,
+                                                                 const int* __restrict__ blkReq, int nbU,
                                                                  const srwd_trj_info* __restrict__ info,
                                                                  const srwd_edge* __restrict__ edges,
                                                                  const double* __restrict__ coord, int termin,
                                                                  long long* last)
 {
     const long long b = blockIdx.x;
-    const int r = blkReq[b];
+    const int r = blkReq ? blkReq[b] : (int)(b / nbU);
     const srwd_req Rq = reqs[r];
     const srwd_trj_info& I = info[r];
     const long long q = (b - Rq.blk0) * SRWD_EDGE_BLOCK + threadIdx.x;
@@ -1978,15 +1985,15 @@ int srwd_launch_sr_fused(const srwd_item* dItems, const int2* dBlocks, int nBloc
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int srwd_launch_finalize(const srwd_item* dItems, const int2* dEntries, int nEntries, int g,
+int srwd_launch_finalize(const srwd_item* dItems, const int2* dEntries, int nbU, int nEntries, int g,
                          const srwd_trj_info* dInfo, const srwd_edge* dEdge, int termin, const double* dPart,
                          int nSplit, long long nPointsPad, float* dEx, float* dEz, int* dWarn, const double* dCond,
                          double condTol, int* dFpList, int* dFpCount, const srwd_req* dReq, const double* dCoord,
                          const long long* dLast, hipStream_t st)
 {
     if (nEntries <= 0) return 0;
-    if (g < 1 || 256 % g) return -1;
-    hipLaunchKernelGGL(k_sr_finalize, dim3((unsigned)nEntries * g), dim3(256), 0, st, dItems, dEntries, g, dInfo,
+    if (g < 1 || 256 % g || (!dEntries && (nbU < 1 || g != 1))) return -1;
+    hipLaunchKernelGGL(k_sr_finalize, dim3((unsigned)nEntries * g), dim3(256), 0, st, dItems, dEntries, nbU, g, dInfo,
                        dEdge, termin, dPart, nSplit, nPointsPad, (float2*)dEx, (float2*)dEz, dWarn, dCond, condTol,
                        dFpList, dFpCount, dReq, dCoord, dLast);
     return hipGetLastError() == hipSuccess ? 0 : -1;
@@ -2000,27 +2007,27 @@ int srwd_launch_cond_sums(const srwd_trj_info* dInfo, int nTraj, const srwd_rec*
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int srwd_launch_sr_fp64(const srwd_item* dItems, const int* dBlockItem, const srwd_trj_info* dInfo,
+int srwd_launch_sr_fp64(const srwd_item* dItems, const int* dBlockItem, int nbU, const srwd_trj_info* dInfo,
                         const srwd_edge* dEdge, int termin, const double* dT64, long long ldI, float* dEx,
                         float* dEz, int* dWarn, const int* dFpList, const int* dFpCount, const srwd_req* dReq,
                         const double* dCoord, const long long* dLast, double* dSums, srwd_patch* dPatch,
                         int* dPatchCount, int patchCap, hipStream_t st)
 {
     if (dSums)
-        hipLaunchKernelGGL(k_sr_fp64_sums, dim3(2048), dim3(256), 0, st, dItems, dBlockItem, dInfo, dT64, ldI, dFpList,
+        hipLaunchKernelGGL(k_sr_fp64_sums, dim3(2048), dim3(256), 0, st, dItems, dBlockItem, nbU, dInfo, dT64, ldI, dFpList,
                            dFpCount, dReq, dCoord, dSums);
-    hipLaunchKernelGGL(k_sr_fp64, dim3(2048), dim3(256), 0, st, dItems, dBlockItem, dInfo, dEdge, termin, dT64, ldI,
+    hipLaunchKernelGGL(k_sr_fp64, dim3(2048), dim3(256), 0, st, dItems, dBlockItem, nbU, dInfo, dEdge, termin, dT64, ldI,
                        (float2*)dEx, (float2*)dEz, dWarn, dFpList, dFpCount, dReq, dCoord, dLast,
                        (const double*)dSums, dPatch, dPatchCount, patchCap);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int srwd_launch_edge_state(const srwd_req* dReq, int nReq, const int* dBlkReq, long long nBlk,
+int srwd_launch_edge_state(const srwd_req* dReq, int nReq, const int* dBlkReq, int nbU, long long nBlk,
                            const srwd_trj_info* dInfo, const srwd_edge* dEdge, const double* dCoord, int termin,
                            long long* dLast, hipStream_t st)
 {
     if (nBlk <= 0 || nReq <= 0) return 0;
-    hipLaunchKernelGGL(k_edge_blocks, dim3((unsigned)nBlk), dim3(SRWD_EDGE_BLOCK), 0, st, dReq, dBlkReq, dInfo, dEdge,
+    hipLaunchKernelGGL(k_edge_blocks, dim3((unsigned)nBlk), dim3(SRWD_EDGE_BLOCK), 0, st, dReq, dBlkReq, nbU, dInfo, dEdge,
                        dCoord, termin, dLast);
     hipLaunchKernelGGL(k_edge_scan, dim3(nReq), dim3(256), 0, st, dReq, dLast);
     return hipGetLastError() == hipSuccess ? 0 : -1;
