@@ -107,6 +107,48 @@ __global__ void __launch_bounds__(256) k_accum_interp(const float* __restrict__ 
     S2[r] += s2;
 }
 
+// Sums of the error estimate over the result mesh: a1 = sum S1^2, a2 = sum S2
+// and, with replicates, v = sum over points and replicates of (Srep_k / nPer -
+// S1 / n)^2; block partials first, then one block (out[3]).  Read back and
+// summed on the host, the replicates of a 512 x 512 mesh (33 MB) took 10 ms.
+#define SRWM_ERR_BLOCKS ((SRWM_ERR_WORK - 3) / 3)
+__device__ __forceinline__ void block_sum3(double* v)
+{
+    __shared__ double sh[4][3];
+    for (int k = 0; k < 3; k++) {
+        for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
+        if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][k] = v[k];
+    }
+    __syncthreads();
+    for (int k = 0; k < 3; k++) v[k] = sh[0][k] + sh[1][k] + sh[2][k] + sh[3][k];
+}
+
+__global__ void __launch_bounds__(256) k_err_partial(const double* __restrict__ S1, const double* __restrict__ S2,
+                                                     const double* __restrict__ Srep, int R, double invN, double invPer,
+                                                     long long nr, double* part)
+{
+    double v[3] = {0., 0., 0.};
+    for (long long r = (long long)blockIdx.x * 256 + threadIdx.x; r < nr; r += 256LL * SRWM_ERR_BLOCKS) {
+        v[0] += S1[r] * S1[r];
+        v[1] += S2[r];
+        if (Srep) {
+            const double m = S1[r] * invN;
+            for (int k = 0; k < R; k++) { const double d = Srep[k * nr + r] * invPer - m; v[2] += d * d; }
+        }
+    }
+    block_sum3(v);
+    if (threadIdx.x < 3) part[3 * blockIdx.x + threadIdx.x] = v[threadIdx.x];
+}
+
+__global__ void __launch_bounds__(256) k_err_total(const double* __restrict__ part, double* out)
+{
+    double v[3] = {0., 0., 0.};
+    for (int b = threadIdx.x; b < SRWM_ERR_BLOCKS; b += 256)
+        for (int k = 0; k < 3; k++) v[k] += part[3 * b + k];
+    block_sum3(v);
+    if (threadIdx.x < 3) out[threadIdx.x] = v[threadIdx.x];
+}
+
 __global__ void k_stokes_out(const double* __restrict__ S1, double scale, long long n, float* out)
 {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -124,6 +166,15 @@ int srwm_launch_accum(const float* I, long long iStride, const srwm_emesh* em, c
     if (Srep && (perRep <= 0 || nb % perRep != 0)) return -1;
     hipLaunchKernelGGL(k_accum_interp, dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, st, I, iStride, em, w, nb,
                        rm, S1, S2, norm2, Srep, perRep);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int srwm_launch_err_sums(const double* S1, const double* S2, const double* Srep, int R, double n, long long nr,
+                         double* work, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_err_partial, dim3(SRWM_ERR_BLOCKS), dim3(256), 0, st, S1, S2, Srep, R, 1. / n, (double)R / n, nr,
+                       work + 3);
+    hipLaunchKernelGGL(k_err_total, dim3(1), dim3(256), 0, st, work + 3, work);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

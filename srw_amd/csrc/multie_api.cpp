@@ -324,7 +324,6 @@ SRWL_EXPORT int srwlEmitPropMultiE(SRWLStokes* pStokes, SRWLWfr* pWfr0, SRWLMagF
         if (!dSrep) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
         HIPCHK(hipMemsetAsync(dSrep, 0, sizeof(double) * R * nr, st));
     }
-    std::vector<double> Srh;
     // arPar[5] > 0: also estimate the gain of the variance-optimal proposal
     // q* ~ p ||I|| for this estimator from the electrons drawn (plain runs)
     int diag = (arPar && arPar[5] > 0 && !useQ) ? 1 : 0;
@@ -379,7 +378,9 @@ SRWL_EXPORT int srwlEmitPropMultiE(SRWLStokes* pStokes, SRWLWfr* pWfr0, SRWLMagF
     long long done = 0;
     double sumW = 0, sumW2 = 0;
     double errEst = -1, lastA1 = 0;
-    std::vector<double> S1h, S2h;
+    double* dErr = (double*)Bf.Err.get(sizeof(double) * SRWM_ERR_WORK);
+    if (!dErr) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+    std::vector<std::vector<srwo_elem>> elems(nDrift);   // per pointwise element of the beamline
     while (done < nMacroElec) {
         long long nb = std::min<long long>(B, nMacroElec - done);
         if (rqmc) nb = (nb / R) * R;
@@ -506,6 +507,8 @@ SRWL_EXPORT int srwlEmitPropMultiE(SRWLStokes* pStokes, SRWLWfr* pWfr0, SRWLMagF
             OneCtx* m = (OneCtx*)c;
             return wfr_moments(*m->w, m->d, m->d + m->nxy, 0, 1, m->nx, m->mx, m->mz);
         };
+        srwo_elem* dElem = nDrift ? (srwo_elem*)Bf.Elem.get(sizeof(srwo_elem) * (size_t)nDrift * nb) : nullptr;
+        if (nDrift && !dElem) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
         for (int d = 0; d < nDrift; d++) {
             if (!isDrift[d]) {
                 // thin lens / aperture / obstacle on each electron's own mesh
@@ -517,8 +520,10 @@ SRWL_EXPORT int srwlEmitPropMultiE(SRWLStokes* pStokes, SRWLWfr* pWfr0, SRWLMagF
                 const bool lens = std::strcmp(ty, "lens") == 0;
                 const SRWLOptL* L = (const SRWLOptL*)pOpt->arOpt[d];
                 const SRWLOptA* A = (const SRWLOptA*)pOpt->arOpt[d];
+                std::vector<srwo_elem>& els = elems[d];
+                els.assign(nb, srwo_elem{});
                 for (long long j = 0; j < nb; j++) {
-                    srwo_elem E{};
+                    srwo_elem& E = els[j];
                     E.nx = nx; E.xStart = em[j].xStart; E.xStep = em[j].xStep; E.zStart = em[j].zStart;
                     E.zStep = em[j].zStep; E.eStart = pWfr0->mesh.eStart; E.eStep = 0.;
                     if (lens) {
@@ -531,7 +536,6 @@ SRWL_EXPORT int srwlEmitPropMultiE(SRWLStokes* pStokes, SRWLWfr* pWfr0, SRWLMagF
                         E.kind = circ ? (ob ? 4 : 3) : (ob ? 2 : 1);
                         E.p0 = A->Dx; E.p1 = A->Dy; E.cx = A->x; E.cy = A->y;
                     }
-                    if (srwo_launch_point_elem((float2*)dF + 2 * j * nxy, nxy, 1, E, st)) return SRWL_AMD_ERR_GPU;
                     if (lens) {
                         const double difX = (L->Fx == ws[j].Rx) ? 1E-23 : L->Fx - ws[j].Rx;
                         const double difZ = (L->Fy == ws[j].Ry) ? 1E-23 : L->Fy - ws[j].Ry;
@@ -546,6 +550,9 @@ SRWL_EXPORT int srwlEmitPropMultiE(SRWLStokes* pStokes, SRWLWfr* pWfr0, SRWLMagF
                     if (ws[j].Rx != 0 && ws[j].dRx == 0) ws[j].dRx = std::fabs(0.1 * ws[j].Rx);
                     if (ws[j].Ry != 0 && ws[j].dRy == 0) ws[j].dRy = std::fabs(0.1 * ws[j].Ry);
                 }
+                srwo_elem* dE = dElem + (size_t)d * nb;
+                HIPCHK(hipMemcpyAsync(dE, els.data(), sizeof(srwo_elem) * nb, hipMemcpyHostToDevice, st));
+                if (srwo_launch_point_elems((float2*)dF, nxy, (int)nb, dE, st)) return SRWL_AMD_ERR_GPU;
                 momValid = false;
                 continue;
             }
@@ -666,27 +673,15 @@ SRWL_EXPORT int srwlEmitPropMultiE(SRWLStokes* pStokes, SRWLWfr* pWfr0, SRWLMagF
         }
         done += nb;
         if (target > 0 || done == nMacroElec) {
-            S1h.resize(nr); S2h.resize(nr);
-            HIPCHK(hipMemcpyAsync(S1h.data(), dS, sizeof(double) * nr, hipMemcpyDeviceToHost, st));
-            HIPCHK(hipMemcpyAsync(S2h.data(), dS + nr, sizeof(double) * nr, hipMemcpyDeviceToHost, st));
+            const double N = (double)done;
+            double es[3];
+            if (srwm_launch_err_sums(dS, dS + nr, dSrep, R, N, nr, dErr, st)) return SRWL_AMD_ERR_GPU;
+            HIPCHK(hipMemcpyAsync(es, dErr, sizeof(es), hipMemcpyDeviceToHost, st));
             HIPCHK(hipStreamSynchronize(st));
-            double a1 = 0, a2 = 0;
-            for (long long r = 0; r < nr; r++) { a1 += S1h[r] * S1h[r]; a2 += S2h[r]; }
-            double N = (double)done;
+            const double a1 = es[0], a2 = es[1];
             errEst = (done > 1 && a1 > 0) ? std::sqrt(std::max(0., N * (a2 - a1 / N) / ((N - 1.) * a1))) : -1;
-            if (rqmc) {
-                // variance of the mean from the R replicate means (each of done / R points)
-                Srh.resize((size_t)R * nr);
-                HIPCHK(hipMemcpyAsync(Srh.data(), dSrep, sizeof(double) * R * nr, hipMemcpyDeviceToHost, st));
-                HIPCHK(hipStreamSynchronize(st));
-                double nPer = N / R, v = 0.;
-                for (long long q = 0; q < nr; q++) {
-                    double m = S1h[q] / N, d2 = 0.;
-                    for (int k = 0; k < R; k++) { double d = Srh[(size_t)k * nr + q] / nPer - m; d2 += d * d; }
-                    v += d2 / ((double)R * (R - 1));
-                }
-                errEst = a1 > 0 ? std::sqrt(v * N * N / a1) : -1;
-            }
+            // variance of the mean from the R replicate means (each of done / R points)
+            if (rqmc) errEst = a1 > 0 ? std::sqrt(es[2] / ((double)R * (R - 1)) * N * N / a1) : -1;
             lastA1 = a1;
             if (target > 0 && errEst > 0 && errEst <= target) break;
         }

@@ -35,11 +35,9 @@ __device__ __forceinline__ void cos_sin_opt(double x, float& c, float& s)
     s = neg ? -ss : ss;
 }
 
-__global__ void __launch_bounds__(256) k_point_elem(float2* d, long long nxy, int ne, srwo_elem E)
+// Element E on point p of photon energy ie of the slices d.
+__device__ __forceinline__ void point_elem(float2* d, long long nxy, long long p, int ie, const srwo_elem& E)
 {
-    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int ie = blockIdx.y;
-    if (p >= nxy || ie >= ne) return;
     const long long iz = p / E.nx, ix = p - iz * E.nx;
     const double xr = E.xStart + ix * E.xStep - E.cx, zr = E.zStart + iz * E.zStep - E.cy;
     float2* a = d + (2LL * ie) * nxy + p;
@@ -65,7 +63,33 @@ __global__ void __launch_bounds__(256) k_point_elem(float2* d, long long nxy, in
     if (zero) { *a = make_float2(0.f, 0.f); *b = make_float2(0.f, 0.f); }
 }
 
+__global__ void __launch_bounds__(256) k_point_elem(float2* d, long long nxy, int ne, srwo_elem E)
+{
+    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < nxy && (int)blockIdx.y < ne) point_elem(d, nxy, p, blockIdx.y, E);
+}
+
+// One element per wavefront of a batch of single-energy wavefronts (slices 2 j
+// and 2 j + 1 of wavefront j), in one launch: one launch per wavefront cost 2.5
+// us each, 0.64 of the 2.5 ms that 128 electrons on 64 x 64 points take.
+__global__ void __launch_bounds__(256) k_point_elems(float2* d, long long nxy, const srwo_elem* __restrict__ E)
+{
+    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < nxy) point_elem(d + 2LL * blockIdx.y * nxy, nxy, p, 0, E[blockIdx.y]);
+}
+
 }  // namespace
+
+extern "C" int srwo_launch_point_elems(float2* d, long long nxy, int n, const srwo_elem* dE, hipStream_t st)
+{
+    if (nxy <= 0 || n <= 0) return -1;
+    for (int j = 0; j < n; j += 65535) {
+        const int m = n - j < 65535 ? n - j : 65535;
+        hipLaunchKernelGGL(k_point_elems, dim3((unsigned)((nxy + 255) / 256), (unsigned)m), dim3(256), 0, st,
+                           d + 2LL * j * nxy, nxy, dE + j);
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
 
 extern "C" int srwo_launch_point_elem(float2* d, long long nxy, int ne, const srwo_elem& E, hipStream_t st)
 {

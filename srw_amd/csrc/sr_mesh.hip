@@ -142,14 +142,14 @@ __device__ __forceinline__ void mesh_cmac(const mesh_op& A, const mesh_op& B, fl
     im = mfma(A.ih, B.rh, im);
 }
 
-__global__ void __launch_bounds__(256, 2) k_sr_mesh(const srwd_item* __restrict__ items, const int2* __restrict__ tiles,
+__global__ void __launch_bounds__(256, 2) k_sr_mesh(const srwd_item* __restrict__ items, const int2* __restrict__ tiles, int ntU,
                                                     const srwd_trj_info* __restrict__ info,
                                                     const srwd_mrec* __restrict__ rec, long long ldM,
                                                     const double* __restrict__ scale, int nSplit, long long nPointsPad,
                                                     double* __restrict__ part)
 {
     __shared__ uint4v lds[2 * MESH_BUF];
-    const int2 tl = tiles[blockIdx.x];
+    const int2 tl = tiles ? tiles[blockIdx.x] : make_int2(blockIdx.x / ntU, blockIdx.x % ntU);
     const srwd_item& IT = items[tl.x];
     const int nxc = IT.nxc, nzr = IT.npts / nxc;
     const int nTx = (nxc + SRWD_MESH_TILE - 1) / SRWD_MESH_TILE;
@@ -231,12 +231,12 @@ __global__ void __launch_bounds__(256, 2) k_sr_mesh(const srwd_item* __restrict_
     }
 }
 
-extern "C" int srwd_launch_sr_mesh(const srwd_item* dItems, const int2* dTiles, int nTiles, const srwd_trj_info* dInfo,
+extern "C" int srwd_launch_sr_mesh(const srwd_item* dItems, const int2* dTiles, int ntU, int nTiles, const srwd_trj_info* dInfo,
                                    const srwd_mrec* dRec, long long ldM, const double* dScale, int nSplit,
                                    long long nPointsPad, double* dPart, hipStream_t st)
 {
     if (nTiles <= 0) return 0;
-    hipLaunchKernelGGL(k_sr_mesh, dim3(nTiles, nSplit), dim3(256), 0, st, dItems, dTiles, dInfo, dRec, ldM, dScale, nSplit,
+    hipLaunchKernelGGL(k_sr_mesh, dim3(nTiles, nSplit), dim3(256), 0, st, dItems, dTiles, ntU, dInfo, dRec, ldM, dScale, nSplit,
                        nPointsPad, dPart);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }

@@ -55,6 +55,7 @@ struct Buffers {
     DBuf Ex, Ez;                  // field outputs
     DBuf W0, W1, W2, W3;          // propagation / accumulation work buffers
     DBuf Stokes, Draws, Wt, Net, Grad, Rep;
+    DBuf Elem, Err;               // multi-electron: pointwise elements per electron, error estimate sums
     DBuf Pic;                     // parallel-in-s RK4 iterates
     DBuf MomSl, MomWork, MomSums, MomLims;   // wavefront moments
     DBuf RsO, RsN;                // resampling

@@ -221,12 +221,15 @@ int srwd_launch_sr_fused(const srwd_item* dItems, const int2* dBlocks, int nBloc
                          const srwd_trj_info* dInfo, const srwd_rec* dRec, const srwd_chunk* dChunk, const float* dA,
                          long long ldI, long long ldC, long long nPointsPad, double* dPart, const srwd_fuse& F,
                          hipStream_t st);
+// In the launches below a list may be nullptr where every request (item) has
+// the same number nbU of blocks (ntU of tiles): entry i is then block i % nbU of
+// request (item) i / nbU.
 // The sums of mesh items (sr_mesh.hip) over a list of tiles of
 // SRWD_MESH_TILE x SRWD_MESH_TILE points: dTiles[i] = {item, tile} with the
 // tiles of an item numbered along x, then z.  dRec: the two
 // sides of every trajectory, ldM groups each (srwd_mesh_ld of the longest);
 // dScale: the inverse amplitude scales of the two sides, 2 per trajectory.
-int srwd_launch_sr_mesh(const srwd_item* dItems, const int2* dTiles, int nTiles, const srwd_trj_info* dInfo,
+int srwd_launch_sr_mesh(const srwd_item* dItems, const int2* dTiles, int ntU, int nTiles, const srwd_trj_info* dInfo,
                         const srwd_mrec* dRec, long long ldM, const double* dScale, int nSplit, long long nPointsPad,
                         double* dPart, hipStream_t st);
 // Edge-derivative state of the reference's point loop: per block of
@@ -234,7 +237,7 @@ int srwd_launch_sr_mesh(const srwd_item* dItems, const int2* dTiles, int nTiles,
 // last point at or before the block's end whose far-field expansion at that
 // edge is accepted (request-local index; -1: none).  dLast holds 2 values per
 // block.
-int srwd_launch_edge_state(const srwd_req* dReq, int nReq, const int* dBlkReq, long long nBlk,
+int srwd_launch_edge_state(const srwd_req* dReq, int nReq, const int* dBlkReq, int nbU, long long nBlk,
                            const srwd_trj_info* dInfo, const srwd_edge* dEdge, const double* dCoord, int termin,
                            long long* dLast, hipStream_t st);
 // Entries (first item, 256-point block in the item) of groups of g items
@@ -245,7 +248,7 @@ int srwd_launch_edge_state(const srwd_req* dReq, int nReq, const int* dBlkReq, l
 // dFpList (item's band-relative block * 256 + point in the block;
 // *dFpCount entries, zeroed by the caller) instead of being stored, for
 // srwd_launch_sr_fp64.  dCond == nullptr stores every point.
-int srwd_launch_finalize(const srwd_item* dItems, const int2* dEntries, int nEntries, int g,
+int srwd_launch_finalize(const srwd_item* dItems, const int2* dEntries, int nbU, int nEntries, int g,
                          const srwd_trj_info* dInfo, const srwd_edge* dEdge, int termin, const double* dPart,
                          int nSplit, long long nPointsPad, float* dEx, float* dEz, int* dWarn, const double* dCond,
                          double condTol, int* dFpList, int* dFpCount, const srwd_req* dReq, const double* dCoord,
@@ -265,7 +268,7 @@ int srwd_launch_cond_sums(const srwd_trj_info* dInfo, int nTraj, const srwd_rec*
 // dPatch (optional, capacity patchCap): every store is also recorded there
 // (*dPatchCount counts them, zeroed by the caller, and may exceed the
 // capacity: then the records past it are dropped).
-int srwd_launch_sr_fp64(const srwd_item* dItems, const int* dBlockItem, const srwd_trj_info* dInfo,
+int srwd_launch_sr_fp64(const srwd_item* dItems, const int* dBlockItem, int nbU, const srwd_trj_info* dInfo,
                         const srwd_edge* dEdge, int termin, const double* dT64, long long ldI, float* dEx,
                         float* dEz, int* dWarn, const int* dFpList, const int* dFpCount, const srwd_req* dReq,
                         const double* dCoord, const long long* dLast, double* dSums, srwd_patch* dPatch,

@@ -21,5 +21,12 @@ extern "C" {
 int srwm_launch_accum(const float* I, long long iStride, const srwm_emesh* em, const float* w, int nb,
                       srwm_rmesh rm, double* S1, double* S2, double* norm2, double* Srep, int perRep,
                       hipStream_t st);
+// Sums of the error estimate after n electrons: out[0] = sum S1^2, out[1] = sum
+// S2, out[2] = the squared deviations of the R replicate means from the mean
+// over points and replicates (0 when Srep is nullptr), in work[0..2]; work
+// holds SRWM_ERR_WORK doubles.
+#define SRWM_ERR_WORK (3 + 3 * 512)
+int srwm_launch_err_sums(const double* S1, const double* S2, const double* Srep, int R, double n, long long nr,
+                         double* work, hipStream_t st);
 int srwm_launch_stokes_out(const double* S1, double scale, long long n, float* out, hipStream_t st);
 }

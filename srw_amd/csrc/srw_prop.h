@@ -48,6 +48,9 @@ struct srwo_elem {
 
 extern "C" {
 int srwo_launch_point_elem(float2* d, long long nxy, int ne, const srwo_elem& E, hipStream_t st);
+// The same for n single-energy wavefronts side by side, element dE[j] (device
+// memory) on wavefront j.
+int srwo_launch_point_elems(float2* d, long long nxy, int n, const srwo_elem* dE, hipStream_t st);
 // rows: ne * nz doubles of scratch for the flux (what == 4)
 int srwx_launch_extract(const float2* ex, const float2* ez, const srwx_extract& P, void* out, double* rows,
                         hipStream_t st);

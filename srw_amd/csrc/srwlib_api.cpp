@@ -213,8 +213,8 @@ struct UpBlob {
     size_t add(const void* src, size_t bytes)
     {
         const size_t at = (h.size() + 255) & ~(size_t)255;
-        h.resize(at + bytes);
-        if (bytes) std::memcpy(h.data() + at, src, bytes);
+        h.resize(at);
+        h.insert(h.end(), (const char*)src, (const char*)src + bytes);
         return at;
     }
     template <typename T> size_t add(const std::vector<T>& v) { return add(v.data(), sizeof(T) * v.size()); }
@@ -435,7 +435,9 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     // sums of the steps, srradint.cpp:342-388) and the edge-derivative state.
     std::vector<srwd_req> reqs(nT);
     std::vector<double> coord;
-    std::vector<int> blkReq;
+    std::vector<int> blkReq;      // request of each edge-state block, unless every request has nbEdge of them
+    long long nEdgeBlk = 0;
+    int nbEdge = 0;
     for (int j = 0; j < nT; j++) {
         const SRWLRadMesh& m = jobs[j].mesh;
         SrRegion G = sr_region(m, info[j]);
@@ -443,23 +445,36 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         std::memset(&R, 0, sizeof(R));
         R.nxc = G.nxc; R.nzc = G.nzc; R.ne = (int)m.ne;
         R.nPts = (long long)G.nzc * G.nxc * m.ne;
-        R.blk0 = (long long)blkReq.size();
-        R.xOff = (int)coord.size();
-        double v = m.xStart;
-        for (int ix = 0; ix < G.nxc; ix++) { coord.push_back(v); v += G.xStep; }
-        R.zOff = (int)coord.size();
-        v = m.yStart;
-        for (int iz = 0; iz < G.nzc; iz++) { coord.push_back(v); v += G.zStep; }
-        R.eOff = (int)coord.size();
-        double eStep = m.ne > 1 ? (m.eFin - m.eStart) / (m.ne - 1) : 0;
-        v = m.eStart;
-        for (int ie = 0; ie < (int)m.ne; ie++) { coord.push_back(v); v += eStep; }
+        R.blk0 = nEdgeBlk;
+        // requests on one and the same mesh (a partially coherent sum) share
+        // their coordinates
+        if (j > 0 && std::memcmp(&jobs[j].mesh, &jobs[j - 1].mesh, sizeof(SRWLRadMesh)) == 0 &&
+            reqs[j - 1].nxc == G.nxc && reqs[j - 1].nzc == G.nzc) {
+            R.xOff = reqs[j - 1].xOff; R.zOff = reqs[j - 1].zOff; R.eOff = reqs[j - 1].eOff;
+        } else {
+            R.xOff = (int)coord.size();
+            double v = m.xStart;
+            for (int ix = 0; ix < G.nxc; ix++) { coord.push_back(v); v += G.xStep; }
+            R.zOff = (int)coord.size();
+            v = m.yStart;
+            for (int iz = 0; iz < G.nzc; iz++) { coord.push_back(v); v += G.zStep; }
+            R.eOff = (int)coord.size();
+            double eStep = m.ne > 1 ? (m.eFin - m.eStart) / (m.ne - 1) : 0;
+            v = m.eStart;
+            for (int ie = 0; ie < (int)m.ne; ie++) { coord.push_back(v); v += eStep; }
+        }
         if (termin > 0) {
-            long long nb = (R.nPts + SRWD_EDGE_BLOCK - 1) / SRWD_EDGE_BLOCK;
-            blkReq.insert(blkReq.end(), (size_t)nb, j);
+            const long long nb = (R.nPts + SRWD_EDGE_BLOCK - 1) / SRWD_EDGE_BLOCK;
+            nEdgeBlk += nb;
+            if (j == 0) nbEdge = (int)nb;
+            else if (nb != nbEdge) nbEdge = -1;
         }
     }
-    long long nEdgeBlk = (long long)blkReq.size();
+    if (nbEdge < 0) {
+        nbEdge = 0;
+        for (int j = 0; j < nT; j++)
+            blkReq.insert(blkReq.end(), (size_t)((reqs[j].nPts + SRWD_EDGE_BLOCK - 1) / SRWD_EDGE_BLOCK), j);
+    }
     long long* dLast = nEdgeBlk ? (long long*)B.Last.get(sizeof(long long) * 2 * (size_t)nEdgeBlk) : nullptr;
     if (nEdgeBlk && !dLast) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
     UpBlob us;
@@ -474,7 +489,8 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         dReq = (srwd_req*)(dUs + oReq);
         dCoord = (double*)(dUs + oCoord);
         if (int e_ = h2d(dUs, us.h.data(), us.h.size(), st)) return e_;
-        if (nEdgeBlk && srwd_launch_edge_state(dReq, nT, (const int*)(dUs + oBlkReq), nEdgeBlk, dInfo, dEdge, dCoord,
+        if (nEdgeBlk && srwd_launch_edge_state(dReq, nT, blkReq.empty() ? nullptr : (const int*)(dUs + oBlkReq),
+                                               nbEdge, nEdgeBlk, dInfo, dEdge, dCoord,
                                                termin, dLast, st))
             return SRWL_AMD_ERR_GPU;
         return 0;
@@ -566,8 +582,21 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             nBands = 1;
         }
     }
+    // mesh requests of one energy and one size (a partially coherent sum):
+    // every item has nbU blocks and ntU tiles, and no list is needed
+    int nbU = 0, ntU = 0;
+    if (allMesh && nBands == 1 && !nDl) {
+        bool same = true;
+        for (int j = 0; j < nT; j++)
+            same = same && jobs[j].mesh.ne == 1 && reqs[j].nxc == reqs[0].nxc && reqs[j].nzc == reqs[0].nzc;
+        if (same) {
+            nbU = (reqs[0].nxc * reqs[0].nzc + 255) / 256;
+            ntU = mesh_tiles(reqs[0].nxc, reqs[0].nzc);
+        }
+    }
     std::vector<srwd_item> items;
     std::vector<int> blockItem;
+    int nBlocks = 0;
     std::vector<int> bandBlock0(nBands + 1, 0), bandRow0(nBands + 1, 0);
     // finalize lists: {item, block of the item}; tile blocks name the first
     // item of a group of SRWD_TILE_E energies.  The sums have lists of their
@@ -579,7 +608,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         bandMesh0[b] = (int)meshTiles.size();
         bandSrTile0[b] = (int)srTileBlocks.size();
         bandSrRest0[b] = (int)srRestBlocks.size();
-        bandBlock0[b] = (int)blockItem.size();
+        bandBlock0[b] = nBlocks;
         bandTile0[b] = (int)tileBlocks.size();
         bandRest0[b] = (int)restBlocks.size();
         for (int j = 0; j < nT; j++) {
@@ -613,14 +642,17 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
                 it.ne = ne; it.ie = ie;
                 it.outOffset = outOff[j] + ie;
                 it.npts = G.nxc * (r1 - r0);
-                it.blockBase = (int)blockItem.size() - bandBlock0[b];   // relative to the band's first block
-                it.pointBase = (long long)blockItem.size() * 256;
+                it.blockBase = nBlocks - bandBlock0[b];   // relative to the band's first block
+                it.pointBase = (long long)nBlocks * 256;
                 it.actNorm = normConst * it.eph * 0.80654658E-03;
                 it.drow = dRowOf[j];
                 it.de = eStepOf[j];
                 it.tiled = isMesh[j] ? SRWD_ITEM_MESH : (ie < nTiled ? SRWD_ITEM_TILE : SRWD_ITEM_POINT);
                 int nb = (it.npts + 255) / 256;
                 const int me = (int)items.size();
+                nBlocks += nb;
+                items.push_back(it);
+                if (nbU) continue;
                 for (int q = 0; q < nb; q++) blockItem.push_back(me);
                 if (ie >= nTiled) for (int q = 0; q < nb; q++) restBlocks.push_back(make_int2(me, q));
                 else if (ie % tE == 0) for (int q = 0; q < nb; q++) tileBlocks.push_back(make_int2(me, q));
@@ -632,11 +664,10 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
                 } else if (ie % tE == 0) {
                     for (int q = 0; q < nb; q++) srTileBlocks.push_back(make_int2(me, q));
                 }
-                items.push_back(it);
             }
         }
     }
-    bandBlock0[nBands] = (int)blockItem.size();
+    bandBlock0[nBands] = nBlocks;
     bandTile0[nBands] = (int)tileBlocks.size();
     bandRest0[nBands] = (int)restBlocks.size();
     bandMesh0[nBands] = (int)meshTiles.size();
@@ -682,8 +713,8 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     }
     int nItems = (int)items.size();
     int nRows = (int)rowTraj.size();
-    int nBlocks = (int)blockItem.size();
     if (nBlocks == 0) return 0;
+    const int nMeshTiles = nbU ? nItems * ntU : (int)meshTiles.size();
     long long nPointsPad = (long long)nBlocks * 256;
     // split the integration range when a band's mesh alone does not fill the GPU
     long long minChunks = ldC;
@@ -698,7 +729,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     const int nWG = (int)(srTileBlocks.size() + srRestBlocks.size());
     int nSplit = 1;
     if (allMesh) {
-        nSplit = mesh_split((long long)meshTiles.size() / nBands, minUnits, nPointsPad / nBands);
+        nSplit = mesh_split((long long)nMeshTiles / nBands, minUnits, nPointsPad / nBands);
         // a no-allocation call keeps its partial sums within what one block
         // per 256 points would take
         if (g_arena) nSplit = std::min(nSplit, std::max(1, 4096 / nBlocks));
@@ -727,7 +758,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     rc = upload_requests();
     if (rc) return rc;
     srwd_item* dItems = (srwd_item*)(dUs + oItems);
-    int* dBlockItem = (int*)(dUs + oBlockItem);
+    const int* dBlockItem = nbU ? nullptr : (const int*)(dUs + oBlockItem);
     int* dWarn = (int*)(dUs + oCounts);
     int* dPatchCount = dWarn + 1;
     int* dFpCount = dWarn + 2;
@@ -834,15 +865,15 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             // download, so one launch forms them and the finalize pass runs
             // band by band, each band's copy queued behind it
             if (g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev0, st));
-            if (srwd_launch_sr_mesh(dItems, dMeshTiles, (int)meshTiles.size(), dInfo, dMrec, ldM, dScale, nSplit,
+            if (srwd_launch_sr_mesh(dItems, dMeshTiles, 0, (int)meshTiles.size(), dInfo, dMrec, ldM, dScale, nSplit,
                                     nPointsPad, dPart, st))
                 return SRWL_AMD_ERR_GPU;
             if (g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev1, st));
             for (int b = 0; b < nDl; b++) {
-                if (srwd_launch_finalize(dItems, dTileBlocks + dlTile0[b], dlTile0[b + 1] - dlTile0[b],
+                if (srwd_launch_finalize(dItems, dTileBlocks + dlTile0[b], 0, dlTile0[b + 1] - dlTile0[b],
                                          std::max(1, g_ctx.tileE), dInfo, dEdge, termin, dPart, nSplit, nPointsPad, dEx,
                                          dEz, dWarn, cnd, g_ctx.condTol, dFpList, dFpCount, dReq, dCoord, dLast, st) ||
-                    srwd_launch_finalize(dItems, dRestBlocks + dlRest0[b], dlRest0[b + 1] - dlRest0[b], 1, dInfo, dEdge,
+                    srwd_launch_finalize(dItems, dRestBlocks + dlRest0[b], 0, dlRest0[b + 1] - dlRest0[b], 1, dInfo, dEdge,
                                          termin, dPart, nSplit, nPointsPad, dEx, dEz, dWarn, cnd, g_ctx.condTol, dFpList,
                                          dFpCount, dReq, dCoord, dLast, st))
                     return SRWL_AMD_ERR_GPU;
@@ -858,7 +889,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         HIPCHK(hipStreamWaitEvent(g_ctx.stream2, g_ctx.evFork, 0));
         if (srwd_launch_sr(dItems, dSrRest, nRest, 0, dInfo, dRec, dChunk, dA, ldI, ldC, 1, nPointsPad, dPart,
                            g_ctx.stream2) ||
-            srwd_launch_finalize(dItems, dRestBlocks, nRest, 1, dInfo, dEdge, termin, dPart, 1, nPointsPad, dEx, dEz,
+            srwd_launch_finalize(dItems, dRestBlocks, 0, nRest, 1, dInfo, dEdge, termin, dPart, 1, nPointsPad, dEx, dEz,
                                  dWarn, cnd, g_ctx.condTol, dFpList, dFpCount, dReq, dCoord, dLast, g_ctx.stream2))
             return SRWL_AMD_ERR_GPU;
         HIPCHK(hipEventRecord(g_ctx.evJoin, g_ctx.stream2));
@@ -876,7 +907,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         }
         // FP64 recomputation, every store also recorded for the host
         if (g_ctx.condTol > 0 &&
-            srwd_launch_sr_fp64(dItems, dBlockItem, dInfo, dEdge, termin, dT64, ldI, dEx, dEz, dWarn, dFpList,
+            srwd_launch_sr_fp64(dItems, dBlockItem, 0, dInfo, dEdge, termin, dT64, ldI, dEx, dEz, dWarn, dFpList,
                                 dFpCount, dReq, dCoord, dLast, dPart, dPatch, dPatchCount, SRWL_AMD_PATCH_CAP, st))
             return SRWL_AMD_ERR_GPU;
         HIPCHK(hipMemcpyAsync(g_ctx.fpCountHost, dWarn, sizeof(int) * 3, hipMemcpyDeviceToHost, st));
@@ -979,8 +1010,8 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
                                nPointsPad, dPart, side ? g_ctx.stream2 : sb) ||
                 srwd_launch_sr(dItems, dSrTile + bandSrTile0[b], nSrTile, g_ctx.tileE, dInfo, dRec, dChunk, dA, ldI,
                                ldC, nSplit, nPointsPad, dPart, sb) ||
-                srwd_launch_sr_mesh(dItems, dMeshTiles + bandMesh0[b], bandMesh0[b + 1] - bandMesh0[b], dInfo, dMrec,
-                                    ldM, dScale, nSplit, nPointsPad, dPart, sb))
+                srwd_launch_sr_mesh(dItems, nbU ? nullptr : dMeshTiles + bandMesh0[b], ntU,
+                                    nbU ? nMeshTiles : bandMesh0[b + 1] - bandMesh0[b], dInfo, dMrec, ldM, dScale, nSplit, nPointsPad, dPart, sb))
                 return SRWL_AMD_ERR_GPU;
             if (side) {
                 HIPCHK(hipEventRecord(g_ctx.evJoin, g_ctx.stream2));
@@ -989,16 +1020,17 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             if (g_ctx.timing) HIPCHK(hipEventRecord(nBands > 1 ? g_ctx.bandEv[4 * b + 3] : g_ctx.ev1, sb));
             // energy tiles in groups (runs of consecutive photon energies stored together), then the rest
             const double* cnd = g_ctx.condTol > 0 ? dCond : nullptr;
-            if (srwd_launch_finalize(dItems, dTileBlocks + bandTile0[b], nTile, g_ctx.tileE > 0 ? g_ctx.tileE : 1,
+            if (srwd_launch_finalize(dItems, dTileBlocks + bandTile0[b], 0, nTile, g_ctx.tileE > 0 ? g_ctx.tileE : 1,
                                      dInfo, dEdge, termin, dPart, nSplit, nPointsPad, dEx, dEz, dWarn, cnd,
                                      g_ctx.condTol, fpList, dFpCount + b, dReq, dCoord, dLast, sb) ||
-                srwd_launch_finalize(dItems, dRestBlocks + bandRest0[b], nRest, 1, dInfo, dEdge, termin, dPart,
+                srwd_launch_finalize(dItems, nbU ? nullptr : dRestBlocks + bandRest0[b], nbU, nbU ? nBlocks : nRest, 1, dInfo, dEdge, termin, dPart,
                                      nSplit, nPointsPad, dEx, dEz, dWarn, cnd, g_ctx.condTol, fpList, dFpCount + b,
                                      dReq, dCoord, dLast, sb))
                 return SRWL_AMD_ERR_GPU;
             // a single band's partial sums are consumed by now: their buffer
             // (at least 4 doubles per point) holds the FP64 pass's sums
-            if (g_ctx.condTol > 0 && srwd_launch_sr_fp64(dItems, dBlockItem + b0, dInfo, dEdge, termin, dT64, ldI, dEx,
+            if (g_ctx.condTol > 0 && srwd_launch_sr_fp64(dItems, dBlockItem ? dBlockItem + b0 : nullptr, nbU, dInfo,
+                                                         dEdge, termin, dT64, ldI, dEx,
                                                          dEz, dWarn, fpList, dFpCount + b, dReq, dCoord, dLast,
                                                          nBands == 1 ? dPart : nullptr, nullptr, nullptr, 0, sb))
                 return SRWL_AMD_ERR_GPU;
