@@ -235,21 +235,34 @@ static int mesh_tiles(int nx, int nz)
 
 // Whether the sums of a request over nxc x nzc computed points go to the mesh
 // kernel.
-static bool mesh_kernel_pays(int nxc, int nzc, int ne)
+static bool mesh_kernel_pays(int nxc, int nzc)
 {
-    (void)ne;
     const long long T2 = SRWD_MESH_TILE * SRWD_MESH_TILE;
     return mesh_tiles(nxc, nzc) * T2 <= 4LL * nxc * nzc;
 }
 
-// Parts of the s-range of a mesh pass of nTiles tiles and nPts points.
-static int mesh_split(long long nTiles, long long nUnits, long long nPts)
+// Parts of the s-range of a mesh pass of nTiles tiles and nPts points: the least
+// of a model of its time.  512 workgroups are resident at once (two a CU, by
+// LDS) and such a round takes 3.7 us per unit of the s-range (512 x 512
+// points of 256 electrons: 32 rounds of 313 units in 37.4 ms); each part writes
+// and reads 32 bytes a point.  Measured, whole calls, parts 2 / 5 / 16: 101 x 101
+// x 101 energies (202 tiles) 1.38 / 1.28 / 1.36 ms; 1 / 13 / 24: 150 x 93 x 5
+// (30 tiles) 1.18 / 0.54 / 0.53 ms; 1 / 4 / 16: 128 electrons on 64 x 64 (128
+// tiles) 1.99 / 1.51 / 1.56 ms.
+// A large field, whose rows are streamed to the host, takes parts of about 24
+// units (0.1 ms) while its partial sums stay under 2 GB: the finalize pass of the rows already summed gets its places
+// as the next rows' workgroups leave, and short ones leave sooner.  201 x 201 x
+// 201, parts 1 / 5 / 13: 8.23 / 7.36 / 6.7 ms; 400 x 400 x 20: 3.80 / 3.12 /
+// 2.65 ms.
+static int mesh_split(long long nTiles, long long nUnits, long long nPts, bool large)
 {
+    if (large)
+        return (int)std::max(1LL, std::min((nUnits + 23) / 24, (1LL << 31) / (32 * std::max(1LL, nPts))));
     int best = 1;
     double bestT = 1e300;
-    for (long long n = 1; n <= std::min<long long>(nUnits, 128); n++) {
+    for (long long n = 1; n <= std::min<long long>(nUnits / 2, 128); n++) {
         const double rounds = (double)((std::max(1LL, nTiles) * n + 511) / 512);
-        const double t = rounds * (double)((nUnits + n - 1) / n) * 4e-6 + (double)n * nPts * 64. / 4e12;
+        const double t = rounds * (double)((nUnits + n - 1) / n) * 3.7e-6 + (double)n * nPts * 64. / 4e12;
         if (t < bestT * 0.98) { bestT = t; best = (int)n; }
     }
     return best;
@@ -533,7 +546,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     std::vector<char> isMesh(nT);
     bool allMesh = true;
     for (int j = 0; j < nT; j++) {
-        isMesh[j] = mesh_kernel_pays(reqs[j].nxc, reqs[j].nzc, (int)jobs[j].mesh.ne);
+        isMesh[j] = mesh_kernel_pays(reqs[j].nxc, reqs[j].nzc);
         allMesh = allMesh && isMesh[j];
     }
     for (int j = 0; j < nT; j++) {
@@ -557,11 +570,13 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         rowTraj.push_back(j); rowE.push_back(eStepOf[j]); rowN.push_back(info[j].nInt);
     }
     int nBands = 1;
+    bool large = false;   // one field of 16 MB or more for the caller's arrays
     if (hostOut && nT == 1 && !g_arena) {
         SrRegion G = sr_region(jobs[0].mesh, info[0]);
         const SRWLRadMesh& m = jobs[0].mesh;
         double outBytes = 16. * m.ne * m.nx * m.ny;
-        if (outBytes >= 16. * (1 << 20)) nBands = std::min(8, G.nzc);
+        large = outBytes >= 16. * (1 << 20);
+        if (large) nBands = std::min(8, G.nzc);
         if (g_ctx.forceBands > 0) nBands = std::min(g_ctx.forceBands, G.nzc);
     }
     // Streamed rows: instead of computing row bands one after another, one
@@ -681,6 +696,10 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         std::stable_sort(tileBlocks.begin(), tileBlocks.end(), byRow);
         std::stable_sort(restBlocks.begin(), restBlocks.end(), byRow);
         std::stable_sort(srTileBlocks.begin(), srTileBlocks.end(), byRow);
+        std::stable_sort(srRestBlocks.begin(), srRestBlocks.end(), byRow);
+        // mesh tiles by tile row, an item's tiles of one row together
+        const int nTx = (items[0].nxc + SRWD_MESH_TILE - 1) / SRWD_MESH_TILE;
+        std::stable_sort(meshTiles.begin(), meshTiles.end(), [nTx](int2 a, int2 b) { return a.y / nTx < b.y / nTx; });
         SrRegion G = sr_region(jobs[0].mesh, info[0]);
         dlRow0.resize(nDl + 1);
         for (int q = 0; q <= nDl; q++)
@@ -718,7 +737,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     long long nPointsPad = (long long)nBlocks * 256;
     // split the integration range when a band's mesh alone does not fill the GPU
     long long minChunks = ldC;
-    long long minUnits = ldM / SRWD_MESH_UNIT;
+    long long minUnits = 1LL << 40;
     for (auto& I : info) {
         minChunks = std::min(minChunks, (I.nInt + SRWD_CHUNK - 1) / SRWD_CHUNK);
         minUnits = std::min(minUnits, (I.nInt + SRWD_MESH_UNIT - 1) / SRWD_MESH_UNIT);
@@ -729,7 +748,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     const int nWG = (int)(srTileBlocks.size() + srRestBlocks.size());
     int nSplit = 1;
     if (allMesh) {
-        nSplit = mesh_split((long long)nMeshTiles / nBands, minUnits, nPointsPad / nBands);
+        nSplit = mesh_split((long long)nMeshTiles / nBands, minUnits, nPointsPad / nBands, large);
         // a no-allocation call keeps its partial sums within what one block
         // per 256 points would take
         if (g_arena) nSplit = std::min(nSplit, std::max(1, 4096 / nBlocks));
@@ -861,27 +880,46 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
             return 0;
         };
         if (!meshTiles.empty()) {
-            // mesh items: the sums of the whole field are short against its
-            // download, so one launch forms them and the finalize pass runs
-            // band by band, each band's copy queued behind it
+            // Mesh items: the sums in launches of whole tile rows (all
+            // energies), the finalize pass of the bands that a launch
+            // completes and their copies behind it on the second stream,
+            // beside the next launch.  A launch keeps at least two blocks per
+            // resident place, so that its last ones leave little idle.
+            const int nTx = (items[0].nxc + SRWD_MESH_TILE - 1) / SRWD_MESH_TILE;
+            const int nzc = items[0].iz0 + items[0].npts / items[0].nxc;
+            const int nRowTiles = nTx * nItems;
             if (g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev0, st));
-            if (srwd_launch_sr_mesh(dItems, dMeshTiles, 0, (int)meshTiles.size(), dInfo, dMrec, ldM, dScale, nSplit,
-                                    nPointsPad, dPart, st))
-                return SRWL_AMD_ERR_GPU;
-            if (g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev1, st));
-            for (int b = 0; b < nDl; b++) {
-                if (srwd_launch_finalize(dItems, dTileBlocks + dlTile0[b], 0, dlTile0[b + 1] - dlTile0[b],
-                                         std::max(1, g_ctx.tileE), dInfo, dEdge, termin, dPart, nSplit, nPointsPad, dEx,
-                                         dEz, dWarn, cnd, g_ctx.condTol, dFpList, dFpCount, dReq, dCoord, dLast, st) ||
-                    srwd_launch_finalize(dItems, dRestBlocks + dlRest0[b], 0, dlRest0[b + 1] - dlRest0[b], 1, dInfo, dEdge,
-                                         termin, dPart, nSplit, nPointsPad, dEx, dEz, dWarn, cnd, g_ctx.condTol, dFpList,
-                                         dFpCount, dReq, dCoord, dLast, st))
+            for (int b = 0, t0 = 0, nTot = (int)meshTiles.size(); t0 < nTot;) {
+                int t1 = t0 + nRowTiles;
+                while (t1 < nTot && (long long)(t1 - t0) * nSplit < 1024) t1 += nRowTiles;
+                if ((long long)(nTot - t1) * nSplit < 1024) t1 = nTot;
+                if (srwd_launch_sr_mesh(dItems, dMeshTiles + t0, 0, t1 - t0, dInfo, dMrec, ldM, dScale, nSplit,
+                                        nPointsPad, dPart, st))
                     return SRWL_AMD_ERR_GPU;
-                HIPCHK(hipEventRecord(g_ctx.bandEv[4 * b], st));
-                HIPCHK(hipStreamWaitEvent(g_ctx.copyStream, g_ctx.bandEv[4 * b], 0));
-                rc = copy_band(b);
-                if (rc) return rc;
+                if (t1 == nTot && g_ctx.timing) HIPCHK(hipEventRecord(g_ctx.ev1, st));
+                HIPCHK(hipEventRecord(g_ctx.evFork, st));
+                HIPCHK(hipStreamWaitEvent(g_ctx.stream2, g_ctx.evFork, 0));
+                const int rows = std::min(nzc, t1 / nRowTiles * SRWD_MESH_TILE);   // computed so far
+                // a band's last entry may hold 255 points of the rows after it
+                const int past = 255 / items[0].nxc + 1;
+                for (; b < nDl && (t1 == nTot || dlRow0[b + 1] + past <= rows); b++) {
+                    if (srwd_launch_finalize(dItems, dTileBlocks + dlTile0[b], 0, dlTile0[b + 1] - dlTile0[b],
+                                             std::max(1, g_ctx.tileE), dInfo, dEdge, termin, dPart, nSplit, nPointsPad,
+                                             dEx, dEz, dWarn, cnd, g_ctx.condTol, dFpList, dFpCount, dReq, dCoord, dLast,
+                                             g_ctx.stream2) ||
+                        srwd_launch_finalize(dItems, dRestBlocks + dlRest0[b], 0, dlRest0[b + 1] - dlRest0[b], 1, dInfo,
+                                             dEdge, termin, dPart, nSplit, nPointsPad, dEx, dEz, dWarn, cnd,
+                                             g_ctx.condTol, dFpList, dFpCount, dReq, dCoord, dLast, g_ctx.stream2))
+                        return SRWL_AMD_ERR_GPU;
+                    HIPCHK(hipEventRecord(g_ctx.bandEv[4 * b], g_ctx.stream2));
+                    HIPCHK(hipStreamWaitEvent(g_ctx.copyStream, g_ctx.bandEv[4 * b], 0));
+                    rc = copy_band(b);
+                    if (rc) return rc;
+                }
+                t0 = t1;
             }
+            HIPCHK(hipEventRecord(g_ctx.evJoin, g_ctx.stream2));
+            HIPCHK(hipStreamWaitEvent(st, g_ctx.evJoin, 0));
         } else {
         // the single-energy items (energies left over from the groups) on the
         // second stream, finished there by the two-pass form

@@ -83,3 +83,33 @@ def test_batch_mixes_both_kernels():
         srwlpy.CalcElecFieldSR(w, 0, m, prec)
         g, o = cfield(b.arEx, b), cfield(w.arEx, w)
         assert np.linalg.norm(g - o) < 1e-6 * np.linalg.norm(o)
+
+
+@pytest.mark.parametrize("nx,ny,ne", [(70, 300, 60), (33, 600, 64), (300, 65, 70), (64, 130, 140)])
+def test_streamed_tile_rows_equal_one_pass(nx, ny, ne):
+    """Fields of 16 MB or more, without mirror symmetry: the sums launched by
+    tile rows with the finished rows' copies beside them, against one launch
+    and one copy.  The s-range is cut alike, so the fields are the same bits.
+    33 x 600 reaches so far off axis that the points recomputed in FP64 are more
+    than the streamed copy patches, and the whole field is copied again."""
+    from srw_amd import srwlpy
+    print("case: %d x %d x %d streamed tile rows" % (nx, ny, ne), flush=True)
+    w, mag, prec = W.single_electron(n=nx, ne=ne, de_rel=0.02)
+    p = w.partBeam.partStatMom1
+    p.x, p.y, p.xp, p.yp = 20e-6, 10e-6, 3e-6, 2e-6
+    span = w.mesh.yFin - w.mesh.yStart
+    w.allocate(ne, nx, ny)
+    w.mesh.yFin = w.mesh.yStart + span * ny / nx * 0.5
+    got = []
+    for bands in (1, 0):
+        wg = clone_wfr(w)
+        srwlpy.set_bands(bands)
+        try:
+            srwlpy.CalcElecFieldSR(wg, 0, mag, prec)
+        finally:
+            srwlpy.set_bands(0)
+        print("bands %d: streamed %s" % (bands, srwlpy.last_streamed()), flush=True)
+        got.append([np.frombuffer(getattr(wg, c), np.float32) for c in ("arEx", "arEy")])
+    for a, b in zip(*got):
+        assert np.isfinite(a).all() and np.abs(a).max() > 0
+        assert np.array_equal(a, b)
