@@ -234,11 +234,17 @@ static int mesh_tiles(int nx, int nz)
 }
 
 // Whether the sums of a request over nxc x nzc computed points go to the mesh
-// kernel.
+// kernel: where its tiles hold at least one point in 8 places.  Below that the
+// kernels of one lane per point have less to do, most of all with many photon
+// energies, which their tiles share phases over.  Whole calls, one lane per
+// point / mesh kernel: 31 x 31 x 50 energies 0.65 / 0.50 ms, 24 x 24 x 50
+// 0.58 / 0.49 ms, 12 x 300 x 10 0.62 / 0.50 ms, 16 x 1000 x 20 1.88 / 1.35 ms;
+// past the line 16 x 16 x 200 0.64 / 0.78 ms, 8 x 8 x 200 0.60 / 0.75 ms, 4 x
+// 100 x 60 0.56 / 0.63 ms.  One photon energy: the same within 2 %.
 static bool mesh_kernel_pays(int nxc, int nzc)
 {
     const long long T2 = SRWD_MESH_TILE * SRWD_MESH_TILE;
-    return mesh_tiles(nxc, nzc) * T2 <= 4LL * nxc * nzc;
+    return mesh_tiles(nxc, nzc) * T2 <= 8LL * nxc * nzc;
 }
 
 // Parts of the s-range of a mesh pass of nTiles tiles and nPts points: the least

@@ -40,7 +40,8 @@ def _case(nx, ny, ne=1, nper=12, np_traj=1201, tilt=False):
     return w, W.planar_undulator(1.5, 0.02, nper), W.traj_prec(np_traj, nper=nper)
 
 
-@pytest.mark.parametrize("nx,ny", [(32, 32), (33, 65), (64, 64), (65, 63), (128, 31), (40, 97), (16, 16), (200, 5)])
+@pytest.mark.parametrize("nx,ny", [(32, 32), (33, 65), (64, 64), (65, 63), (128, 31), (40, 97), (16, 16), (200, 5),
+                                   (22, 23), (23, 23), (12, 300)])
 def test_mesh_sizes_around_a_tile(nx, ny):
     """The last two are too small or too narrow for the kernel: the per-point one."""
     print("case:", nx, ny, flush=True)
