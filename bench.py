@@ -23,19 +23,13 @@ import time
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-FP32_VALU_PEAK_TFLOPS = 157.3      # MI355X published FP32 vector peak (packed FMA)
+MFMA_F16_PEAK_TFLOPS = 2500.       # MI355X dense FP16 matrix peak
 HBM_PEAK_GBS = 8000.0
-# FP32 flops the k_sr_integral loop executes per integrand evaluation: two
-# phase FMAs, two amplitude FMAs and four accumulating FMAs (8 FMA = 16 flops);
-# the hardware sine and cosine are not counted.
-FLOPS_PER_EVAL = 16
-# the same for k_sr_integral_tile<8>, per energy of a group of 8: four
-# accumulating FMAs (8), the two recurrence FMAs for 4 of the 8 energies
-# (4, over 2), and the per-s work shared by the 8 (four phase FMAs, the
-# second chain's start phase FMA and two adds, the doubled cosine, two
-# amplitude FMAs: 17, over 8)
-FLOPS_PER_EVAL_TILE = 8 + 4 * 4 / 8 + 17 / 8
-VALU_LANE_ISSUE_PER_S = 256 * 4 * 16 * 2.4e9   # CUs x SIMDs x lanes per cycle x clock
+# FP16 matrix flops of k_sr_mesh per integrand evaluation: two complex products
+# of FP16 hi + lo pairs, three of the four parts of each of their four real
+# products (24 multiply-adds); the phasors, one per (row or column, s), and the
+# places of a tile outside the mesh are not counted.
+FLOPS_PER_EVAL = 48
 
 
 def log(msg):
@@ -165,11 +159,11 @@ def multi_e_runs(srwlpy, W, n, nmax, seeds=8, validate=True):
 
 
 def sr_traffic(n, ne):
-    """HBM bytes per k_sr_integral launch from the committed PMC summary
+    """HBM bytes per k_sr_mesh launch from the committed PMC summary
     (FETCH_SIZE + WRITE_SIZE, calibrated against a plain copy), when it was
     measured for this workload; None otherwise."""
     import re
-    path = os.path.join(ROOT, "profiles", "k_sr_integral_%dx%dx%d_traffic.md" % (n, n, ne))
+    path = os.path.join(ROOT, "profiles", "k_sr_mesh_%dx%dx%d_traffic.md" % (n, n, ne))
     if not os.path.exists(path):
         return None
     m = re.search(r"hbm_bytes_per_launch\s*=\s*([0-9.eE+]+)", open(path).read())
@@ -185,21 +179,6 @@ def fft_traffic(n, slices):
         return None
     m = re.search(r"hbm_bytes_per_drift\s*=\s*([0-9.eE+]+)", open(path).read())
     return float(m.group(1)) if m else None
-
-
-def sr_valu_per_eval(n, ne):
-    """(vector, transcendental) instructions per integrand evaluation of
-    k_sr_integral from the committed counter summary (SQ_INSTS_VALU and
-    SQ_INSTS_VALU_TRANS_F32 per 64 evaluations); (None, None) when not
-    measured for this workload."""
-    import re
-    path = os.path.join(ROOT, "profiles", "k_sr_integral_%dx%dx%d_sq_counters.md" % (n, n, ne))
-    if not os.path.exists(path):
-        return None, None
-    txt = open(path).read()
-    m = re.search(r"valu_instr_per_eval\s*=\s*([0-9.eE+]+)", txt)
-    t = re.search(r"valu_trans_per_eval\s*=\s*([0-9.eE+]+)", txt)
-    return (float(m.group(1)) if m else None), (float(t.group(1)) if t else None)
 
 
 def uneven_batch(srwlpy, W, n):
@@ -441,17 +420,7 @@ def main():
     st_dev = srwlpy.stats()
     srwlpy.set_keep_on_device(False)
     k_ms_dev = st_dev["sum_sr_ms"] / max(st_dev["n_sr"], 1)
-    # executed FP32 flops per evaluation: the energy-tile kernel takes the
-    # energies of whole groups of 8, the single-energy kernel the rest
-    tiled = (a.ne // 8) * 8 / a.ne if a.ne >= 8 else 0.
-    flops_per_eval = tiled * FLOPS_PER_EVAL_TILE + (1. - tiled) * FLOPS_PER_EVAL
-    achieved = flops_per_eval * evals / (k_ms_dev * 1e-3) / 1e12
-    vpe, tpe = sr_valu_per_eval(a.n, a.ne)
-    # vector instructions issued per second over one wave64 instruction per 4
-    # cycles per SIMD; and the same with each transcendental taking two slots
-    # (they issue at a lower rate than FMAs)
-    issue = vpe * evals / (k_ms_dev * 1e-3) / VALU_LANE_ISSUE_PER_S if vpe else None
-    issue2 = (vpe + tpe) * evals / (k_ms_dev * 1e-3) / VALU_LANE_ISSUE_PER_S if vpe and tpe is not None else None
+    achieved = FLOPS_PER_EVAL * evals / (k_ms_dev * 1e-3) / 1e12
     c1 = c1_methods(srwlpy, W)
     log("101x101 methods 0 and 1 done")
     prop = None
@@ -483,25 +452,21 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f32",
-        "precision": ("FP32 integrand, 64-point FP32 block sums added with Kahan compensation per 256-point chunk, "
-                      "FP64 chunk sums; FP64 trajectory, tables and per-chunk phase reference; points failing the "
-                      "FP32 condition check recomputed in FP64 (%d in the timed calls' last pass)" % fp64_points),
+        "precision": ("FP64 trajectory, tables and phase references; FP32 phase increments and phasors, multiplied as "
+                      "FP16 hi + lo pairs (22 bits) with FP32 sums over 32 points, FP64 beyond; points failing the "
+                      "condition check recomputed in FP64 (%d in the timed calls' last pass)" % fp64_points),
         "data": "synthetic",
         "config": {"workload": "planar undulator 3 GeV, lambda_u 20 mm x 100, K 1.5; %dx%d mesh at 20 m, %d photon "
                                "energies +/-5%% around the 1st harmonic; 10001-point trajectory, method 0; field "
                                "delivered into the caller's host arrays" % (a.n, a.n, a.ne),
                    "mesh": [a.n, a.n], "energies": a.ne, "trajectory_points": 10001, "parallelism": "single GPU"},
-        "roofline": {"bound": "valu", "achieved": achieved, "peak": FP32_VALU_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / FP32_VALU_PEAK_TFLOPS, "traffic": sr_traffic(a.n, a.ne),
-                     "kernel": "k_sr_integral_tile<8, false> + k_sr_integral", "kernel_ms": k_ms_dev,
-                     "evals_per_launch": evals, "flops_per_eval": flops_per_eval,
-                     "flops_counted": ("executed FP32 flops, an FMA counted as 2 (sin/cos excluded): 16 per evaluation "
-                                       "in the single-energy kernel; 12.125 in the energy-tile kernel (4 accumulating "
-                                       "FMAs, 2 recurrence FMAs for half of the energies, 1/8 of the per-s phase, "
-                                       "chain-start and amplitude work)"),
-                     "valu_instr_per_eval": vpe, "valu_trans_per_eval": tpe, "valu_issue_frac": issue,
-                     "valu_issue_frac_trans_two_slots": issue2,
-                     "nonpacked_fma_ceiling_frac": 0.5},
+        "roofline": {"bound": "mfma", "achieved": achieved, "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s",
+                     "frac": achieved / MFMA_F16_PEAK_TFLOPS, "traffic": sr_traffic(a.n, a.ne),
+                     "kernel": "k_sr_mesh", "kernel_ms": k_ms_dev,
+                     "evals_per_launch": evals, "flops_per_eval": FLOPS_PER_EVAL,
+                     "flops_counted": ("FP16 matrix flops of the mesh points: 24 multiply-adds per evaluation (both "
+                                       "components, hi + lo pairs); phasors and the tiles' places outside the mesh "
+                                       "(101 of 128 rows and columns used at 201 x 201) not counted")},
         "device_resident_points_per_s": pts * a.steps / dt_dev,
         "sr_kernel_ms_in_api_run": k_ms,
         "api_call_ms": {"min": 1e3 * min(call_s), "median": 1e3 * sorted(call_s)[len(call_s) // 2],

@@ -11,8 +11,9 @@
 // Precision: trajectory, tables and the per-chunk phase reference are FP64;
 // the per-point phase increment (|t| < ~2 revolutions) and the integrand sum
 // are FP32: 64-point FMA block sums, added with Kahan compensation within a
-// 256-point chunk, chunk sums in FP64.  A condition check of every point's
-// FP32 sum sends ill-conditioned points to an FP64 recomputation.
+// 256-point chunk, chunk sums in FP64 (transverse meshes: sr_mesh.hip).  A
+// condition check of every point's sum sends ill-conditioned points to an FP64
+// recomputation.
 #include "srw_sr_dev.h"
 
 // ------------------------------------------------------------------------

@@ -10,6 +10,23 @@
 //   Ex(x, z) = sum_s F'(x, s) G(z, s),   Ez(x, z) = sum_s F(x, s) G'(z, s)
 // are complex matrix products over s: (nx + nz) ns phasors and 8 real
 // multiply-adds per evaluation replace a phase, a sine and a cosine each.
+//
+// What bounds it: the matrix instructions (24 of 32x32x16 per 16 points and
+// 32 x 32 places, 48 FP16 flops an evaluation) and the vector work of the
+// phasors, which share a SIMD's issue: with either left out a launch took 5.2
+// of 8.1 ms (64 electrons on 512 x 512), so about half of the matrix time hides
+// behind the vector work.  512 x 512 points of 256 electrons: 36 ms, 0.9 of
+// 1.85 PFLOP/s that a plain loop of these instructions reaches here; one lane
+// per point with vector FMAs (k_sr_integral) took 176 ms.
+// * 64 x 64 tile: a phasor serves 64 points, and the two buffers of a stage
+//   (64 KB of LDS) leave two workgroups a CU, one's phasors beside the other's
+//   products.
+// * 16 points a stage: one instruction's k.  The products of hi and lo parts
+//   are summed small ones first.
+// * FP32 sums flushed to FP64 every 32 points (SRWD_MESH_UNIT): at 64 the
+//   kernel was 3 to 11 % faster and fields far below their peak carried more
+//   error than one lane per point gives; at 128 single points failed 1e-4.
+// * s_setprio around the products: 3 %.
 #include "srw_sr_dev.h"
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
