@@ -944,19 +944,42 @@ __device__ __forceinline__ double int_point_s(const srwd_trj_info& I, long long 
     return (i == I.nInt - 1) ? I.sIntegFin : I.sIntegStart + (double)i * I.h;
 }
 
+// Whether the field b of one plane and its slope dbds at s are rounding and no
+// more.  Both are derivatives of the quintic through six trajectory points, so
+// rounding errors of the positions (of size eps * the largest of them and of
+// the initial offset that they are summed from) come out divided by sStep^2 and
+// sStep^3.  At 2114 field-free edges (undulators of K 0.3 to 3, 5 to 120
+// periods of 10 to 50 mm; 300 to 10^5 points; offsets up to 3 mm, 0.5 to 6 GeV)
+// the field reached 338 and the slope 512 of these units, the medians 10 and 9.
+#define SRWD_EDGE_NOISE 1024.
+__device__ __forceinline__ bool edge_is_rounding(const srwd_trj_info& I, const double* crd, double x0, double s, double b,
+                                                 double dbds)
+{
+    long long idx = (long long)((s - I.sStart) / I.sStep);
+    if (idx >= I.np - 1) idx = I.np - 2;
+    if (idx < 0) idx = 0;
+    const double* f = crd + offset5(idx, I.np);
+    double m = 0.;
+    for (int k = 0; k < 6; k++) m = fmax(m, fabs(f[k]));
+    const double lim = SRWD_EDGE_NOISE * 1.1102230246251565e-16 * (m + fabs(x0)) / (fabs(I.betaNorm) * I.sStep * I.sStep);
+    return fabs(b) <= lim && fabs(dbds) * I.sStep <= lim;
+}
+
 // Edge data at the integration limits (srtrjdat.h:1006-1034), end 0 or 1.
-// Outside the magnet the field and its slope there are the rounding of the
-// interpolation's higher derivatives (about 1e-13 T and 5e-10 T/m, decided by
-// the low bits of the positions), which moves fields of low photon energies by
-// 1e-4: a field below 1e-10 T, the reference's own limit of a field-free edge
-// (srtrjdat.h:119), is taken as zero.
+// Outside the magnet the field and its slope there are rounding (about 1e-13 T
+// and 5e-10 T/m on axis at steps of 0.2 mm), which moves fields of low photon
+// energies by 1e-4, and by as much as the field itself for an electron 0.1 mm
+// off axis at steps of 0.05 mm: a plane where both are is field-free.  Where
+// only one is, both stay: at a zero of the field inside the magnet the slope
+// counts, and the expansion of the end terms takes another branch at b = 0 than
+// at any other value (residual()).
 __device__ __forceinline__ void sr_edge(const srwd_trj_info& I, const double* cx, const double* cz, const double* ix,
                                         const double* iz, int end, srwd_edge& E)
 {
     const double s = end ? I.sIntegFin : I.sIntegStart;
     trj_pt px = eval_plane(I, cx, ix, -1. / I.betaNorm, s, true), pz = eval_plane(I, cz, iz, 1. / I.betaNorm, s, true);
-    if (fabs(px.b) < 1.E-10) px.b = px.dbds = 0.;
-    if (fabs(pz.b) < 1.E-10) pz.b = pz.dbds = 0.;
+    if (edge_is_rounding(I, cx, I.x0, s, px.b, px.dbds)) px.b = px.dbds = 0.;
+    if (edge_is_rounding(I, cz, I.z0, s, pz.b, pz.dbds)) pz.b = pz.dbds = 0.;
     double* v = E.v[end];
     v[0] = px.dbds; v[1] = px.b; v[2] = px.bt; v[3] = px.crd; v[4] = px.ib;
     v[5] = pz.dbds; v[6] = pz.b; v[7] = pz.bt; v[8] = pz.crd; v[9] = pz.ib;
