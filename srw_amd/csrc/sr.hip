@@ -1467,8 +1467,14 @@ __global__ void __launch_bounds__(256) k_sr_integral_tile(const srwd_item* __res
 // Energy-tile items: the phasor of energy k carries k times the rounding of
 // the step's phase and the recurrence's roundings on top.
 #define SRWD_EPS_TERM_TILE 4e-6
-// Mesh items (sr_mesh.hip): phases reduced in FP64 before their sine and
-// cosine, phasors as FP16 pairs of about 22 bits.
+// Mesh items (sr_mesh.hip): the phase is an FP64 reference, reduced, plus FP32
+// increments of up to srwd_mesh_turns revolutions; the phasor is an FP16 pair of
+// about 22 bits.  48 requests of harmonics 1-5, K 0.5-2.5 (2.0e6 points, 1.0e6
+// computed), against every point in FP64; points recomputed / worst error left:
+// without the check 0 / 3.6e-3 (6.1e-3 with one lane per point), 1e-6 5.6e4 /
+// 5.3e-5 (7.9e-5), 2e-6 8.9e4 / 3.0e-5 (3.8e-5), 4e-6 1.4e5 / 2.8e-5 (2.1e-5):
+// 2e-6 leaves a factor 3.3.  Those turns stay below 0.5; beyond SRWD_MESH_TURNS
+// the increments' rounding (4e-7 a turn) leads and the estimate grows with them.
 #define SRWD_EPS_TERM_MESH 2e-6
 
 // Terminating terms, the derivative correction, the float store and the
@@ -1511,8 +1517,9 @@ __device__ void sr_finish_point(const srwd_item& IT, const srwd_trj_info& I, con
     if (fpList) {
         // condition check of the FP32 sums against the point's field
         // magnitude: hand the point to the FP64 pass
-        const double eps = IT.tiled == SRWD_ITEM_MESH ? SRWD_EPS_TERM_MESH
-                                                      : (IT.tiled ? SRWD_EPS_TERM_TILE : SRWD_EPS_TERM);
+        const double eps = IT.tiled == SRWD_ITEM_MESH
+                               ? SRWD_EPS_TERM_MESH * fmax(1., srwd_mesh_turns(I, IT.eph, xo, zo) / SRWD_MESH_TURNS)
+                               : (IT.tiled ? SRWD_EPS_TERM_TILE : SRWD_EPS_TERM);
         const double e2 = eps * eps * w * w, t2 = condTol * condTol;
         const double mag2 = ex.re * ex.re + ex.im * ex.im + ez.re * ez.re + ez.im * ez.im;
         if (e2 * (fmax(sumSqX, 0.) + fmax(sumSqZ, 0.)) > t2 * mag2) {
@@ -1546,9 +1553,10 @@ __device__ void sr_finish_point(const srwd_item& IT, const srwd_trj_info& I, con
 // cond[0..4] = sum b^2, sum b bPx, sum b bPz, sum bPx^2, sum bPz^2, so that
 // the squared x terms of point (xo, zo) add up to
 // cond[0] xo^2 - 2 xo cond[1] + cond[3] (and the z terms likewise).  The
-// largest |b|, |bPx| and |bPz| give the amplitude scales of the mesh records.
+// largest |b|, |bPx| and |bPz| give the amplitude scales of the mesh records, the
+// last two also angX and angZ: b P = w P / R^2 with w at most 16.
 #define SRWD_CS_THREADS 1024
-__global__ void __launch_bounds__(SRWD_CS_THREADS) k_cond_sums(const srwd_trj_info* __restrict__ info,
+__global__ void __launch_bounds__(SRWD_CS_THREADS) k_cond_sums(srwd_trj_info* __restrict__ info,
                                                                const srwd_rec* __restrict__ rec, long long ldI,
                                                                double* cond, srwd_mrec* M, long long ldM,
                                                                const double* __restrict__ mesh, double* scale)
@@ -1579,6 +1587,11 @@ __global__ void __launch_bounds__(SRWD_CS_THREADS) k_cond_sums(const srwd_trj_in
         v[k] = x;
     }
     if (threadIdx.x < 5) cond[5 * tr + threadIdx.x] = v[threadIdx.x];
+    if (threadIdx.x == 0) {
+        const double far = info[tr].yObs - info[tr].sIntegStart;
+        info[tr].angX = v[6] * far / 14.;
+        info[tr].angZ = v[7] * far / 14.;
+    }
     const double* ml = mesh + 4 * tr;
     for (int side = 0; side < 2; side++) {
         const double a = v[5] * fmax(fabs(ml[2 * side]), fabs(ml[2 * side + 1])) + v[6 + side];
@@ -2023,7 +2036,7 @@ int srwd_launch_finalize(const srwd_item* dItems, const int2* dEntries, int nbU,
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int srwd_launch_cond_sums(const srwd_trj_info* dInfo, int nTraj, const srwd_rec* dRec, long long ldI, double* dCond,
+int srwd_launch_cond_sums(srwd_trj_info* dInfo, int nTraj, const srwd_rec* dRec, long long ldI, double* dCond,
                           srwd_mrec* dMrec, long long ldM, const double* dMesh, double* dScale, hipStream_t st)
 {
     hipLaunchKernelGGL(k_cond_sums, dim3(nTraj), dim3(SRWD_CS_THREADS), 0, st, dInfo, dRec, ldI, dCond, dMrec, ldM,

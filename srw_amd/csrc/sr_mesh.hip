@@ -99,7 +99,7 @@ struct mesh_row {
 // The phasor and the weighted phasor of one row at the 8 integration points
 // of G, as 8 planes (phasor re hi, re lo, im hi, im lo; weighted the same) of
 // 8 FP16 values.  The phase at the reference point is formed and reduced in FP64;
-// the other points add FP32 increments, a fraction of a revolution.
+// the other points add FP32 increments (srwd_mesh_turns).
 __device__ __forceinline__ void mesh_gen(const mesh_row& W, const mesh_grp& G, uint4v* dst)
 {
     unsigned o[8][4];

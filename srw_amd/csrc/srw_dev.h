@@ -57,6 +57,7 @@ struct srwd_trj_info {
     double sIntegStart, sIntegFin, h;   // integration range and step
     long long nInt;          // integration points (odd)
     double yObs;             // longitudinal observation position
+    double angX, angZ;       // largest angles of the projected positions Px, Pz (srwd_mrec) seen from the observation plane
 };
 
 // Per integration point, energy independent (FP32), 32 bytes: phase increments
@@ -131,6 +132,18 @@ struct srwd_mrec {
 inline long long srwd_mesh_ld(long long nInt)
 {
     return (nInt + SRWD_MESH_UNIT - 1) / SRWD_MESH_UNIT * (SRWD_MESH_UNIT / 8) + 2;
+}
+// Revolutions of the phase from the reference point of a group of records to its
+// farthest point, 4 steps away, at observation point (x, z): about the largest
+// sum of the magnitudes of the FP32 increments that the mesh kernel adds there.
+// A sampled integrand turns by less than 2; up to SRWD_MESH_TURNS the rounding
+// of the increments is below that of the phasors.
+#define SRWD_MESH_TURNS 4.
+inline __host__ __device__ double srwd_mesh_turns(const srwd_trj_info& I, double eph, double x, double z)
+{
+    const double inv = 1. / (I.yObs - I.sIntegFin);
+    const double ax = I.angX + (x < 0. ? -x : x) * inv, az = I.angZ + (z < 0. ? -z : z) * inv;
+    return 4. * I.h * 0.40327329e+06 * eph * (I.gammaEm2 + ax * ax + az * az);
 }
 
 // One request of a field computation, for the parts that follow the
@@ -256,8 +269,9 @@ int srwd_launch_finalize(const srwd_item* dItems, const int2* dEntries, int nbU,
 // It also scales the mesh records' b (see srwd_mrec) so that the largest
 // amplitude of a side over the integration points and the request's mesh
 // (dMesh: xStart, xEnd, zStart, zEnd per trajectory) lies in [2^11, 2^12),
-// and writes the inverse scales (powers of two) to dScale.
-int srwd_launch_cond_sums(const srwd_trj_info* dInfo, int nTraj, const srwd_rec* dRec, long long ldI, double* dCond,
+// and writes the inverse scales (powers of two) to dScale, and angX, angZ of
+// dInfo.
+int srwd_launch_cond_sums(srwd_trj_info* dInfo, int nTraj, const srwd_rec* dRec, long long ldI, double* dCond,
                           srwd_mrec* dMrec, long long ldM, const double* dMesh, double* dScale, hipStream_t st);
 // FP64 recomputation and store of the listed points (block indices relative
 // to dBlockItem, as passed to srwd_launch_finalize).

@@ -247,6 +247,25 @@ static bool mesh_kernel_pays(int nxc, int nzc)
     return mesh_tiles(nxc, nzc) * T2 <= 8LL * nxc * nzc;
 }
 
+// Whether the FP32 phase increments of the mesh kernel are as fine over the mesh
+// as those of one lane per point.  They hold the whole phase over 4 steps, the
+// other kernels' the part that depends on the observation point over a chunk,
+// with the rest from a table reduced in FP64: where a sampled integrand ends
+// (SRWD_MESH_TURNS), the kernel of the smaller phase.  1 MeV in steps of 8.6 mm,
+// 870 turns: 40 x 40 points over 20 um, one lane per point / mesh kernel
+// 3.4e-7 / 2.3e-4 rel-L2; over 2 mm, where a chunk turns 2200 times, 2.3e-4 /
+// 1.3e-4.
+static bool mesh_kernel_fine(const srwd_trj_info& I, const SRWLRadMesh& m)
+{
+    const double e = std::max(m.eStart, m.eFin);
+    const double x = std::max(std::fabs(m.xStart), std::fabs(m.xFin)), z = std::max(std::fabs(m.yStart), std::fabs(m.yFin));
+    const double turns = srwd_mesh_turns(I, e, x, z);
+    srwd_trj_info C = I;   // a chunk's steps, of the observation angles alone
+    C.h *= 0.25 * (double)std::min<long long>(I.nInt, SRWD_CHUNK);
+    C.gammaEm2 = C.angX = C.angZ = 0.;
+    return turns <= std::max(SRWD_MESH_TURNS, srwd_mesh_turns(C, e, x, z));
+}
+
 // Parts of the s-range of a mesh pass of nTiles tiles and nPts points: the least
 // of a model of its time.  512 workgroups are resident at once (two a CU, by
 // LDS) and such a round takes 3.7 us per unit of the s-range (512 x 512
@@ -552,7 +571,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     std::vector<char> isMesh(nT);
     bool allMesh = true;
     for (int j = 0; j < nT; j++) {
-        isMesh[j] = mesh_kernel_pays(reqs[j].nxc, reqs[j].nzc);
+        isMesh[j] = mesh_kernel_pays(reqs[j].nxc, reqs[j].nzc) && mesh_kernel_fine(info[j], jobs[j].mesh);
         allMesh = allMesh && isMesh[j];
     }
     for (int j = 0; j < nT; j++) {

@@ -114,3 +114,29 @@ def test_streamed_tile_rows_equal_one_pass(nx, ny, ne):
     for a, b in zip(*got):
         assert np.isfinite(a).all() and np.abs(a).max() > 0
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("e_ev,step,half", [(1e6, 40, 1e-5), (1e6, 10, 1e-5), (1e7, 10, 1e-5), (1e5, 40, 1e-5),
+                                            (1e5, 2, 1e-5), (1e5, 1, 1e-4), (1e6, 40, 1e-3), (1.6e3, 1, 5e-2)])
+def test_coarse_steps_keep_the_phase(e_ev, step, half):
+    """Photon energies and steps at which the phase turns by 1 to 2000
+    revolutions over 4 steps, on both sides of the rule that takes the kernel,
+    and a mesh far off axis: every point against its own FP64 recomputation.
+    Tolerance: the condition check's, 1e-4 of a point's field."""
+    from srw_amd import srwlpy
+    print("case: %g eV, step x %g, half %g m" % (e_ev, step, half), flush=True)
+    w = W.wavefront(W.electron_beam(x=2e-6, y=1e-6), 1, e_ev, e_ev, 40, 40, half, half, 20.)
+    prec = W.traj_prec(10001)
+    prec[1] *= step
+    got = []
+    for tol in (1e-4, 1e-12):
+        wg = clone_wfr(w)
+        srwlpy.set_cond_tol(tol)
+        try:
+            srwlpy.CalcElecFieldSR(wg, 0, W.planar_undulator(), prec)
+        finally:
+            srwlpy.set_cond_tol(1e-4)
+        got.append(np.stack([cfield(wg.arEx, wg), cfield(wg.arEy, wg)]))
+    err = np.sqrt((np.abs(got[0] - got[1]) ** 2).sum(0) / (np.abs(got[1]) ** 2).sum(0))
+    print("worst %.2e, rel-L2 %.2e" % (err.max(), np.linalg.norm(got[0] - got[1]) / np.linalg.norm(got[1])), flush=True)
+    assert err.max() < 1e-4
