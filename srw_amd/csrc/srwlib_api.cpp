@@ -767,20 +767,27 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         minChunks = std::min(minChunks, (I.nInt + SRWD_CHUNK - 1) / SRWD_CHUNK);
         minUnits = std::min(minUnits, (I.nInt + SRWD_MESH_UNIT - 1) / SRWD_MESH_UNIT);
     }
-    // workgroups of a band: every block of the single-energy items, one per
-    // group of SRWD_TILE_E energies for the tiles (the tile kernel's
-    // workgroups each do SRWD_TILE_E times the work, so fewer fill the GPU)
-    const int nWG = (int)(srTileBlocks.size() + srRestBlocks.size());
     int nSplit = 1;
     if (allMesh) {
-        nSplit = mesh_split((long long)nMeshTiles / nBands, minUnits, nPointsPad / nBands, large);
+        nSplit = mesh_split((long long)nMeshTiles / nBands, minUnits, large ? nPointsPad : nPointsPad / nBands, large);
         // a no-allocation call keeps its partial sums within what one block
         // per 256 points would take
         if (g_arena) nSplit = std::min(nSplit, std::max(1, 4096 / nBlocks));
     } else {
-        const int bandWG = (nWG + nBands - 1) / nBands;
-        const int wgTarget = srTileBlocks.empty() ? 4096 : 1024;
-        nSplit = (int)std::min<long long>(std::max<long long>(1, (wgTarget + bandWG - 1) / bandWG), minChunks);
+        // workgroups of a band: every block of the single-energy items, one per
+        // group of SRWD_TILE_E energies for the tiles (the tile kernel's
+        // workgroups each do SRWD_TILE_E times the work, so fewer fill the GPU).
+        // Mesh items have a place in every part: among them the parts stop at
+        // 16384 blocks of 256 points (134 MB, 70 us to write and read), or where
+        // all items counted alike would.  Parts for the small request alone / so
+        // bounded: 24 of 512 x 512 and one axis point, 40 / 1, 8.3 / 6.7 ms.
+        auto parts = [&](size_t nTile, size_t nRest) {
+            const int bandWG = ((int)(nTile + nRest) + nBands - 1) / nBands, target = nTile ? 1024 : 4096;
+            return std::max(1, (target + bandWG - 1) / bandWG);
+        };
+        nSplit = (int)std::min<long long>(parts(srTileBlocks.size(), srRestBlocks.size()), minChunks);
+        if (!meshTiles.empty())
+            nSplit = std::min(nSplit, std::max(parts(tileBlocks.size(), restBlocks.size()), 16384 / nBlocks));
     }
     if (g_ctx.forceSplit > 0) nSplit = (int)std::min<long long>(g_ctx.forceSplit, minChunks);
     std::vector<int2> srLists;   // finalize lists, then the lists of the sums

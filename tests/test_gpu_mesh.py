@@ -86,6 +86,27 @@ def test_batch_mixes_both_kernels():
         assert np.linalg.norm(g - o) < 1e-6 * np.linalg.norm(o)
 
 
+@pytest.mark.parametrize("small,ne", [((1, 1), 1), ((1, 3), 9), ((9, 1), 1)])
+def test_small_request_among_meshes_keeps_the_parts(small, ne):
+    """One request off the mesh kernel in a batch of large meshes: the partial
+    sums, which hold every point of the batch once per part of the s-range, stay
+    within 16384 blocks of 256 points."""
+    from srw_amd import srwlpy
+    print("case: 6 meshes of 256 x 256 and one of %d x %d x %d" % (small[0], small[1], ne), flush=True)
+    reqs = [_case(256, 256, ne if k % 2 else 1, tilt=True, np_traj=4001) for k in range(6)]
+    reqs.append(_case(small[0], small[1], ne, tilt=True, np_traj=4001))
+    ws, ms, prec = [r[0] for r in reqs], [r[1] for r in reqs], reqs[0][2]
+    wb = [clone_wfr(w) for w in ws]
+    srwlpy.CalcElecFieldSRBatch(wb, ms, prec)
+    st = srwlpy.stats()
+    print("%d blocks in %d parts" % (st["sr_blocks"], st["sr_split"]), flush=True)
+    assert st["sr_blocks"] * st["sr_split"] <= 16384
+    for k in (0, 1, 6):
+        srwlpy.CalcElecFieldSR(ws[k], 0, ms[k], prec)
+        g, o = cfield(wb[k].arEx, wb[k]), cfield(ws[k].arEx, ws[k])
+        assert np.linalg.norm(g - o) < 1e-6 * np.linalg.norm(o)
+
+
 @pytest.mark.parametrize("nx,ny,ne", [(70, 300, 60), (33, 600, 64), (300, 65, 70), (64, 130, 140)])
 def test_streamed_tile_rows_equal_one_pass(nx, ny, ne):
     """Fields of 16 MB or more, without mirror symmetry: the sums launched by
