@@ -9,6 +9,7 @@
 //   srwlCalcPartTraj       cpp/src/lib/srwlib.cpp:328-373
 //   srwlUtiGetErrText etc. cpp/src/lib/srwlib.cpp:78-140
 #include "srw_api_internal.h"
+#include "srw_moments.h"
 #include "srw_fft.h"
 
 #include <emmintrin.h>
@@ -770,9 +771,6 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     int nSplit = 1;
     if (allMesh) {
         nSplit = mesh_split((long long)nMeshTiles / nBands, minUnits, large ? nPointsPad : nPointsPad / nBands, large);
-        // a no-allocation call keeps its partial sums within what one block
-        // per 256 points would take
-        if (g_arena) nSplit = std::min(nSplit, std::max(1, 4096 / nBlocks));
     } else {
         // workgroups of a band: every block of the single-energy items, one per
         // group of SRWD_TILE_E energies for the tiles (the tile kernel's
@@ -798,16 +796,26 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     // warning, FP64 stores recorded for the host, FP64 points per band: zero, read back in one copy
     const size_t oCounts = us.zeros(sizeof(int) * (2 + (size_t)nBands));
     float* dA = (float*)B.A.get(sizeof(float) * (size_t)ldI * nRows);
-    double* dPart = (double*)B.Part.get(sizeof(double) * 4 * (size_t)nSplit * nPointsPad);
     // condition check of the FP32 sums and the FP64 recomputation list (one band at a time)
     int maxBandBlocks = 0;
     for (int b = 0; b < nBands; b++) maxBandBlocks = std::max(maxBandBlocks, bandBlock0[b + 1] - bandBlock0[b]);
     // one list per compute stream: consecutive bands run on alternate streams
     const int nLists = nBands > 1 ? 2 : 1;
     int* dFpList = (int*)B.FpList.get(sizeof(int) * 256 * (size_t)maxBandBlocks * nLists);
-    if (!dA || !dPart || !dFpList) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+    if (!dA || !dFpList) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
     rc = upload_requests();
     if (rc) return rc;
+    // a no-allocation call takes the parts that its scratch still holds beside
+    // the moments that follow (long integration tables leave few)
+    const size_t partBytes = sizeof(double) * 4 * (size_t)nPointsPad;
+    if (g_arena) {
+        const SRWLRadMesh& m = jobs[0].mesh;
+        const size_t keep = (size_t)srwm_work_bytes((int)m.ne, (int)m.nx, (int)m.ny, m.ne > 1) + ((size_t)1 << 20);
+        const size_t left = g_arena->cap - g_arena->used;
+        nSplit = (int)std::min<size_t>(nSplit, std::max<size_t>(1, left > keep ? (left - keep) / partBytes : 1));
+    }
+    double* dPart = (double*)B.Part.get((size_t)nSplit * partBytes);
+    if (!dPart) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
     srwd_item* dItems = (srwd_item*)(dUs + oItems);
     const int* dBlockItem = nbU ? nullptr : (const int*)(dUs + oBlockItem);
     int* dWarn = (int*)(dUs + oCounts);

@@ -57,6 +57,28 @@ def test_no_alloc_matches_allocating_entry_point_twice():
         np.testing.assert_allclose(np.array(wn.arMomX), np.array(wa.arMomX), rtol=1e-6, atol=1e-30)
 
 
+@pytest.mark.parametrize("nx,ny,n_int", [(256, 256, 240001), (256, 256, 280001), (64, 64, 320001), (65536, 1, 280001)])
+def test_no_alloc_takes_long_integration_tables(nx, ny, n_int):
+    """The largest fields with integration points far finer than the
+    trajectory's: the tables fill most of the scratch, and the s-range goes in the
+    parts that the rest holds."""
+    srwlpy, lib = _lib()
+    assert lib.srwlAmdNoAllocInit() == 0
+    print("case: no-alloc field %d x %d, %d integration points" % (nx, ny, n_int), flush=True)
+    w, mag, prec = W.single_electron(n=16, np_traj=20001)
+    span = w.mesh.xFin - w.mesh.xStart
+    w.allocate(1, nx, ny)
+    w.mesh.xFin = w.mesh.xStart + 0.9 * span   # no mirror symmetry in x
+    prec[1] = 2 * (0.5 * 100 * 0.02 + 4 * 0.02) / (n_int - 0.5)
+    wa, wn = clone_wfr(w), clone_wfr(w)
+    srwlpy.CalcElecFieldSR(wa, 0, mag, prec)
+    assert _noalloc(lib, wn, mag, prec) == 0
+    for a, b in ((wa.arEx, wn.arEx), (wa.arEy, wn.arEy)):
+        ea, eb = cfield(a, wa), cfield(b, wn)
+        if np.abs(ea).max() > 0:
+            assert rel_l2(eb, ea) < 1e-6, rel_l2(eb, ea)
+
+
 def test_no_alloc_refuses_requests_beyond_its_scratch():
     srwlpy, lib = _lib()
     assert lib.srwlAmdNoAllocInit() == 0
