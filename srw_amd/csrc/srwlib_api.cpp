@@ -1170,6 +1170,11 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
 char* grow_pinned(char*& p, size_t& have, size_t bytes)
 {
     if (bytes > have) {
+        // queued copies may still read or write the buffer that goes: an
+        // upload of the same call (upload_segs returns before its DMAs end), on
+        // any of the streams
+        for (hipStream_t st : {g_ctx.stream, g_ctx.stream2, g_ctx.copyStream})
+            if (p && hipStreamSynchronize(st) != hipSuccess) return nullptr;
         if (p) (void)hipHostFree(p);
         p = nullptr;
         have = 0;

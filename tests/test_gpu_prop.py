@@ -214,3 +214,37 @@ def test_resize_to_good_size_then_drift():
     i_e = rel_l2(ig, io)
     print("rel-L2 I %.3e" % i_e, flush=True)
     assert i_e < 1e-4
+
+
+_FIRST_TRANSFERS = """
+import sys
+sys.path.insert(0, %r)
+import numpy as np
+from srw_amd import srwlpy
+from srw_amd.srwlib import SRWLOptC, SRWLOptD
+from tests.golden import cases
+from tests.util import clone_wfr
+w = cases.radsub_wavefront(dict(w0=20e-6, z0=10., n=600, half=1.2e-3, L=20., R=None, dRf=0.01))
+opt = SRWLOptC([SRWLOptD(5.)], [[0, 0, 1.0, 0, 0, 1.0, 2.0, 1.0, 2.0]])
+out = []
+for k in range(2):
+    wg = clone_wfr(w)
+    srwlpy.PropagElecField(wg, opt)
+    out.append([np.frombuffer(a, np.float32) for a in (wg.arEx, wg.arEy)])
+    assert wg.mesh.nx >= 1150 and np.isfinite(out[-1][0]).all() and np.abs(out[-1][0]).max() > 0
+assert all(np.array_equal(a, b) for a, b in zip(*out))
+print("same")
+"""
+
+
+def test_staging_grown_between_the_transfers_of_a_call():
+    """The first propagation of a process uploads 5.8 MB through the pinned
+    staging and then needs a larger one for the 23 MB it downloads: the same bits
+    as the second call, which finds it grown."""
+    import os
+    import subprocess
+    import sys
+    print("case: first propagation of a process, 600 x 600 to 1200 x 1200", flush=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", _FIRST_TRANSFERS % root], cwd=root, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "same" in r.stdout, r.stdout + r.stderr
