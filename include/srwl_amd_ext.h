@@ -44,9 +44,10 @@ SRWL_EXPORT int srwlAmdSetSplit(int nSplit);
 SRWL_EXPORT int srwlAmdSetBands(int nBands);
 
 /* on != 0 (default): a single request whose field takes the banded download
- * and has energy tiles is computed in one pass whose blocks finish their own
- * points and count finished row bands, each band downloaded as soon as it is
- * complete; 0: row bands computed one after another. */
+ * is computed in one pass, each row band downloaded as soon as it is complete:
+ * a mesh in launches of whole tile rows, a request with energy tiles by blocks
+ * that finish their own points and flag themselves done; 0: row bands computed
+ * one after another. */
 SRWL_EXPORT int srwlAmdSetStreamRows(int on);
 
 /* 1 when the last single-request call took the streamed-rows download to the
@@ -57,6 +58,17 @@ SRWL_EXPORT int srwlAmdLastStreamed(void);
  * trajectory) instead of the parallel-in-s solver; both give the serial RK4
  * recurrence, the switch exists to compare them. */
 SRWL_EXPORT int srwlAmdSetTrajSerial(int on);
+
+/* on != 0 (default): transverse meshes that fill its tiles are summed by the
+ * matrix-product kernel; 0: every request by the kernels of one lane per point.
+ * The switch exists to compare them. */
+SRWL_EXPORT int srwlAmdSetMeshKernel(int on);
+
+/* Sweeps after which the two chains (upstream, downstream of ct = 0) of the
+ * first trajectory of the last parallel RK4 had converged: out2[k] = 0 when
+ * chain k had not and was handed to the one-workgroup solver, the largest
+ * number of sweeps when there is no such chain. */
+SRWL_EXPORT int srwlAmdLastTrajSweeps(int* out2);
 
 /* Tolerance of the condition check of the FP32 SR sums (method 0): a point
  * whose estimated rounding error exceeds tol times the magnitude of its field

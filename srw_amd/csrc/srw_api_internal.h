@@ -85,6 +85,8 @@ struct Context {
     bool lastStreamFallback = false;
     bool lastStreamed = false;    // the last single-request call streamed rows without falling back
     bool trajSerial = false;      // test switch: serial RK4 kernel instead of the parallel one
+    bool meshKernel = true;       // test switch: mesh requests on the matrix cores (else one lane per point)
+    long long trajLd = 0;         // points of the longest trajectory of the last parallel RK4
     bool keepOnDevice = false;    // benchmark switch: leave results in HBM
     bool resizePerPoint = false;  // test switch: resample per new point instead of per old cell
     bool tuneTiles = true;        // FFT tile shapes from the autotuner (else the fixed defaults)

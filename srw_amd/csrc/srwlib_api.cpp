@@ -419,6 +419,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
         if (!g_ctx.trajSerial) {
             dPic = (double*)B.Pic.get(sizeof(double) * (size_t)srwd_traj_scratch(ldT) * nT);
             if (!dPic) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+            g_ctx.trajLd = ldT;
         }
         int one = 1;
         for (auto& f : fields) one = one && (f.n == 1 && f.u[0].nh == 1);
@@ -572,7 +573,8 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     std::vector<char> isMesh(nT);
     bool allMesh = true;
     for (int j = 0; j < nT; j++) {
-        isMesh[j] = mesh_kernel_pays(reqs[j].nxc, reqs[j].nzc) && mesh_kernel_fine(info[j], jobs[j].mesh);
+        isMesh[j] = g_ctx.meshKernel && mesh_kernel_pays(reqs[j].nxc, reqs[j].nzc) &&
+                    mesh_kernel_fine(info[j], jobs[j].mesh);
         allMesh = allMesh && isMesh[j];
     }
     for (int j = 0; j < nT; j++) {
@@ -1634,6 +1636,7 @@ SRWL_EXPORT int srwlCalcPartTraj(SRWLPrtTrj* pTrj, SRWLMagFldC* pMagFld, double*
     if (!g_ctx.trajSerial) {
         dPic = (double*)B.Pic.get(sizeof(double) * (size_t)srwd_traj_scratch(pTrj->np));
         if (!dPic) return SRWL_ERR_MEMORY_ALLOCATION_FAILURE;
+        g_ctx.trajLd = pTrj->np;
     }
     int one = (f.n == 1 && f.u[0].nh == 1);
     if (srwd_launch_traj((srwd_traj_job*)(dUp + oJob), (srwd_field*)(dUp + oField), 1, dX, dXp, dY, dYp, dZ, pTrj->np,
@@ -1905,6 +1908,26 @@ SRWL_EXPORT int srwlAmdSetBands(int nBands)
 {
     if (nBands < 0 || nBands > SRWL_AMD_MAX_BANDS) return SRWL_AMD_ERR_UNSUPPORTED;
     g_ctx.forceBands = nBands;
+    return 0;
+}
+
+SRWL_EXPORT int srwlAmdSetMeshKernel(int on) { g_ctx.meshKernel = on != 0; return 0; }
+
+SRWL_EXPORT int srwlAmdLastTrajSweeps(int* out2)
+{
+    if (!g_ctx.ready || out2 == nullptr || g_ctx.trajLd < 16 || !g_ctx.buf.Pic.p) return SRWL_NO_FUNC_ARG_DATA;
+    // the two chains' records (sw_scratch in sr.hip): in their last two doubles
+    // the sweep that found the chain converged, and two bits per sweep
+    double rec[2 * 12];
+    const double* at = (const double*)g_ctx.buf.Pic.p + srwd_traj_scratch(g_ctx.trajLd) - 2 * 12;
+    HIPCHK(hipMemcpy(rec, at, sizeof(rec), hipMemcpyDeviceToHost));
+    for (int side = 0; side < 2; side++) {
+        int conv;
+        unsigned moved;
+        std::memcpy(&conv, rec + side * 12 + 10, sizeof(conv));
+        std::memcpy(&moved, rec + side * 12 + 11, sizeof(moved));
+        out2[side] = conv ? conv : ((moved >> (2 * SRWD_SW_MAX - 2) & 3) ? 0 : SRWD_SW_MAX);
+    }
     return 0;
 }
 

@@ -181,6 +181,18 @@ def set_traj_serial(on=True):
     lib.srwlAmdSetTrajSerial(1 if on else 0)
 
 
+def set_mesh_kernel(on=True):
+    """Matrix-product kernel for the sums of meshes (default on); off: one lane per point."""
+    _check(lib.srwlAmdSetMeshKernel(1 if on else 0))
+
+
+def last_traj_sweeps():
+    """Sweeps to convergence of the (upstream, downstream) chain of the last trajectory; 0: handed on unconverged."""
+    out = (C.c_int * 2)()
+    _check(lib.srwlAmdLastTrajSweeps(out))
+    return list(out)
+
+
 def set_stream_rows(on=True):
     """Streamed-rows download of a single request's field (default on)."""
     _check(lib.srwlAmdSetStreamRows(1 if on else 0))

@@ -43,7 +43,8 @@ def _case(nx, ny, ne=1, nper=12, np_traj=1201, tilt=False):
 @pytest.mark.parametrize("nx,ny", [(32, 32), (33, 65), (64, 64), (65, 63), (128, 31), (40, 97), (16, 16), (200, 5),
                                    (22, 23), (23, 23), (12, 300)])
 def test_mesh_sizes_around_a_tile(nx, ny):
-    """The last two are too small or too narrow for the kernel: the per-point one."""
+    """16 x 16, 200 x 5 and 22 x 23 fill less than an eighth of their tiles: the
+    one-lane kernel."""
     print("case:", nx, ny, flush=True)
     e = _error(*_case(nx, ny, tilt=True))
     print("rel-L2 %.2e" % e, flush=True)
@@ -84,6 +85,27 @@ def test_batch_mixes_both_kernels():
         srwlpy.CalcElecFieldSR(w, 0, m, prec)
         g, o = cfield(b.arEx, b), cfield(w.arEx, w)
         assert np.linalg.norm(g - o) < 1e-6 * np.linalg.norm(o)
+
+
+@pytest.mark.parametrize("nx,ny,ne", [(64, 64, 1), (70, 45, 11), (150, 93, 3)])
+def test_agrees_with_one_lane_per_point(nx, ny, ne):
+    """The same mesh with the kernel on and off.  Tolerance: twice TOL's share of
+    a kernel, 1e-6 of rounding each (see above), with the factor of 10 shared."""
+    from srw_amd import srwlpy
+    print("case:", nx, ny, ne, flush=True)
+    w, mag, prec = _case(nx, ny, ne=ne, tilt=True)
+    got = []
+    for on in (True, False):
+        wg = clone_wfr(w)
+        srwlpy.set_mesh_kernel(on)
+        try:
+            srwlpy.CalcElecFieldSR(wg, 0, mag, prec)
+        finally:
+            srwlpy.set_mesh_kernel(True)
+        got.append(np.stack([cfield(wg.arEx, wg), cfield(wg.arEy, wg)]))
+    d = np.linalg.norm(got[0] - got[1]) / np.linalg.norm(got[1])
+    print("rel-L2 %.2e" % d, flush=True)
+    assert 0 < d < TOL
 
 
 @pytest.mark.parametrize("small,ne", [((1, 1), 1), ((1, 3), 9), ((9, 1), 1)])
@@ -130,7 +152,11 @@ def test_streamed_tile_rows_equal_one_pass(nx, ny, ne):
             srwlpy.CalcElecFieldSR(wg, 0, mag, prec)
         finally:
             srwlpy.set_bands(0)
-        print("bands %d: streamed %s" % (bands, srwlpy.last_streamed()), flush=True)
+        fp64 = int(srwlpy.stats()["sr_fp64_points"])
+        print("bands %d: streamed %s, FP64 points %d" % (bands, srwlpy.last_streamed(), fp64), flush=True)
+        overflow = fp64 > 1 << 18
+        assert overflow == ((nx, ny) == (33, 600))
+        assert srwlpy.last_streamed() == (bands == 0 and not overflow)
         got.append([np.frombuffer(getattr(wg, c), np.float32) for c in ("arEx", "arEy")])
     for a, b in zip(*got):
         assert np.isfinite(a).all() and np.abs(a).max() > 0

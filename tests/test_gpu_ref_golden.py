@@ -102,19 +102,22 @@ def test_gpu_multi_energy_call_equals_single_energy_slices():
 def test_gpu_energy_tiles_per_point_error_and_agreement():
     """The energy-tile kernel (8 photon energies per workgroup, the phasor of
     each energy advanced from the previous one's): a 101 x 101 mesh at 16
-    energies over +/-5 % of the first harmonic against the FP64 oracle, every
+    energies over +/-5 % of the first harmonic, with the matrix-product kernel
+    that meshes take otherwise switched off, against the FP64 oracle, every
     point of every energy within 1e-4 of its field's magnitude, and within
     1e-6 rel-L2 of the one-energy-per-workgroup kernel."""
     from srw_amd import srwlpy
     w, mag, prec = W.single_electron(n=101, ne=16, de_rel=0.05)
     wt, w1, wo = clone_wfr(w), clone_wfr(w), clone_wfr(w)
-    srwlpy.CalcElecFieldSR(wt, 0, mag, prec)
-    fp64 = int(srwlpy.stats()["sr_fp64_points"])
     try:
+        srwlpy.set_mesh_kernel(False)
+        srwlpy.CalcElecFieldSR(wt, 0, mag, prec)
+        fp64 = int(srwlpy.stats()["sr_fp64_points"])
         srwlpy.set_energy_tiles(0)
         srwlpy.CalcElecFieldSR(w1, 0, mag, prec)
     finally:
         srwlpy.set_energy_tiles(8)
+        srwlpy.set_mesh_kernel(True)
     assert oracle.calc_field(wo, mag, prec, nthreads=16) == 0
     ext, eyt = cfield(wt.arEx, wt), cfield(wt.arEy, wt)
     exo, eyo = cfield(wo.arEx, wo), cfield(wo.arEy, wo)
