@@ -1517,9 +1517,8 @@ __device__ void sr_finish_point(const srwd_item& IT, const srwd_trj_info& I, con
     if (fpList) {
         // condition check of the FP32 sums against the point's field
         // magnitude: hand the point to the FP64 pass
-        const double eps = IT.tiled == SRWD_ITEM_MESH
-                               ? SRWD_EPS_TERM_MESH * fmax(1., srwd_mesh_turns(I, IT.eph, xo, zo) / SRWD_MESH_TURNS)
-                               : (IT.tiled ? SRWD_EPS_TERM_TILE : SRWD_EPS_TERM);
+        double eps = IT.tiled >= SRWD_ITEM_MESH ? SRWD_EPS_TERM_MESH : (IT.tiled ? SRWD_EPS_TERM_TILE : SRWD_EPS_TERM);
+        if (IT.tiled == SRWD_ITEM_MESH_FAR) eps *= fmax(1., srwd_mesh_turns(I, IT.eph, xo, zo) / SRWD_MESH_TURNS);
         const double e2 = eps * eps * w * w, t2 = condTol * condTol;
         const double mag2 = ex.re * ex.re + ex.im * ex.im + ez.re * ez.re + ez.im * ez.im;
         if (e2 * (fmax(sumSqX, 0.) + fmax(sumSqZ, 0.)) > t2 * mag2) {

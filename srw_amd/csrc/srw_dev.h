@@ -103,6 +103,7 @@ struct srwd_item {
 #define SRWD_ITEM_POINT 0
 #define SRWD_ITEM_TILE 1
 #define SRWD_ITEM_MESH 2
+#define SRWD_ITEM_MESH_FAR 3   // the same, somewhere beyond SRWD_MESH_TURNS
 
 #define SRWD_CHUNK 256
 // Photon energies per workgroup of the energy-tile SR kernel (4 or 8): the

@@ -248,23 +248,24 @@ static bool mesh_kernel_pays(int nxc, int nzc)
     return mesh_tiles(nxc, nzc) * T2 <= 8LL * nxc * nzc;
 }
 
-// Whether the FP32 phase increments of the mesh kernel are as fine over the mesh
-// as those of one lane per point.  They hold the whole phase over 4 steps, the
-// other kernels' the part that depends on the observation point over a chunk,
-// with the rest from a table reduced in FP64: where a sampled integrand ends
-// (SRWD_MESH_TURNS), the kernel of the smaller phase.  1 MeV in steps of 8.6 mm,
-// 870 turns: 40 x 40 points over 20 um, one lane per point / mesh kernel
-// 3.4e-7 / 2.3e-4 rel-L2; over 2 mm, where a chunk turns 2200 times, 2.3e-4 /
-// 1.3e-4.
-static bool mesh_kernel_fine(const srwd_trj_info& I, const SRWLRadMesh& m)
+// The kind of a request's mesh items, by whether the FP32 phase increments of the
+// mesh kernel are as fine over the mesh as those of one lane per point (else
+// SRWD_ITEM_POINT).  They hold the whole phase over 4 steps, the other kernels'
+// the part that depends on the observation point over a chunk, with the rest from
+// a table reduced in FP64: beyond a sampled integrand (SRWD_MESH_TURNS), the
+// kernel of the smaller phase.  1 MeV in steps of 8.6 mm, 870 turns: 40 x 40
+// points over 20 um, one lane per point / mesh kernel 3.4e-7 / 2.3e-4 rel-L2; over
+// 2 mm, where a chunk turns 2200 times, 2.6e-4 / 1.3e-4.
+static int mesh_item_kind(const srwd_trj_info& I, const SRWLRadMesh& m)
 {
     const double e = std::max(m.eStart, m.eFin);
     const double x = std::max(std::fabs(m.xStart), std::fabs(m.xFin)), z = std::max(std::fabs(m.yStart), std::fabs(m.yFin));
     const double turns = srwd_mesh_turns(I, e, x, z);
+    if (turns <= SRWD_MESH_TURNS) return SRWD_ITEM_MESH;
     srwd_trj_info C = I;   // a chunk's steps, of the observation angles alone
     C.h *= 0.25 * (double)std::min<long long>(I.nInt, SRWD_CHUNK);
     C.gammaEm2 = C.angX = C.angZ = 0.;
-    return turns <= std::max(SRWD_MESH_TURNS, srwd_mesh_turns(C, e, x, z));
+    return turns <= srwd_mesh_turns(C, e, x, z) ? SRWD_ITEM_MESH_FAR : SRWD_ITEM_POINT;
 }
 
 // Parts of the s-range of a mesh pass of nTiles tiles and nPts points: the least
@@ -570,11 +571,11 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
     const double normBase = 1. / 137.0360411;
     std::vector<int> rowBase(nT);
     // requests whose mesh goes to the matrix-product kernel (no phase table)
-    std::vector<char> isMesh(nT);
+    std::vector<char> isMesh(nT);   // SRWD_ITEM_MESH or SRWD_ITEM_MESH_FAR; 0: one lane per point
     bool allMesh = true;
     for (int j = 0; j < nT; j++) {
-        isMesh[j] = g_ctx.meshKernel && mesh_kernel_pays(reqs[j].nxc, reqs[j].nzc) &&
-                    mesh_kernel_fine(info[j], jobs[j].mesh);
+        isMesh[j] = g_ctx.meshKernel && mesh_kernel_pays(reqs[j].nxc, reqs[j].nzc) ? mesh_item_kind(info[j], jobs[j].mesh)
+                                                                                   : SRWD_ITEM_POINT;
         allMesh = allMesh && isMesh[j];
     }
     for (int j = 0; j < nT; j++) {
@@ -690,7 +691,7 @@ int sr_run(std::vector<SrJob>& jobs, const std::vector<srwd_field>& fields, floa
                 it.actNorm = normConst * it.eph * 0.80654658E-03;
                 it.drow = dRowOf[j];
                 it.de = eStepOf[j];
-                it.tiled = isMesh[j] ? SRWD_ITEM_MESH : (ie < nTiled ? SRWD_ITEM_TILE : SRWD_ITEM_POINT);
+                it.tiled = isMesh[j] ? isMesh[j] : (ie < nTiled ? SRWD_ITEM_TILE : SRWD_ITEM_POINT);
                 int nb = (it.npts + 255) / 256;
                 const int me = (int)items.size();
                 nBlocks += nb;
