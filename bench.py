@@ -466,7 +466,8 @@ def main():
                      "evals_per_launch": evals, "flops_per_eval": FLOPS_PER_EVAL,
                      "flops_counted": ("FP16 matrix flops of the mesh points: 24 multiply-adds per evaluation (both "
                                        "components, hi + lo pairs); phasors and the tiles' places outside the mesh "
-                                       "(101 of 128 rows and columns used at 201 x 201) not counted")},
+                                       "(201 of 256 columns and 101 of 128 rows used at 201 x 201, mirrored in "
+                                       "y) not counted")},
         "device_resident_points_per_s": pts * a.steps / dt_dev,
         "sr_kernel_ms_in_api_run": k_ms,
         "api_call_ms": {"min": 1e3 * min(call_s), "median": 1e3 * sorted(call_s)[len(call_s) // 2],

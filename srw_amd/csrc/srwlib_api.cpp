@@ -272,15 +272,17 @@ static int mesh_item_kind(const srwd_trj_info& I, const SRWLRadMesh& m)
 // of a model of its time.  512 workgroups are resident at once (two a CU, by
 // LDS) and such a round takes 3.7 us per unit of the s-range (512 x 512
 // points of 256 electrons: 32 rounds of 313 units in 37.4 ms); each part writes
-// and reads 32 bytes a point.  Measured, whole calls, parts 2 / 5 / 16: 101 x 101
-// x 101 energies (202 tiles) 1.38 / 1.28 / 1.36 ms; 1 / 13 / 24: 150 x 93 x 5
-// (30 tiles) 1.18 / 0.54 / 0.53 ms; 1 / 4 / 16: 128 electrons on 64 x 64 (128
-// tiles) 1.99 / 1.51 / 1.56 ms.
+// and reads 32 bytes a point, at the rate of many points (the 105 parts of 101 x
+// 101 points, which 21 blocks of the finalize pass add, take 33 us, not the 9 of
+// the model).  Measured, whole calls, parts 2 / 5 / 16: 101 x 101 x 101 energies
+// (202 tiles) 1.38 / 1.28 / 1.36 ms; 1 / 13 / 24: 150 x 93 x 5 (30 tiles) 1.18 /
+// 0.54 / 0.53 ms; 1 / 4 / 16: 128 electrons on 64 x 64 (128 tiles) 1.99 / 1.51 /
+// 1.56 ms.
 // A large field, whose rows are streamed to the host, takes parts of about 24
-// units (0.1 ms) while its partial sums stay under 2 GB: the finalize pass of the rows already summed gets its places
-// as the next rows' workgroups leave, and short ones leave sooner.  201 x 201 x
-// 201, parts 1 / 5 / 13: 8.23 / 7.36 / 6.7 ms; 400 x 400 x 20: 3.80 / 3.12 /
-// 2.65 ms.
+// units (0.1 ms) while its partial sums stay under 2 GB: the finalize pass of the
+// rows already summed gets its places as the next rows' workgroups leave, and
+// short ones leave sooner.  201 x 201 x 201, parts 1 / 5 / 13: 8.23 / 7.36 / 6.7
+// ms; 400 x 400 x 20: 3.80 / 3.12 / 2.65 ms.
 static int mesh_split(long long nTiles, long long nUnits, long long nPts, bool large)
 {
     if (large)
