@@ -930,9 +930,13 @@ __global__ void __launch_bounds__(SRWD_QT_THREADS) k_angle_scan(const srwd_trj_i
         if (lane == 63) inc[w] = x;
         __syncthreads();
         for (int q = 0; q < w; q++) x += inc[q];
+        // the terms between the nodes, one a lane (with the index the same for all
+        // lanes the compiler chose the window of angle_term by a stale condition
+        // bit, and s0 between two trajectory points got a wrong integral)
+        const double between = angle_term(ang, off + lane, n1, stepMult);
         double f[6], c[6];
         f[0] = node;
-        for (int k = 1; k < 6; k++) f[k] = f[k - 1] + angle_term(ang, off + k, n1, stepMult);
+        for (int k = 1; k < 6; k++) f[k] = f[k - 1] + __shfl(between, k, 64);
         coefs5(sStep, f, c);
         const double sv = c[0] + rel * (c[1] + rel * (c[2] + rel * (c[3] + rel * (c[4] + rel * c[5]))));
         if (i < np) (pl ? IBz : IBx)[tr * ld + i] = (before + x) - sv;
