@@ -1477,9 +1477,10 @@ __global__ void __launch_bounds__(256) k_sr_integral_tile(const srwd_item* __res
 // computed), against every point in FP64; points recomputed / worst error left:
 // without the check 0 / 3.6e-3 (6.1e-3 with one lane per point), 1e-6 5.6e4 /
 // 5.3e-5 (7.9e-5), 2e-6 8.9e4 / 3.0e-5 (3.8e-5), 4e-6 1.4e5 / 2.8e-5 (2.1e-5):
-// 2e-6 leaves a factor 3.3.  Those turns stay below 0.5; beyond SRWD_MESH_TURNS
-// the increments' rounding (4e-7 a turn) leads and the estimate grows with them.
+// 2e-6 leaves a factor 3.3.  Those turns stay below 0.5; from 4 on the rounding of
+// the increments (4e-7 a turn) leads and the estimate grows with them.
 #define SRWD_EPS_TERM_MESH 2e-6
+#define SRWD_EPS_TURNS 4.
 
 // Terminating terms, the derivative correction, the float store and the
 // mirrored parts of one point; S = sum over the integration points of
@@ -1522,7 +1523,7 @@ __device__ void sr_finish_point(const srwd_item& IT, const srwd_trj_info& I, con
         // condition check of the FP32 sums against the point's field
         // magnitude: hand the point to the FP64 pass
         double eps = IT.tiled >= SRWD_ITEM_MESH ? SRWD_EPS_TERM_MESH : (IT.tiled ? SRWD_EPS_TERM_TILE : SRWD_EPS_TERM);
-        if (IT.tiled == SRWD_ITEM_MESH_FAR) eps *= fmax(1., srwd_mesh_turns(I, IT.eph, xo, zo) / SRWD_MESH_TURNS);
+        if (IT.tiled == SRWD_ITEM_MESH_FAR) eps *= fmax(1., srwd_mesh_turns(I, IT.eph, xo, zo) / SRWD_EPS_TURNS);
         const double e2 = eps * eps * w * w, t2 = condTol * condTol;
         const double mag2 = ex.re * ex.re + ex.im * ex.im + ez.re * ez.re + ez.im * ez.im;
         if (e2 * (fmax(sumSqX, 0.) + fmax(sumSqZ, 0.)) > t2 * mag2) {
@@ -1556,8 +1557,8 @@ __device__ void sr_finish_point(const srwd_item& IT, const srwd_trj_info& I, con
 // cond[0..4] = sum b^2, sum b bPx, sum b bPz, sum bPx^2, sum bPz^2, so that
 // the squared x terms of point (xo, zo) add up to
 // cond[0] xo^2 - 2 xo cond[1] + cond[3] (and the z terms likewise).  The
-// largest |b|, |bPx| and |bPz| give the amplitude scales of the mesh records, the
-// last two also angX and angZ: b P = w P / R^2 with w at most 16.
+// largest |b|, |bPx| and |bPz| give the amplitude scales of the mesh records;
+// angX and angZ are the largest |P| / R, where b = w / R^2.
 #define SRWD_CS_THREADS 1024
 __global__ void __launch_bounds__(SRWD_CS_THREADS) k_cond_sums(srwd_trj_info* __restrict__ info,
                                                                const srwd_rec* __restrict__ rec, long long ldI,
@@ -1567,15 +1568,17 @@ __global__ void __launch_bounds__(SRWD_CS_THREADS) k_cond_sums(srwd_trj_info* __
     int tr = blockIdx.x;
     long long n = info[tr].nInt;
     const srwd_rec* R = rec + (long long)tr * ldI;
-    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    double v[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     for (long long i = threadIdx.x; i < n; i += blockDim.x) {
         double bb = R[i].b, px = R[i].bPx, pz = R[i].bPz;
         v[0] += bb * bb; v[1] += bb * px; v[2] += bb * pz; v[3] += px * px; v[4] += pz * pz;
         v[5] = fmax(v[5], fabs(bb)); v[6] = fmax(v[6], fabs(px)); v[7] = fmax(v[7], fabs(pz));
+        const double ir = rsqrtf(R[i].b * ((i == 0 || i == n - 1) ? 7.f : ((i & 1) ? 16.f : 14.f)));
+        v[8] = fmax(v[8], fabs(px) * ir); v[9] = fmax(v[9], fabs(pz) * ir);
     }
-    __shared__ double sh[SRWD_CS_THREADS / 64][8];
+    __shared__ double sh[SRWD_CS_THREADS / 64][10];
     const int lane = threadIdx.x & 63;
-    for (int k = 0; k < 8; k++) {
+    for (int k = 0; k < 10; k++) {
         double x = v[k];
         for (int off = 32; off > 0; off >>= 1) {
             const double y = __shfl_xor(x, off, 64);
@@ -1584,16 +1587,15 @@ __global__ void __launch_bounds__(SRWD_CS_THREADS) k_cond_sums(srwd_trj_info* __
         if (lane == 0) sh[threadIdx.x >> 6][k] = x;
     }
     __syncthreads();
-    for (int k = 0; k < 8; k++) {
+    for (int k = 0; k < 10; k++) {
         double x = sh[0][k];
         for (int q = 1; q < SRWD_CS_THREADS / 64; q++) x = k < 5 ? x + sh[q][k] : fmax(x, sh[q][k]);
         v[k] = x;
     }
     if (threadIdx.x < 5) cond[5 * tr + threadIdx.x] = v[threadIdx.x];
     if (threadIdx.x == 0) {
-        const double far = info[tr].yObs - info[tr].sIntegStart;
-        info[tr].angX = v[6] * far / 14.;
-        info[tr].angZ = v[7] * far / 14.;
+        info[tr].angX = v[8];
+        info[tr].angZ = v[9];
     }
     const double* ml = mesh + 4 * tr;
     for (int side = 0; side < 2; side++) {

@@ -252,8 +252,10 @@ static bool mesh_kernel_pays(int nxc, int nzc)
 // mesh kernel are as fine over the mesh as those of one lane per point (else
 // SRWD_ITEM_POINT).  They hold the whole phase over 4 steps, the other kernels'
 // the part that depends on the observation point over a chunk, with the rest from
-// a table reduced in FP64: beyond a sampled integrand (SRWD_MESH_TURNS), the
-// kernel of the smaller phase.  1 MeV in steps of 8.6 mm, 870 turns: 40 x 40
+// a table reduced in FP64: beyond SRWD_MESH_TURNS, the kernel of the smaller
+// phase.  40 x 48 points over 0.2 mm, ninth harmonic in steps of 0.9 mm (2.4
+// turns), one lane per point / mesh kernel 1.6e-6 / 4.3e-6 rel-L2; over 2 mm (3.2
+// turns) 4.3e-6 / 2.9e-6.  1 MeV in steps of 8.6 mm, 870 turns: 40 x 40
 // points over 20 um, one lane per point / mesh kernel 3.4e-7 / 2.3e-4 rel-L2; over
 // 2 mm, where a chunk turns 2200 times, 2.6e-4 / 1.3e-4.
 static int mesh_item_kind(const srwd_trj_info& I, const SRWLRadMesh& m)

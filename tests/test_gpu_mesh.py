@@ -108,6 +108,34 @@ def test_agrees_with_one_lane_per_point(nx, ny, ne):
     assert 0 < d < TOL
 
 
+@pytest.mark.parametrize("harm,step,half", [(1, 16, 1e-4), (5, 4, 1e-4), (9, 2, 1e-4), (9, 4, 1e-4), (15, 2, 1e-5),
+                                            (9, 4, 1e-3)])
+def test_errors_no_larger_than_one_lane_per_point(harm, step, half):
+    """Harmonics and steps at which the phase turns by 0.5 to 3 revolutions over 4
+    steps: the errors against FP64 at most 1.2 of those with the kernel off."""
+    from srw_amd import srwlpy
+    print("case: harmonic %d, step x %d, half %g m" % (harm, step, half), flush=True)
+    beam = W.electron_beam(x=2e-6, y=1e-6)
+    e = harm * 0.995 * W.first_harmonic_eV(beam.partStatMom1.gamma, 1.5, 0.02)
+    w = W.wavefront(beam, 1, e, e, 48, 40, half, half, 20.)
+    prec = W.traj_prec(10001)
+    prec[1] *= step
+    got = []
+    for on, tol in ((True, 0.), (False, 0.), (True, 1e-12)):
+        wg = clone_wfr(w)
+        srwlpy.set_mesh_kernel(on)
+        srwlpy.set_cond_tol(tol)
+        try:
+            srwlpy.CalcElecFieldSR(wg, 0, W.planar_undulator(), prec)
+        finally:
+            srwlpy.set_mesh_kernel(True)
+            srwlpy.set_cond_tol(1e-4)
+        got.append(np.stack([cfield(wg.arEx, wg), cfield(wg.arEy, wg)]))
+    mesh, lane = (np.linalg.norm(g - got[2]) / np.linalg.norm(got[2]) for g in got[:2])
+    print("kernel on %.2e, off %.2e" % (mesh, lane), flush=True)
+    assert mesh <= 1.2 * lane
+
+
 @pytest.mark.parametrize("small,ne", [((1, 1), 1), ((1, 3), 9), ((9, 1), 1)])
 def test_small_request_among_meshes_keeps_the_parts(small, ne):
     """One request off the mesh kernel in a batch of large meshes: the partial
